@@ -121,4 +121,46 @@ __device__ __forceinline__ u64 mont_mul(u64 normal, u64 mont, u64 q, u64 qninv) 
     return redc128(normal * mont, __umul64hi(normal, mont), q, qninv);
 }
 
+// ---- integers below 2^52 as doubles ----
+// The exponent of 2^52 over the integer's bits is 2^52 + x; both conversions
+// are one add and one bitwise operation.
+__device__ __forceinline__ double fp_from_u64(u64 x) {
+    return __builtin_bit_cast(double, x | 0x4330000000000000ull) - 0x1p52;
+}
+__device__ __forceinline__ u64 fp_to_u64(double x) {
+    return __builtin_bit_cast(u64, x + 0x1p52) & 0x000fffffffffffffull;
+}
+
+// Residues modulo q < 2^50 as integer-valued doubles of either sign.  With
+// |x| < 2^53 every sum and product below is an exact integer computation.
+struct FpMod {
+    double q, qinv;  // qinv = RN(1/q)
+    // x w mod q for a constant w, |w| <= q/2, wq = RN(w/q).  h = RN(x w), its
+    // exact error is l = fma(x, w, -h), and k = rint(x wq) is within 1/2 +
+    // |x| 2^-53 of x w / q (two roundings of a value of at most |x|/2), so
+    // fma(-k, q, h) + l is x w - k q itself: an integer of magnitude at most
+    // (1/2 + |x| 2^-53) q, hence representable at every step.
+    __device__ __forceinline__ double mul(double x, double w, double wq) const {
+        const double h = x * w, l = __builtin_fma(x, w, -h);
+        const double k = __builtin_rint(x * wq);
+        return __builtin_fma(-k, q, h) + l;
+    }
+    // x y mod q for two variables: the quotient estimate is off by at most
+    // 1/2 + |x y / q| 2^-52, so the result is at most 3/4 q for canonical
+    // operands and 9/2 q for operands up to 4q.
+    __device__ __forceinline__ double mulq(double x, double y) const {
+        const double h = x * y, l = __builtin_fma(x, y, -h);
+        const double k = __builtin_rint(h * qinv);
+        return __builtin_fma(-k, q, h) + l;
+    }
+    // to [-q/2, q/2] (|x| <= 2^53: the estimate is off by far less than 1/2)
+    __device__ __forceinline__ double centred(double x) const {
+        return __builtin_fma(-__builtin_rint(x * qinv), q, x);
+    }
+    __device__ __forceinline__ u64 canonical(double x) const {
+        const double c = centred(x);
+        return fp_to_u64(c < 0.0 ? c + q : c);
+    }
+};
+
 }  // namespace mi

@@ -35,6 +35,13 @@ struct LiftJob {
         const u64* c0;
         u64* o;
         u64 q0, q, mu_hi;
+        double qd, qinv;
+        __device__ double load_fp(int i) const {
+            if (q0 >= (1ull << FP_BITS)) return fp_from_u64(load(i));  // uniform
+            const u64 v = c0[i];
+            const double x = v > (q0 >> 1) ? -fp_from_u64(q0 - v) : fp_from_u64(v);
+            return FpMod{qd, qinv}.centred(x);
+        }
         __device__ u64 load(int i) const {
             const u64 v = c0[i];
             if (v > (q0 >> 1)) {
@@ -47,7 +54,7 @@ struct LiftJob {
     };
     __device__ View view(int k) const {
         const BasisConst b = bc[k];
-        return View{k, coeff0, out + (long long)k * N, q0, b.q, b.mu_hi};
+        return View{k, coeff0, out + (long long)k * N, q0, b.q, b.mu_hi, b.qd, b.inv_d};
     }
     __device__ bool skip(int) const { return false; }
 };
@@ -94,7 +101,7 @@ struct LiftListJob {
     __device__ LiftJob::View view(int k) const {
         const int l = per_limb.div(k), it = k - l * n;
         const BasisConst b = bc[l];
-        return LiftJob::View{l, coeff0 + (long long)it * N, out[it] + (long long)l * N, q0, b.q, b.mu_hi};
+        return LiftJob::View{l, coeff0 + (long long)it * N, out[it] + (long long)l * N, q0, b.q, b.mu_hi, b.qd, b.inv_d};
     }
     __device__ bool skip(int) const { return false; }
 };

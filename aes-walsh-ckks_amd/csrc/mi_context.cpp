@@ -74,10 +74,11 @@ static void make_twiddles(u64 N, int logN, u64 q, u64* fwd, u64* fws, u64* inv, 
             inv[m + i] = pw[(2 * N - ex) % (2 * N)];
         }
     }
-    for (u64 i = 0; i < N; ++i) {
-        fws[i] = shoup_of(fwd[i], q);
-        ivs[i] = shoup_of(inv[i], q);
-    }
+    if (q >= (1ull << FP_BITS))
+        for (u64 i = 0; i < N; ++i) {
+            fws[i] = shoup_of(fwd[i], q);
+            ivs[i] = shoup_of(inv[i], q);
+        }
     u128 mu = (~(u128)0) / q;
     bc.q = q;
     bc.mu_lo = (u64)mu;
@@ -92,6 +93,27 @@ static void make_twiddles(u64 N, int logN, u64 q, u64* fwd, u64* fws, u64* inv, 
     bc.negq = (u64)0 - q;
     bc.w1_ninv = (u64)(((u128)inv[1] * bc.n_inv) % q);
     bc.w1_ninv_shoup = shoup_of(bc.w1_ninv, q);
+    bc.qd = (double)q;
+    bc.fp = q < (1ull << FP_BITS) ? 1 : 0;
+    if (bc.fp) {
+        // (w, companion) -> centred w and w/q as doubles, in place
+        auto centred = [q](u64 w) { return w > q / 2 ? -(double)(q - w) : (double)w; };
+        bc.n_inv_fp = centred(bc.n_inv);
+        bc.n_inv_fpq = bc.n_inv_fp / bc.qd;
+        bc.w1_ninv_fp = centred(bc.w1_ninv);
+        bc.w1_ninv_fpq = bc.w1_ninv_fp / bc.qd;
+        bc.rinv_fp = centred(invm(bc.r_mod_q, q));
+        bc.rinv_fpq = bc.rinv_fp / bc.qd;
+        auto convert = [&](u64* w, u64* ws) {
+            for (u64 i = 0; i < N; ++i) {
+                const double c = centred(w[i]), cq = c / bc.qd;
+                std::memcpy(&w[i], &c, 8);
+                std::memcpy(&ws[i], &cq, 8);
+            }
+        };
+        convert(fwd, fws);
+        convert(inv, ivs);
+    }
     (void)logN;
 }
 

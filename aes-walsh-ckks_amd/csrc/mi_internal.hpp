@@ -26,7 +26,16 @@ struct BasisConst {
     u64 negq;           // 2^64 - q
     u64 w1_ninv, w1_ninv_shoup;  // inverse twiddle 1 times N^-1: the last inverse
                                  //   stage fused with the scaling
+    // Moduli below 2^50 (fp != 0) are transformed in exact double arithmetic:
+    // their twiddle tables hold the centred w and w/q as doubles in place of w
+    // and its Shoup companion, and so do these.
+    int fp;
+    double qd;                   // q
+    double n_inv_fp, n_inv_fpq;
+    double w1_ninv_fp, w1_ninv_fpq;
+    double rinv_fp, rinv_fpq;    // 2^-64 mod q: a Montgomery-form factor's excess
 };
+constexpr int FP_BITS = 50;
 
 // HPS ModUp tables of one (level, digit): source limbs are the digit's chain
 // limbs [s0, s1); destinations are the remaining chain limbs of the level

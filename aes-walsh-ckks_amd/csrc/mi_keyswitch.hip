@@ -12,22 +12,18 @@
 //                outputs with Add/Assign, P slots kept for ModDown) or whole in
 //                the QP basis, optionally through a Galois automorphism and
 //                with a b term added (:675-852, :373-416).
-//   ks_moddown   folded ModDown (:521-673): INTT of the P slots, contribution
-//                sum_j x_j p_j^-1 - alpha per Q limb (the P-side HPS estimate
-//                computed once per coefficient), NTT, subtracted from Q.
+//   ks_moddown   folded ModDown (:521-673, mi_moddown.hip), also with the key
+//                inner product folded in (mi_moddown_mac.hip).
 // Reordering "+ acc" before "- NTT(contribution)" leaves every canonical
 // residue unchanged.
-#include "mi_ntt_kernels.hpp"
+#include "mi_moddown.hpp"
 
 #include <algorithm>
 #include <vector>
 
 namespace mi {
 
-constexpr int KS_THREADS = 256;
-constexpr int MAX_ALPHA = 16;   // digit width held in registers
 constexpr int MODUP_DCH = 8;    // destination limbs per ModUp thread
-constexpr int MODDOWN_TCH = 4;  // target limbs per ModDown-contribution thread
 
 // ---- out-of-place inverse NTT of n key terms -> C (item-minor within a limb) ----
 struct CopyListJob {
@@ -47,25 +43,6 @@ struct CopyListJob {
     __device__ View view(int k) const {
         const int l = per_limb.div(k), it = k - l * n;
         return View{l, src[it] + (long long)l * N, dst + it * dstride + (long long)l * N};
-    }
-    __device__ bool skip(int) const { return false; }
-};
-
-// ---- in-place NTT over a list of polys (limb-major: shared twiddles) ----
-struct ListJob {
-    u64* p[2 * KS_MAX_ITEMS];
-    int npoly, basis0;
-    u64 N;
-    FastDiv per_limb;  // npoly
-    struct View {
-        int basis;
-        u64* p;
-        __device__ u64 load(int i) const { return p[i]; }
-        __device__ void store(int i, u64 v) const { p[i] = v; }
-    };
-    __device__ View view(int k) const {
-        const int l = per_limb.div(k), poly = k - l * npoly;
-        return View{basis0 + l, p[poly] + (long long)l * N};
     }
     __device__ bool skip(int) const { return false; }
 };
@@ -154,8 +131,6 @@ __global__ void __launch_bounds__(KS_THREADS) k_modup(ModUpArgs a) {
         D[(long long)s_slot[jj] * N + c] = v;
     }
 }
-
-#define MI_NS_CASES(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11) X(12) X(13) X(14) X(15) X(16)
 
 // ---- forward NTT of the ModUp'd slots ----
 struct DigitJob {
@@ -282,33 +257,55 @@ __global__ void __launch_bounds__(KS_THREADS) k_mac(MacArgs a) {
     const long long src = a.galois ? (long long)galois_src((u32)i, a.galois, a.logN) : i;
     const u64* digits = a.digits + it * a.digits_stride;
     const u64* key = a.key[it];
-    // Exact 128-bit sums of the digit products: at most 16 digits of
-    // residues below q < 2^62 keep the sum below 2^128.  One reduction at the
-    // end (REDC for Montgomery-form keys, Barrett otherwise) gives the
-    // canonical residue of the sum.
-    U128 sb{0, 0}, sa{0, 0};
-    for (int d = 0; d < a.parts; ++d) {
-        const u64 x = reduce_4q(digits[((long long)d * slots + slot) * N + src], b.q);
-        const u64* kb = key + ((long long)d * 2 * key_limbs + basis) * N;
-        const u64* ka = kb + (long long)key_limbs * N;
-        const u64 kbv = reduce_4q(kb[src], b.q), kav = reduce_4q(ka[src], b.q);
-        mac128(sb, x, kbv);
-        mac128(sa, x, kav);
-    }
     u64 acc_b, acc_a;
-    if (a.montgomery) {
-        if (a.parts <= 4) {
-            // at most 4 products of residues below q: the sum is below 4 q^2 <
-            // q 2^64 (q < 2^62), REDC's precondition, without reducing the high word
+    const u64* dg = digits + (long long)slot * N + src;
+    const u64* kp = key + (long long)basis * N + src;
+    const long long dstep = (long long)slots * N, kstep = 2LL * key_limbs * N, to_a = (long long)key_limbs * N;
+    // Operands are residues below 4q.
+    if (b.fp) {  // uniform over the block
+        // each product at most 9/2 q (FpMod::mulq), centred; 16 of them stay at 8q
+        const FpMod m{b.qd, b.inv_d};
+        double sb = 0.0, sa = 0.0;
+        for (int d = 0; d < a.parts; ++d) {
+            const double x = fp_from_u64(dg[d * dstep]);
+            const u64* k = kp + d * kstep;
+            sb += m.centred(m.mulq(x, fp_from_u64(k[0])));
+            sa += m.centred(m.mulq(x, fp_from_u64(k[to_a])));
+        }
+        if (a.montgomery) {
+            sb = m.mul(sb, b.rinv_fp, b.rinv_fpq);
+            sa = m.mul(sa, b.rinv_fp, b.rinv_fpq);
+        }
+        acc_b = m.canonical(sb);
+        acc_a = m.canonical(sa);
+    } else {
+        // Exact 128-bit sums.  Up to 3 products below 16 q^2 (q < 2^61) fit and
+        // their high word is reduced once; otherwise the operands are brought
+        // below q and at most 16 products of residues below 2^62 fit.  One
+        // reduction at the end (REDC for Montgomery-form keys, Barrett
+        // otherwise) gives the canonical residue of the sum.
+        U128 sb{0, 0}, sa{0, 0};
+        const bool lazy = a.parts <= 3 && b.q < (1ull << 61);
+        for (int d = 0; d < a.parts; ++d) {
+            const u64* k = kp + d * kstep;
+            u64 x = dg[d * dstep], kbv = k[0], kav = k[to_a];
+            if (!lazy) {
+                x = reduce_4q(x, b.q);
+                kbv = reduce_4q(kbv, b.q);
+                kav = reduce_4q(kav, b.q);
+            }
+            mac128(sb, x, kbv);
+            mac128(sa, x, kav);
+        }
+        sb.hi = reduce64(sb.hi, b.q, b.mu_hi);
+        sa.hi = reduce64(sa.hi, b.q, b.mu_hi);
+        if (a.montgomery) {
             acc_b = redc128(sb.lo, sb.hi, b.q, b.qninv);
             acc_a = redc128(sa.lo, sa.hi, b.q, b.qninv);
         } else {
-            acc_b = redc128_any(sb.lo, sb.hi, b.q, b.qninv, b.mu_hi);
-            acc_a = redc128_any(sa.lo, sa.hi, b.q, b.qninv, b.mu_hi);
+            acc_b = barrett128(sb.lo, sb.hi, b.q, b.mu_lo, b.mu_hi);
+            acc_a = barrett128(sa.lo, sa.hi, b.q, b.mu_lo, b.mu_hi);
         }
-    } else {
-        acc_b = reduce128(sb.lo, sb.hi, b.q, b.mu_lo, b.mu_hi);
-        acc_a = reduce128(sa.lo, sa.hi, b.q, b.mu_lo, b.mu_hi);
     }
     const u64* ib = a.init_b[it];
     if (ib && slot < a.L) acc_b = add_mod(acc_b, ib[(long long)slot * N + src], b.q);
@@ -354,377 +351,6 @@ MacArgs mac_args(const Context& c, int level, const u64* digits, const u64* key,
     a.montgomery = montgomery ? 1 : 0;
     a.bc = c.d_bc;
     return a;
-}
-
-// ---- folded ModDown ----
-struct MdContribArgs {
-    const u64* src[2 * KS_MAX_ITEMS];   // P limbs (coefficient domain) of each poly, K limbs apart by N
-    u64* tmp;                           // [npoly][L][N]
-    const u64* pinv;                    // [L][K]
-    int L, K, nq, logN;
-    const BasisConst* bc;
-};
-
-// One block: 256 coefficients of one poly, up to MODDOWN_TCH target limbs;
-// the P-side constants and the targets' p_j^-1 rows are staged in LDS.
-template <int K>
-__global__ void __launch_bounds__(KS_THREADS) k_moddown_contrib(MdContribArgs a) {
-    __shared__ u64 s_pinv[MODDOWN_TCH][K];
-    __shared__ u64 s_tq[MODDOWN_TCH], s_ninv[MODDOWN_TCH], s_muhi[MODDOWN_TCH];
-    __shared__ u64 s_pq[K];
-    __shared__ double s_pinvd[K];
-    const u64 N = (u64)1 << a.logN;
-    const int poly = blockIdx.y;
-    const int t0 = blockIdx.z * MODDOWN_TCH;
-    if (t0 >= a.L) return;  // uniform over the block
-    const int nt = t0 + MODDOWN_TCH < a.L ? MODDOWN_TCH : a.L - t0;
-    for (int e = threadIdx.x; e < nt * K; e += KS_THREADS)
-        s_pinv[e / K][e % K] = a.pinv[(long long)(t0 + e / K) * K + e % K];
-    if (threadIdx.x < nt) {
-        const BasisConst b = a.bc[t0 + threadIdx.x];
-        s_tq[threadIdx.x] = b.q;
-        s_ninv[threadIdx.x] = b.qninv;
-        s_muhi[threadIdx.x] = b.mu_hi;
-    }
-    if (threadIdx.x >= 64 && threadIdx.x < 64 + K) {
-        const BasisConst pb = a.bc[a.nq + threadIdx.x - 64];
-        s_pq[threadIdx.x - 64] = pb.q;
-        s_pinvd[threadIdx.x - 64] = pb.inv_d;
-    }
-    __syncthreads();
-    // N is a multiple of KS_THREADS: every thread has a coefficient
-    const long long i = (long long)blockIdx.x * KS_THREADS + threadIdx.x;
-    const u64* src = a.src[poly];
-    u64 x[K];
-    double est = 0.0;
-#pragma unroll
-    for (int j = 0; j < K; ++j) {
-        x[j] = reduce_4q(src[(long long)j * N + i], s_pq[j]);
-        est = __dadd_rn(est, __dmul_rn((double)x[j], s_pinvd[j]));
-    }
-    u64 al = (u64)__dadd_rn(est, 0.5);
-    if (al > (u64)K) al = (u64)K;
-    for (int tt = 0; tt < nt; ++tt) {
-        U128 acc{0, 0};
-#pragma unroll
-        for (int j = 0; j < K; ++j) mac128(acc, x[j], s_pinv[tt][j]);  // Montgomery-form p_j^-1
-        const u64 q = s_tq[tt];
-        const u64 v = redc128_any(acc.lo, acc.hi, q, s_ninv[tt], s_muhi[tt]);
-        a.tmp[((long long)poly * a.L + t0 + tt) * N + i] = sub_mod(v, al, q);
-    }
-}
-
-// forward NTT of the contributions, limb-major (all polys of one modulus together)
-struct MdInJob {
-    u64* tmp;
-    int L, npoly;
-    u64 N;
-    FastDiv per_limb;  // npoly
-    struct View {
-        int basis;
-        u64* p;
-        __device__ u64 load(int i) const { return p[i]; }
-        __device__ void store(int i, u64 v) const { p[i] = v; }
-    };
-    __device__ View view(int k) const {
-        const int t = per_limb.div(k), poly = k - t * npoly;
-        return View{t, tmp + ((long long)poly * L + t) * N};
-    }
-    __device__ bool skip(int) const { return false; }
-};
-
-struct MdOutJob {
-    const u64* tmp;
-    const u64* base[2 * KS_MAX_ITEMS];
-    u64* out[2 * KS_MAX_ITEMS];
-    int L, npoly;
-    u64 N;
-    const BasisConst* bc;
-    FastDiv per_limb;  // npoly
-    struct View {
-        int basis;
-        const u64* src;
-        const u64* base;
-        u64* out;
-        u64 q;
-        __device__ u64 load(int i) const { return src[i]; }
-        __device__ u64 pre(int i) const { return base[i]; }
-        __device__ void store_pre(int i, u64 v, u64 b) const { out[i] = sub_mod(b, v, q); }
-    };
-    __device__ View view(int k) const {
-        const int t = per_limb.div(k), poly = k - t * npoly;
-        return View{t, tmp + ((long long)poly * L + t) * N, base[poly] + (long long)t * N,
-                    out[poly] + (long long)t * N, bc[t].q};
-    }
-    __device__ bool skip(int) const { return false; }
-};
-
-void ks_moddown_n(Context& c, int level, int npoly, u64* const* p, const u64* const* base, u64* const* out,
-                  u64* T, hipStream_t s) {
-    const int L = level + 1, K = c.np;
-    const u64 N = c.N;
-    if (npoly < 1 || npoly > 2 * KS_MAX_ITEMS) throw Error(-1, "ModDown batch size out of range");
-    if (K > MAX_ALPHA) throw Error(-1, "more than 16 special moduli");
-    {
-        ListJob j{};
-        for (int k = 0; k < npoly; ++k) j.p[k] = p[k];
-        j.npoly = npoly;
-        j.per_limb = fast_div(npoly);
-        j.basis0 = c.nq;
-        j.N = N;
-        run_ntt_inv(c, j, j, K * npoly, s);
-    }
-    MdContribArgs a{};
-    for (int k = 0; k < npoly; ++k) a.src[k] = p[k];
-    a.tmp = T;
-    a.pinv = c.moddown[level].pinv;
-    a.L = L;
-    a.K = K;
-    a.nq = c.nq;
-    a.logN = c.logN;
-    a.bc = c.d_bc;
-    dim3 grid((unsigned)(N / KS_THREADS), npoly, (L + MODDOWN_TCH - 1) / MODDOWN_TCH);
-    switch (K) {
-#define MI_MODDOWN_CASE(KK) \
-        case KK: hipLaunchKernelGGL(k_moddown_contrib<KK>, grid, dim3(KS_THREADS), 0, s, a); break;
-        MI_NS_CASES(MI_MODDOWN_CASE)
-#undef MI_MODDOWN_CASE
-        default: throw Error(-1, "more than 16 special moduli");
-    }
-    MI_HIP(hipGetLastError());
-    MdInJob in{T, L, npoly, N, fast_div(npoly)};
-    MdOutJob o{};
-    o.tmp = T;
-    for (int k = 0; k < npoly; ++k) {
-        o.base[k] = base[k];
-        o.out[k] = out[k];
-    }
-    o.L = L;
-    o.npoly = npoly;
-    o.per_limb = fast_div(npoly);
-    o.N = N;
-    o.bc = c.d_bc;
-    run_ntt_fwd(c, in, o, npoly * L, s);
-}
-
-void ks_moddown(Context& c, int level, u64* p0, u64* p1, const u64* base0, const u64* base1, u64* out0,
-                u64* out1, u64* T, hipStream_t s) {
-    u64* p[2] = {p0, p1};
-    const u64* b[2] = {base0, base1};
-    u64* o[2] = {out0, out1};
-    ks_moddown_n(c, level, p1 ? 2 : 1, p, b, o, T, s);
-}
-
-// ---- ModDown with the key inner product folded in ----
-// The split form of k_mac (Q slots combined into the outputs, P slots kept
-// for ModDown) computed where ModDown reads it: the P slots' products in the
-// load of the inverse NTT's first pass, the Q slots' in the store of the
-// forward NTT's last pass (with the combine mode, the b term and the
-// subtraction of the NTT'd contribution).  The products are neither written
-// nor read back.  Each sum holds PARTS <= 3 canonical products (below q
-// 2^64: REDC's precondition), reduced once.
-template <bool MONT, int PARTS>
-__device__ __forceinline__ u64 key_product(const u64* dig, long long dstep, const u64* key, long long kstep, int i,
-                                           const BasisConst& b) {
-    U128 s{0, 0};
-#pragma unroll
-    for (int d = 0; d < PARTS; ++d) mac128(s, reduce_4q(dig[d * dstep + i], b.q), reduce_4q(key[d * kstep + i], b.q));
-    return MONT ? redc128(s.lo, s.hi, b.q, b.qninv) : reduce128(s.lo, s.hi, b.q, b.mu_lo, b.mu_hi);
-}
-
-struct KeyProductLists {
-    const u64* digits;  // item i's digits at digits + i * dstride: [parts][L+K][N]
-    long long dstride;
-    const u64* key[KS_MAX_ITEMS];
-    int L, K, nq;
-    u64 N;
-    const BasisConst* bc;
-    // slot `slot` of poly k (even: a, odd: b) of item k / 2
-    __device__ void at(int k, int slot, int basis, const u64*& dig, const u64*& key_p) const {
-        const int item = k >> 1;
-        dig = digits + item * dstride + (long long)slot * N;
-        key_p = key[item] + ((long long)((k & 1) ? 0 : nq + K) + basis) * N;
-    }
-};
-
-// inverse NTT first (row) pass over the P slots: load = key product
-template <bool MONT, int PARTS>
-struct MacPJob {
-    KeyProductLists kp;
-    u64* p[2 * KS_MAX_ITEMS];  // poly k's P accumulator (K limbs)
-    int npoly;
-    FastDiv per_limb;  // npoly
-    struct View {
-        int basis;
-        u64* p;
-        const u64* dig;
-        const u64* key;
-        long long dstep, kstep;
-        BasisConst b;
-        __device__ u64 load(int i) const { return key_product<MONT, PARTS>(dig, dstep, key, kstep, i, b); }
-        __device__ void store(int i, u64 v) const { p[i] = v; }
-    };
-    __device__ View view(int k) const {
-        const int pi = per_limb.div(k), poly = k - pi * npoly;
-        const int basis = kp.nq + pi;
-        View v;
-        v.basis = basis;
-        v.p = p[poly] + (long long)pi * kp.N;
-        kp.at(poly, kp.L + pi, basis, v.dig, v.key);
-        v.dstep = (long long)(kp.L + kp.K) * kp.N;
-        v.kstep = 2LL * (kp.nq + kp.K) * kp.N;
-        v.b = kp.bc[basis];
-        return v;
-    }
-    __device__ bool skip(int) const { return false; }
-};
-
-// forward NTT last (row) pass over the Q slots: out = combine(old, key
-// product + b term) - NTT(contribution); old and the b term read from a zero
-// row where the mode assigns / there is no b term
-template <bool MONT, int PARTS>
-struct MdMacOutJob {
-    KeyProductLists kp;
-    const u64* tmp;                        // [npoly][L][N] NTT'd contributions
-    u64* out[2 * KS_MAX_ITEMS];
-    const u64* old[2 * KS_MAX_ITEMS];      // out (add mode) or the zero row
-    const u64* add[2 * KS_MAX_ITEMS];      // the b term or the zero row
-    long long old_step[2 * KS_MAX_ITEMS];  // limb step of old / add: N, or 0 for the zero row
-    long long add_step[2 * KS_MAX_ITEMS];
-    int npoly;
-    FastDiv per_limb;  // npoly
-    struct View {
-        int basis;
-        const u64* src;
-        u64* out;
-        const u64* old;
-        const u64* add;
-        const u64* dig;
-        const u64* key;
-        long long dstep, kstep;
-        BasisConst b;
-        __device__ u64 load(int i) const { return src[i]; }
-        __device__ u64 pre(int i) const { return add_mod(old[i], add[i], b.q); }
-        __device__ void store_pre(int i, u64 v, u64 base) const {
-            const u64 acc = add_mod(key_product<MONT, PARTS>(dig, dstep, key, kstep, i, b), base, b.q);
-            out[i] = sub_mod(acc, v, b.q);
-        }
-    };
-    __device__ View view(int k) const {
-        const int t = per_limb.div(k), poly = k - t * npoly;
-        View v;
-        v.basis = t;
-        v.src = tmp + ((long long)poly * kp.L + t) * kp.N;
-        v.out = out[poly] + (long long)t * kp.N;
-        v.old = old[poly] + (long long)t * old_step[poly];
-        v.add = add[poly] + (long long)t * add_step[poly];
-        kp.at(poly, t, t, v.dig, v.key);
-        v.dstep = (long long)(kp.L + kp.K) * kp.N;
-        v.kstep = 2LL * (kp.nq + kp.K) * kp.N;
-        v.b = kp.bc[t];
-        return v;
-    }
-    __device__ bool skip(int) const { return false; }
-};
-
-template <bool MONT, int PARTS>
-void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,
-                   u64* T, hipStream_t s) {
-    const int L = level + 1, K = c.np, npoly = 2 * n;
-    const u64 N = c.N;
-    KeyProductLists kp{};
-    kp.digits = D;
-    kp.dstride = dstride;
-    for (int i = 0; i < n; ++i) kp.key[i] = items[i].key;
-    kp.L = L;
-    kp.K = K;
-    kp.nq = c.nq;
-    kp.N = N;
-    kp.bc = c.d_bc;
-    u64* p[2 * KS_MAX_ITEMS];
-    for (int i = 0; i < n; ++i) {
-        p[2 * i] = AP + (size_t)i * 2 * K * N;
-        p[2 * i + 1] = p[2 * i] + (size_t)K * N;
-    }
-    {
-        MacPJob<MONT, PARTS> in{};
-        in.kp = kp;
-        for (int k = 0; k < npoly; ++k) in.p[k] = p[k];
-        in.npoly = npoly;
-        in.per_limb = fast_div(npoly);
-        ListJob o{};
-        for (int k = 0; k < npoly; ++k) o.p[k] = p[k];
-        o.npoly = npoly;
-        o.per_limb = fast_div(npoly);
-        o.basis0 = c.nq;
-        o.N = N;
-        const long long probe = c.probe_open(s, K * npoly);
-        launch_rows_w4<false>(c, in, K * npoly, s);
-        launch_pass<false, false>(c, o, K * npoly, s);
-        c.probe_close(probe, s);
-    }
-    MdContribArgs a{};
-    for (int k = 0; k < npoly; ++k) a.src[k] = p[k];
-    a.tmp = T;
-    a.pinv = c.moddown[level].pinv;
-    a.L = L;
-    a.K = K;
-    a.nq = c.nq;
-    a.logN = c.logN;
-    a.bc = c.d_bc;
-    dim3 grid((unsigned)(N / KS_THREADS), npoly, (L + MODDOWN_TCH - 1) / MODDOWN_TCH);
-    switch (K) {
-#define MI_MODDOWN_CASE(KK) \
-        case KK: hipLaunchKernelGGL(k_moddown_contrib<KK>, grid, dim3(KS_THREADS), 0, s, a); break;
-        MI_NS_CASES(MI_MODDOWN_CASE)
-#undef MI_MODDOWN_CASE
-        default: throw Error(-1, "more than 16 special moduli");
-    }
-    MI_HIP(hipGetLastError());
-    MdInJob in{T, L, npoly, N, fast_div(npoly)};
-    MdMacOutJob<MONT, PARTS> o{};
-    o.kp = kp;
-    o.tmp = T;
-    for (int i = 0; i < n; ++i) {
-        const KsItem& it = items[i];
-        // poly 2i: a, poly 2i+1: b
-        o.out[2 * i] = it.a_out;
-        o.out[2 * i + 1] = it.b_out;
-        o.old[2 * i] = it.a_mode == 0 ? it.a_out : c.d_zero;
-        o.old_step[2 * i] = it.a_mode == 0 ? (long long)N : 0;
-        o.old[2 * i + 1] = it.b_mode == 0 ? it.b_out : c.d_zero;
-        o.old_step[2 * i + 1] = it.b_mode == 0 ? (long long)N : 0;
-        o.add[2 * i] = c.d_zero;
-        o.add_step[2 * i] = 0;
-        o.add[2 * i + 1] = it.init_b ? it.init_b : c.d_zero;
-        o.add_step[2 * i + 1] = it.init_b ? (long long)N : 0;
-    }
-    o.npoly = npoly;
-    o.per_limb = fast_div(npoly);
-    const long long probe = c.probe_open(s, npoly * L);
-    launch_pass<true, false>(c, in, npoly * L, s);
-    launch_rows_w4<true>(c, o, npoly * L, s);
-    c.probe_close(probe, s);
-}
-
-void ks_moddown_mac(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,
-                    u64* T, bool montgomery, hipStream_t s) {
-    if (n < 1 || n > KS_MAX_ITEMS) throw Error(-1, "key switch batch size out of range");
-    if (c.np > MAX_ALPHA) throw Error(-1, "more than 16 special moduli");
-    const int parts = c.parts(level);
-#define MI_MDMAC(M, PP) moddown_mac_t<M, PP>(c, level, n, items, D, dstride, AP, T, s)
-    if (montgomery) {
-        if (parts == 1) MI_MDMAC(true, 1);
-        else if (parts == 2) MI_MDMAC(true, 2);
-        else if (parts == 3) MI_MDMAC(true, 3);
-        else throw Error(-1, "folded key product takes at most 3 digits");
-    } else {
-        if (parts == 1) MI_MDMAC(false, 1);
-        else if (parts == 2) MI_MDMAC(false, 2);
-        else if (parts == 3) MI_MDMAC(false, 3);
-        else throw Error(-1, "folded key product takes at most 3 digits");
-    }
-#undef MI_MDMAC
 }
 
 // ---------------------------------------------------------------- entry points

@@ -13,6 +13,33 @@
 
 namespace mi {
 
+namespace {
+template <bool FWD, bool ROWS>
+void plain_pass(const Context& c, int variant, const PlainJob& job, int count, hipStream_t s) {
+    switch (variant) {
+        case 2:
+            if constexpr (ROWS) launch_rows<FWD, 2, false>(c, job, count, s);
+            else launch_cols<FWD, 2, false>(c, job, count, s);
+            break;
+        case 3:
+            if constexpr (ROWS) launch_rows<FWD, 1, true>(c, job, count, s);
+            else launch_cols<FWD, 1, true>(c, job, count, s);
+            break;
+        default:
+            if constexpr (ROWS) launch_rows<FWD, 1, false>(c, job, count, s);
+            else launch_cols<FWD, 1, false>(c, job, count, s);
+    }
+}
+}  // namespace
+
+void launch_plain_pass(const Context& c, bool fwd, bool rows, int variant, const PlainJob& job, int count,
+                       hipStream_t s) {
+    if (fwd && rows) plain_pass<true, true>(c, variant, job, count, s);
+    else if (fwd) plain_pass<true, false>(c, variant, job, count, s);
+    else if (rows) plain_pass<false, true>(c, variant, job, count, s);
+    else plain_pass<false, false>(c, variant, job, count, s);
+}
+
 void ntt_forward(const Context& c, const LimbBatch& b, hipStream_t s) {
     if (b.count <= 0) return;
     const PlainJob j = plain_job(b, c.N);

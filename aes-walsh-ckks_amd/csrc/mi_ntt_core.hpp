@@ -11,6 +11,7 @@
 // thread-local.  Twiddle indices are the reference's global table indices.
 #pragma once
 #include "mi_arith.hpp"
+#include "mi_internal.hpp"
 
 namespace mi {
 
@@ -23,29 +24,96 @@ constexpr int NTT_LDS_WORDS = NTT_THREADS * E + NTT_THREADS + 128;
 
 __device__ __forceinline__ int lpad(int p) { return p + (p >> LOGE); }
 
-// Modulus constants of one limb for the butterflies: q2 = 2q, and the
-// negations negq = 2^64 - q (read from the basis table) and negq2 = 2^64 - 2q,
-// so conditional subtractions become selects of a 64-bit add.
-struct BfConst {
-    u64 q2, negq, negq2;
+// Butterfly arithmetic of one limb, chosen by its modulus (BasisConst::fp).
+// A word travels through registers, LDS and the intermediate between the two
+// passes as 64 bits; a policy says what the bits mean.
+//
+// BfInt (any q < 2^62): Harvey lazy residues, Shoup products.  q2 = 2q, and
+// the negations negq = 2^64 - q (read from the basis table) and negq2 =
+// 2^64 - 2q, so conditional subtractions become selects of a 64-bit add.
+struct BfInt {
+    u64 q, q2, negq, negq2;
+    static __device__ __forceinline__ BfInt of(const BasisConst& b) {
+        return BfInt{b.q, b.q << 1, b.negq, b.negq << 1};
+    }
+    __device__ __forceinline__ u64 in(u64 x) const { return x; }  // canonical -> working form
+    // Forward (DIT, Harvey lazy): x0,x1 in [0,4q) -> [0,4q).
+    __device__ __forceinline__ void fwd(u64& x0, u64& x1, u64 w, u64 ws) const {
+        const u64 t = x0 >= q2 ? x0 + negq2 : x0;
+        const u64 u = shoup_lazy_neg(x1, w, ws, negq);
+        x0 = t + u;
+        x1 = t + q2 - u;
+    }
+    // Inverse (DIF): x0,x1 in [0,2q) -> [0,2q).
+    __device__ __forceinline__ void inv(u64& x0, u64& x1, u64 w, u64 ws) const {
+        const u64 t = x0, u = x1;
+        const u64 s = t + u;
+        x1 = shoup_lazy_neg(t - u + q2, w, ws, negq);
+        x0 = s >= q2 ? s + negq2 : s;
+    }
+    // Range control between sub-stages: the butterflies above need none.
+    template <int D>
+    __device__ __forceinline__ void tame(u64 (&)[E], bool) const {}
+    __device__ __forceinline__ u64 out_fwd(u64 x) const { return reduce_4q(x, q); }
+    // Last inverse stage (distance N/2) with the N^-1 scaling, canonical:
+    // x0 = (x0 + x1) N^-1, x1 = (x0 - x1) w_1 N^-1.
+    __device__ __forceinline__ void inv_last(u64& x0, u64& x1, const BasisConst& b) const {
+        const u64 s = x0 + x1, d = x0 - x1 + q2;
+        x0 = shoup(s, b.n_inv, b.n_inv_shoup, q);
+        x1 = shoup(d, b.w1_ninv, b.w1_ninv_shoup, q);
+    }
 };
-__device__ __forceinline__ BfConst bf_const(u64 q, u64 negq) { return BfConst{q << 1, negq, negq << 1}; }
 
-// Forward (DIT, Harvey lazy): x0,x1 in [0,4q) -> [0,4q).
-__device__ __forceinline__ void bf_fwd(u64& x0, u64& x1, u64 w, u64 ws, const BfConst& k) {
-    const u64 t = x0 >= k.q2 ? x0 + k.negq2 : x0;
-    const u64 u = shoup_lazy_neg(x1, w, ws, k.negq);
-    x0 = t + u;
-    x1 = t + k.q2 - u;
-}
-
-// Inverse (DIF): x0,x1 in [0,2q) -> [0,2q).
-__device__ __forceinline__ void bf_inv(u64& x0, u64& x1, u64 w, u64 ws, const BfConst& k) {
-    const u64 t = x0, u = x1;
-    const u64 s = t + u;
-    x1 = shoup_lazy_neg(t - u + k.q2, w, ws, k.negq);
-    x0 = s >= k.q2 ? s + k.negq2 : s;
-}
+// BfFp (q < 2^50): the integer-valued doubles of FpMod, at most 8q < 2^53 in
+// magnitude.  A twiddle product is six full-rate FP64 instructions against
+// the fourteen of a Shoup product (measured on the device: 6.3e12 against
+// 2.8e12 products/s); a butterfly takes 8 instructions instead of 25.
+//
+// Ranges, in units of q, with |x| 2^-53 <= |x|/8 at q = 2^50:
+//   forward: a stage adds at most 1/2 + B/8 to the bound B.  Inputs up to 4,
+//     5, 6.1, reduced to 1/2 after two stages (`tame`), then 1.1, 1.7, 2.4,
+//     3.2, 4.1, 5.1 after the pass; the second pass enters at 5.1, 6.2, 7.5,
+//     reduced, and leaves at 5.1.
+//   inverse: a stage doubles the sums.  Inputs up to 2: 4, 8, the sums
+//     reduced after every second stage and after the pass's last one, the
+//     differences' products at most 3/2; then 3, 6, ... again.
+// Below 2^44 (`wide` false) the bounds hold without the reductions inside a
+// pass: forward 1 + 16 (1/2 + 2^-5) < 10 q; inverse 2^8 q <= 2^52 after
+// eight doublings, reduced at the end of the pass.
+constexpr u64 FP_WIDE = 1ull << 44;
+struct BfFp {
+    FpMod m;
+    bool wide;
+    static __device__ __forceinline__ BfFp of(const BasisConst& b) { return BfFp{{b.qd, b.inv_d}, b.q >= FP_WIDE}; }
+    static __device__ __forceinline__ double d(u64 x) { return __builtin_bit_cast(double, x); }
+    static __device__ __forceinline__ u64 u(double x) { return __builtin_bit_cast(u64, x); }
+    __device__ __forceinline__ u64 in(u64 x) const { return u(fp_from_u64(x)); }
+    __device__ __forceinline__ void fwd(u64& x0, u64& x1, u64 w, u64 ws) const {
+        const double t = d(x0), r = m.mul(d(x1), d(w), d(ws));
+        x0 = u(t + r);
+        x1 = u(t - r);
+    }
+    __device__ __forceinline__ void inv(u64& x0, u64& x1, u64 w, u64 ws) const {
+        const double s = d(x0) + d(x1), r = m.mul(d(x0) - d(x1), d(w), d(ws));
+        x0 = u(s);
+        x1 = u(r);
+    }
+    // Reduces the words j with (j & D) == 0 (all of them for D = 0) where the
+    // modulus needs it there (`always`) or is wide.
+    template <int D>
+    __device__ __forceinline__ void tame(u64 (&x)[E], bool always) const {
+        if (!always && !wide) return;  // uniform over the workgroup
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+            if ((j & D) == 0) x[j] = u(m.centred(d(x[j])));
+    }
+    __device__ __forceinline__ u64 out_fwd(u64 x) const { return m.canonical(d(x)); }
+    __device__ __forceinline__ void inv_last(u64& x0, u64& x1, const BasisConst& b) const {
+        const double s = d(x0) + d(x1), t = d(x0) - d(x1);
+        x0 = m.canonical(m.mul(s, b.n_inv_fp, b.n_inv_fpq));
+        x1 = m.canonical(m.mul(t, b.w1_ninv_fp, b.w1_ninv_fpq));
+    }
+};
 
 template <int LOGR>
 struct Grp {
@@ -79,73 +147,6 @@ __device__ __forceinline__ void to_strided(u64 (&x)[E], int t, u64* lds) {
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < E; ++j) x[j] = lds[lpad(t + G::TG * j)];
-}
-
-// Forward group transform.  In: strided layout; out: strided layout.
-// idx(s, i) gives the global twiddle index of group sub-stage s, block i.
-template <int LOGR, class IDX>
-__device__ __forceinline__ void group_fwd(u64 (&x)[E], int t, u64* lds, const BfConst& kq,
-                                          const u64* __restrict__ W, const u64* __restrict__ WS,
-                                          IDX idx) {
-    using G = Grp<LOGR>;
-#pragma unroll
-    for (int s = 0; s < LOGE; ++s) {
-        const int dj = E >> (s + 1);
-#pragma unroll
-        for (int j0 = 0; j0 < E; ++j0) {
-            if (j0 & dj) continue;
-            const int k = idx(s, j0 >> (LOGE - s));
-            bf_fwd(x[j0], x[j0 + dj], W[k], WS[k], kq);
-        }
-    }
-    __syncthreads();
-    to_contiguous<LOGR>(x, t, lds);
-#pragma unroll
-    for (int s = LOGE; s < LOGR; ++s) {
-        const int d = G::R >> (s + 1);
-#pragma unroll
-        for (int j0 = 0; j0 < E; ++j0) {
-            if (j0 & d) continue;
-            const int k = idx(s, (t * E + j0) >> (LOGR - s));
-            bf_fwd(x[j0], x[j0 + d], W[k], WS[k], kq);
-        }
-    }
-    __syncthreads();
-    to_strided<LOGR>(x, t, lds);
-}
-
-// Inverse group transform.  In: strided layout; out: strided layout.
-// idx(u, i): global twiddle index for group sub-stage u (distance 2^u), block i.
-// LAST = false leaves the last sub-stage (pairs j, j + E/2) to the caller.
-template <int LOGR, bool LAST = true, class IDX>
-__device__ __forceinline__ void group_inv(u64 (&x)[E], int t, u64* lds, const BfConst& kq,
-                                          const u64* __restrict__ W, const u64* __restrict__ WS,
-                                          IDX idx) {
-    using G = Grp<LOGR>;
-    __syncthreads();
-    to_contiguous<LOGR>(x, t, lds);
-#pragma unroll
-    for (int u = 0; u < LOGE; ++u) {
-        const int d = 1 << u;
-#pragma unroll
-        for (int j0 = 0; j0 < E; ++j0) {
-            if (j0 & d) continue;
-            const int k = idx(u, (t * E + j0) >> (u + 1));
-            bf_inv(x[j0], x[j0 + d], W[k], WS[k], kq);
-        }
-    }
-    __syncthreads();
-    to_strided<LOGR>(x, t, lds);
-#pragma unroll
-    for (int u = LOGE; u < (LAST ? LOGR : LOGR - 1); ++u) {
-        const int dj = 1 << (u - G::LOGTG);
-#pragma unroll
-        for (int j0 = 0; j0 < E; ++j0) {
-            if (j0 & dj) continue;
-            const int k = idx(u, j0 >> (u + 1 - G::LOGTG));
-            bf_inv(x[j0], x[j0 + dj], W[k], WS[k], kq);
-        }
-    }
 }
 
 // The same exchanges through 32-bit LDS words, the low halves and then the
@@ -218,8 +219,10 @@ struct TwPre {
     u64 w[NT], ws[NT];
 };
 
-template <int LOGR, int LPB, class IDX, class LW>
-__device__ __forceinline__ void group_fwd_n(u64 (&x)[LPB][E], int t, LW* lds, const BfConst (&kq)[LPB],
+// Forward group transform.  In and out: strided layout.  idx(s, i) gives the
+// global twiddle index of group sub-stage s, block i.
+template <int LOGR, int LPB, class BF, class IDX, class LW>
+__device__ __forceinline__ void group_fwd_n(u64 (&x)[LPB][E], int t, LW* lds, const BF (&kq)[LPB],
                                             const u64* const (&W)[LPB], const u64* const (&WS)[LPB], IDX idx) {
     using G = Grp<LOGR>;
 #pragma unroll
@@ -230,7 +233,11 @@ __device__ __forceinline__ void group_fwd_n(u64 (&x)[LPB][E], int t, LW* lds, co
             if (j0 & dj) continue;
             const int k = idx(s, j0 >> (LOGE - s));
 #pragma unroll
-            for (int i = 0; i < LPB; ++i) bf_fwd(x[i][j0], x[i][j0 + dj], W[i][k], WS[i][k], kq[i]);
+            for (int i = 0; i < LPB; ++i) kq[i].fwd(x[i][j0], x[i][j0 + dj], W[i][k], WS[i][k]);
+        }
+        if (s == 1) {
+#pragma unroll
+            for (int i = 0; i < LPB; ++i) kq[i].template tame<0>(x[i], false);
         }
     }
     // first contiguous sub-stage (s = LOGE): twiddle (t*E + j0) >> (LOGR - LOGE)
@@ -253,20 +260,23 @@ __device__ __forceinline__ void group_fwd_n(u64 (&x)[LPB][E], int t, LW* lds, co
         for (int j0 = 0; j0 < E; ++j0) {
             if (j0 & d) continue;
             if (LPB == 1 && s == LOGE) {
-                bf_fwd(x[0][j0], x[0][j0 + d], pf.w[j0 >> SH], pf.ws[j0 >> SH], kq[0]);
+                kq[0].fwd(x[0][j0], x[0][j0 + d], pf.w[j0 >> SH], pf.ws[j0 >> SH]);
                 continue;
             }
             const int k = idx(s, (t * E + j0) >> (LOGR - s));
 #pragma unroll
-            for (int i = 0; i < LPB; ++i) bf_fwd(x[i][j0], x[i][j0 + d], W[i][k], WS[i][k], kq[i]);
+            for (int i = 0; i < LPB; ++i) kq[i].fwd(x[i][j0], x[i][j0 + d], W[i][k], WS[i][k]);
         }
     }
     __syncthreads();
     to_strided_n<LOGR, LPB>(x, t, lds);
 }
 
-template <int LOGR, bool LAST, int LPB, class IDX, class LW>
-__device__ __forceinline__ void group_inv_n(u64 (&x)[LPB][E], int t, LW* lds, const BfConst (&kq)[LPB],
+// Inverse group transform.  In and out: strided layout.  idx(u, i): global
+// twiddle index of group sub-stage u (distance 2^u), block i.  LAST = false
+// leaves the last sub-stage (pairs j, j + E/2) to the caller.
+template <int LOGR, bool LAST, int LPB, class BF, class IDX, class LW>
+__device__ __forceinline__ void group_inv_n(u64 (&x)[LPB][E], int t, LW* lds, const BF (&kq)[LPB],
                                             const u64* const (&W)[LPB], const u64* const (&WS)[LPB], IDX idx) {
     using G = Grp<LOGR>;
     // first contiguous sub-stage (u = 0): twiddle (t*E + j0) >> 1
@@ -289,12 +299,17 @@ __device__ __forceinline__ void group_inv_n(u64 (&x)[LPB][E], int t, LW* lds, co
         for (int j0 = 0; j0 < E; ++j0) {
             if (j0 & d) continue;
             if (LPB == 1 && u == 0) {
-                bf_inv(x[0][j0], x[0][j0 + d], pc.w[j0 >> 1], pc.ws[j0 >> 1], kq[0]);
+                kq[0].inv(x[0][j0], x[0][j0 + d], pc.w[j0 >> 1], pc.ws[j0 >> 1]);
                 continue;
             }
             const int k = idx(u, (t * E + j0) >> (u + 1));
 #pragma unroll
-            for (int i = 0; i < LPB; ++i) bf_inv(x[i][j0], x[i][j0 + d], W[i][k], WS[i][k], kq[i]);
+            for (int i = 0; i < LPB; ++i) kq[i].inv(x[i][j0], x[i][j0 + d], W[i][k], WS[i][k]);
+        }
+#pragma unroll
+        for (int i = 0; i < LPB; ++i) {
+            if (u == 1) kq[i].template tame<2>(x[i], false);
+            if (u == 3) kq[i].template tame<8>(x[i], false);
         }
     }
     // first strided sub-stage (u = LOGE): twiddle j0 >> (LOGE + 1 - LOGTG)
@@ -318,24 +333,24 @@ __device__ __forceinline__ void group_inv_n(u64 (&x)[LPB][E], int t, LW* lds, co
         for (int j0 = 0; j0 < E; ++j0) {
             if (j0 & dj) continue;
             if (LPB == 1 && u == LOGE) {
-                bf_inv(x[0][j0], x[0][j0 + dj], ps.w[j0 >> SS], ps.ws[j0 >> SS], kq[0]);
+                kq[0].inv(x[0][j0], x[0][j0 + dj], ps.w[j0 >> SS], ps.ws[j0 >> SS]);
                 continue;
             }
             const int k = idx(u, j0 >> (u + 1 - G::LOGTG));
 #pragma unroll
-            for (int i = 0; i < LPB; ++i) bf_inv(x[i][j0], x[i][j0 + dj], W[i][k], WS[i][k], kq[i]);
+            for (int i = 0; i < LPB; ++i) kq[i].inv(x[i][j0], x[i][j0 + dj], W[i][k], WS[i][k]);
+        }
+        if ((u & 1) || (LAST && u == LOGR - 1)) {
+#pragma unroll
+            for (int i = 0; i < LPB; ++i) {
+                const bool last = LAST && u == LOGR - 1;
+                if (dj == 1) kq[i].template tame<1>(x[i], last);
+                if (dj == 2) kq[i].template tame<2>(x[i], last);
+                if (dj == 4) kq[i].template tame<4>(x[i], last);
+                if (dj == 8) kq[i].template tame<8>(x[i], last);
+            }
         }
     }
 }
-
-// Geometry of one pass.  Column passes: group = column (stride R2 words
-// between elements), thread (g = tid % G, t = tid / G).  Row passes: group =
-// contiguous block of R2 words, thread (g = tid / TG, t = tid % TG).
-struct PassGeom {
-    int n, n1, n2;
-    int threads;     // workgroup size
-    int groups;      // groups per workgroup
-    int wg_per_limb; // workgroups per limb
-};
 
 }  // namespace mi

@@ -12,10 +12,18 @@
 // for its output positions together with its input, before the butterflies,
 // and stores through store_pre, so an output that combines the transform
 // with another operand does not wait for that operand's loads at the end.
-// Forward column pass: load = job input, store = intermediate ([0,4q)).
+// For limbs in double arithmetic (BasisConst::fp) a View of a first pass may
+// offer `double load_fp(int i) const`, its input as an integer-valued double
+// below q in magnitude, and a View of a forward transform's second pass
+// `void store_fp(int i, double x, u64 pre) const` (`pre` as above, else 0),
+// which takes the transform's output x before it is made canonical
+// (|x| < 5.2q) and stores the canonical result.
+// Forward column pass: load = job input, store = intermediate.
 // Forward row pass: load = intermediate, store = canonical output.
-// Inverse row pass: load = input (canonical), store = intermediate ([0,2q)).
+// Inverse row pass: load = input (canonical), store = intermediate.
 // Inverse column pass: load = intermediate, store = canonical output.
+// The intermediate is in the working form of the limb's modulus (lazy residues
+// or doubles, mi_ntt_core.hpp): the two passes only hand it to each other.
 #pragma once
 #include <type_traits>
 #include "mi_internal.hpp"
@@ -30,10 +38,21 @@ struct NttTabs {
     const u64* inv_shoup;
     const BasisConst* bc;
     u64 N;
+    // BasisConst::fp of the first 128 basis indices as kernel arguments: the
+    // choice of the arithmetic comes before the first data load and must not
+    // wait for a table (reading it from bc cost the 60-bit batch 2 %).
+    u64 fp_mask[2];
+    __device__ __forceinline__ bool fp(int basis) const {
+        if (basis >= 128) return bc[basis].fp != 0;
+        return ((basis < 64 ? fp_mask[0] : fp_mask[1]) >> (basis & 63)) & 1;
+    }
 };
 
 inline NttTabs tabs_of(const Context& c) {
-    return NttTabs{c.d_fwd, c.d_fwd_shoup, c.d_inv, c.d_inv_shoup, c.d_bc, c.N};
+    NttTabs t{c.d_fwd, c.d_fwd_shoup, c.d_inv, c.d_inv_shoup, c.d_bc, c.N, {0, 0}};
+    for (int b = 0; b < c.nb() && b < 128; ++b)
+        if (c.h_bc[b].fp) t.fp_mask[b >> 6] |= 1ull << (b & 63);
+    return t;
 }
 
 // In-place NTT over a strided batch.  Workgroups walk the batch modulus-major
@@ -74,6 +93,14 @@ template <class V, class = void>
 struct HasPre : std::false_type {};
 template <class V>
 struct HasPre<V, std::void_t<decltype(&V::pre)>> : std::true_type {};
+template <class V, class = void>
+struct HasLoadFp : std::false_type {};
+template <class V>
+struct HasLoadFp<V, std::void_t<decltype(&V::load_fp)>> : std::true_type {};
+template <class V, class = void>
+struct HasStoreFp : std::false_type {};
+template <class V>
+struct HasStoreFp<V, std::void_t<decltype(&V::store_fp)>> : std::true_type {};
 
 // LPB limbs per workgroup (1 or 2): workgroup b serves limbs LPB*(b / wpl) +
 // 0..LPB-1 of a launch over `count` limbs; a limb past `count` or skipped by
@@ -95,134 +122,131 @@ __device__ __forceinline__ bool limb_views(const Job& job, int first, int count,
     return true;
 }
 
-template <int LOGN, bool FWD, int LPB, bool HALF, class Job>
-__global__ void __launch_bounds__(NTT_THREADS)
-k_ntt_cols(NttTabs tb, Job job, int count) {
-    constexpr int n1 = LOGN / 2, n2 = LOGN - n1, LOGR = n1;
-    constexpr int G = pass_groups(n1, n2), wpl = pass_wpl(n1, n2);
-    using LW = std::conditional_t<HALF, u32, u64>;  // LDS exchange word
-    __shared__ LW lds[NTT_LDS_WORDS];
+// One pass over the LPB limbs of a workgroup in the arithmetic BF (all of
+// them; see mi_ntt_core.hpp).  Column pass (ROWS false): the groups are the
+// limb's columns (stride 2^n2); row pass: its contiguous blocks of 2^n2.  The
+// first pass of a transform (FWD columns, inverse rows) converts the input to
+// the working form, the second one gives canonical residues.
+template <int LOGN, bool FWD, bool ROWS, int LPB, class BF, class LW, class V>
+__device__ __forceinline__ void pass_body(const NttTabs& tb, const V (&v)[LPB], const bool (&live)[LPB], int w,
+                                          LW* lds) {
+    constexpr int n1 = LOGN / 2, n2 = LOGN - n1, LOGR = ROWS ? n2 : n1;
+    constexpr int G = pass_groups(LOGR, LOGN - LOGR);
     using Gr = Grp<LOGR>;
-    using V = decltype(job.view(0));
-    const int blk = blockIdx.x / wpl, w = blockIdx.x - blk * wpl;
-    V v[LPB];
-    bool live[LPB];
-    if (!limb_views<LPB>(job, blk * LPB, count, v, live)) return;
-    const int g = threadIdx.x % G, t = threadIdx.x / G;
-    const int col = w * G + g;
+    const int g = ROWS ? threadIdx.x / Gr::TG : threadIdx.x % G;
+    const int t = ROWS ? threadIdx.x % Gr::TG : threadIdx.x / G;
+    const int grp = w * G + g;
+    auto at = [grp, t](int j) {
+        return ROWS ? (grp << n2) + t + Gr::TG * j : ((t + Gr::TG * j) << n2) + grp;
+    };
+    constexpr bool FIRST = FWD != ROWS;
+    constexpr bool FP = std::is_same_v<BF, BfFp>;
     constexpr bool PRE = HasPre<V>::value;
+    constexpr bool LOAD_FP = FP && FIRST && HasLoadFp<V>::value;
+    constexpr bool STORE_FP = FP && FWD && !FIRST && HasStoreFp<V>::value;
     u64 x[LPB][E], pre[LPB][PRE ? E : 1];
-    BasisConst bc[LPB];
-    BfConst kq[LPB];
+    BF kq[LPB];
     const u64* W[LPB];
     const u64* WS[LPB];
 #pragma unroll
     for (int i = 0; i < LPB; ++i) {
+        kq[i] = BF::of(tb.bc[v[i].basis]);
         if (live[i]) {
 #pragma unroll
-            for (int j = 0; j < E; ++j) x[i][j] = v[i].load(((t + Gr::TG * j) << n2) + col);
+            for (int j = 0; j < E; ++j) {
+                if constexpr (LOAD_FP) x[i][j] = BfFp::u(v[i].load_fp(at(j)));
+                else x[i][j] = FIRST ? kq[i].in(v[i].load(at(j))) : v[i].load(at(j));
+            }
             if constexpr (PRE) {
 #pragma unroll
-                for (int j = 0; j < E; ++j) pre[i][j] = v[i].pre(((t + Gr::TG * j) << n2) + col);
+                for (int j = 0; j < E; ++j) pre[i][j] = v[i].pre(at(j));
             }
         }
-        bc[i] = tb.bc[v[i].basis];
-        kq[i] = bf_const(bc[i].q, bc[i].negq);
         W[i] = (FWD ? tb.fwd : tb.inv) + (long long)v[i].basis * tb.N;
         WS[i] = (FWD ? tb.fwd_shoup : tb.inv_shoup) + (long long)v[i].basis * tb.N;
     }
     LW* my = lds + g * Gr::LDS;
     if constexpr (FWD) {
-        group_fwd_n<LOGR, LPB>(x, t, my, kq, W, WS, [](int s, int i) { return (1 << s) + i; });
+        if constexpr (ROWS)
+            group_fwd_n<LOGR, LPB>(x, t, my, kq, W, WS,
+                                   [grp](int s, int i) { return (1 << (n1 + s)) + (grp << s) + i; });
+        else
+            group_fwd_n<LOGR, LPB>(x, t, my, kq, W, WS, [](int s, int i) { return (1 << s) + i; });
     } else {
-        group_inv_n<LOGR, false, LPB>(x, t, my, kq, W, WS, [](int u, int i) { return (1 << (n1 - 1 - u)) + i; });
-        // last stage (distance N/2, twiddle index 1) with the N^-1 scaling:
-        // x0 = (t + u) N^-1, x1 = (t - u) w_1 N^-1, canonical
-#pragma unroll
-        for (int i = 0; i < LPB; ++i) {
-            const u64 q2 = bc[i].q << 1;
-#pragma unroll
-            for (int j = 0; j < E / 2; ++j) {
-                const u64 a = x[i][j], b = x[i][j + E / 2];
-                x[i][j] = shoup(a + b, bc[i].n_inv, bc[i].n_inv_shoup, bc[i].q);
-                x[i][j + E / 2] = shoup(a - b + q2, bc[i].w1_ninv, bc[i].w1_ninv_shoup, bc[i].q);
-            }
-        }
+        if constexpr (ROWS)
+            group_inv_n<LOGR, true, LPB>(x, t, my, kq, W, WS, [grp](int u, int i) {
+                return (1 << (LOGN - 1 - u)) + (grp << (n2 - 1 - u)) + i;
+            });
+        else
+            group_inv_n<LOGR, false, LPB>(x, t, my, kq, W, WS, [](int u, int i) { return (1 << (n1 - 1 - u)) + i; });
     }
 #pragma unroll
     for (int i = 0; i < LPB; ++i) {
         if (!live[i]) continue;
+        if constexpr (STORE_FP) {
+#pragma unroll
+            for (int j = 0; j < E; ++j) v[i].store_fp(at(j), BfFp::d(x[i][j]), PRE ? pre[i][PRE ? j : 0] : 0);
+            continue;
+        }
+        if constexpr (!FIRST && FWD) {
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[i][j] = kq[i].out_fwd(x[i][j]);
+        }
+        if constexpr (!FIRST && !FWD) {
+            const BasisConst b = tb.bc[v[i].basis];
+#pragma unroll
+            for (int j = 0; j < E / 2; ++j) kq[i].inv_last(x[i][j], x[i][j + E / 2], b);
+        }
 #pragma unroll
         for (int j = 0; j < E; ++j) {
-            if constexpr (PRE) v[i].store_pre(((t + Gr::TG * j) << n2) + col, x[i][j], pre[i][j]);
-            else v[i].store(((t + Gr::TG * j) << n2) + col, x[i][j]);
+            if constexpr (PRE) v[i].store_pre(at(j), x[i][j], pre[i][j]);
+            else v[i].store(at(j), x[i][j]);
         }
     }
 }
 
-template <int LOGN, bool FWD, int LPB, bool HALF, class Job>
-__device__ __forceinline__ void ntt_rows_body(const NttTabs& tb, const Job& job, int count) {
-    constexpr int n1 = LOGN / 2, n2 = LOGN - n1, LOGR = n2;
-    constexpr int G = pass_groups(n2, n1), wpl = pass_wpl(n2, n1);
+// A workgroup's limbs (limb_views) through one pass in the arithmetic of their
+// moduli; two limbs are interleaved only if both are integer limbs.
+template <int LOGN, bool FWD, bool ROWS, int LPB, bool HALF, class Job>
+__device__ __forceinline__ void ntt_pass(const NttTabs& tb, const Job& job, int count) {
+    constexpr int n1 = LOGN / 2, n2 = LOGN - n1;
+    constexpr int wpl = ROWS ? pass_wpl(n2, n1) : pass_wpl(n1, n2);
     using LW = std::conditional_t<HALF, u32, u64>;  // LDS exchange word
     __shared__ LW lds[NTT_LDS_WORDS];
-    using Gr = Grp<LOGR>;
     using V = decltype(job.view(0));
     const int blk = blockIdx.x / wpl, w = blockIdx.x - blk * wpl;
     V v[LPB];
     bool live[LPB];
     if (!limb_views<LPB>(job, blk * LPB, count, v, live)) return;
-    const int g = threadIdx.x / Gr::TG, t = threadIdx.x % Gr::TG;
-    const int row = w * G + g;
-    const int off = row << n2;
-    constexpr bool PRE = HasPre<V>::value;
-    u64 x[LPB][E], pre[LPB][PRE ? E : 1];
-    BasisConst bc[LPB];
-    BfConst kq[LPB];
-    const u64* W[LPB];
-    const u64* WS[LPB];
+    int fp = 0;
 #pragma unroll
-    for (int i = 0; i < LPB; ++i) {
-        if (live[i]) {
-#pragma unroll
-            for (int j = 0; j < E; ++j) x[i][j] = v[i].load(off + t + Gr::TG * j);
-            if constexpr (PRE) {
-#pragma unroll
-                for (int j = 0; j < E; ++j) pre[i][j] = v[i].pre(off + t + Gr::TG * j);
-            }
-        }
-        bc[i] = tb.bc[v[i].basis];
-        kq[i] = bf_const(bc[i].q, bc[i].negq);
-        W[i] = (FWD ? tb.fwd : tb.inv) + (long long)v[i].basis * tb.N;
-        WS[i] = (FWD ? tb.fwd_shoup : tb.inv_shoup) + (long long)v[i].basis * tb.N;
-    }
-    LW* my = lds + g * Gr::LDS;
-    if constexpr (FWD) {
-        group_fwd_n<LOGR, LPB>(x, t, my, kq, W, WS,
-                               [row](int s, int i) { return (1 << (n1 + s)) + (row << s) + i; });
-#pragma unroll
-        for (int i = 0; i < LPB; ++i)
-#pragma unroll
-            for (int j = 0; j < E; ++j) x[i][j] = reduce_4q(x[i][j], bc[i].q);
+    for (int i = 0; i < LPB; ++i) fp += tb.fp(v[i].basis) ? 1 : 0;
+    if constexpr (LPB == 1) {
+        if (fp) pass_body<LOGN, FWD, ROWS, 1, BfFp>(tb, v, live, w, lds);
+        else pass_body<LOGN, FWD, ROWS, 1, BfInt>(tb, v, live, w, lds);
+    } else if (fp == 0) {
+        pass_body<LOGN, FWD, ROWS, LPB, BfInt>(tb, v, live, w, lds);
     } else {
-        group_inv_n<LOGR, true, LPB>(x, t, my, kq, W, WS, [row](int u, int i) {
-            return (1 << (LOGN - 1 - u)) + (row << (n2 - 1 - u)) + i;
-        });
-    }
-#pragma unroll
-    for (int i = 0; i < LPB; ++i) {
-        if (!live[i]) continue;
-#pragma unroll
-        for (int j = 0; j < E; ++j) {
-            if constexpr (PRE) v[i].store_pre(off + t + Gr::TG * j, x[i][j], pre[i][j]);
-            else v[i].store(off + t + Gr::TG * j, x[i][j]);
+        static_assert(LPB == 2, "one or two limbs per workgroup");
+        const bool l1[1] = {true};
+#pragma unroll 1
+        for (int i = 0; i < 2; ++i) {
+            if (!(i ? live[1] : live[0])) continue;  // uniform
+            const V v1[1] = {i ? v[1] : v[0]};
+            __syncthreads();  // the previous limb's LDS reads are done
+            if (tb.fp(v1[0].basis)) pass_body<LOGN, FWD, ROWS, 1, BfFp>(tb, v1, l1, w, lds);
+            else pass_body<LOGN, FWD, ROWS, 1, BfInt>(tb, v1, l1, w, lds);
         }
     }
 }
 
+template <int LOGN, bool FWD, int LPB, bool HALF, class Job>
+__global__ void __launch_bounds__(NTT_THREADS) k_ntt_cols(NttTabs tb, Job job, int count) {
+    ntt_pass<LOGN, FWD, false, LPB, HALF>(tb, job, count);
+}
 template <int LOGN, bool FWD, int LPB, bool HALF, class Job>
 __global__ void __launch_bounds__(NTT_THREADS) k_ntt_rows(NttTabs tb, Job job, int count) {
-    ntt_rows_body<LOGN, FWD, LPB, HALF>(tb, job, count);
+    ntt_pass<LOGN, FWD, true, LPB, HALF>(tb, job, count);
 }
 // The same pass held to 128 VGPRs (four waves per SIMD, the LDS limit), for
 // jobs whose load or store does enough work of its own that the scheduler
@@ -230,7 +254,7 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ntt_rows(NttTabs tb, Job job, i
 template <int LOGN, bool FWD, class Job>
 __global__ void __launch_bounds__(NTT_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 k_ntt_rows_w4(NttTabs tb, Job job, int count) {
-    ntt_rows_body<LOGN, FWD, 1, false>(tb, job, count);
+    ntt_pass<LOGN, FWD, true, 1, false>(tb, job, count);
 }
 
 #define MI_NTT_LOGN_CASES(K)                                                                          \
@@ -283,29 +307,24 @@ void launch_rows_w4(const Context& c, const Job& job, int count, hipStream_t s) 
     MI_HIP(hipGetLastError());
 }
 
-// One pass in the configuration `variant` of the context's NTT plan:
-// 1 = one limb per workgroup, 2 = two limbs per workgroup, 3 = one limb
-// with the LDS exchanges in 32-bit halves.
+// One pass of an in-place batch (mi_ntt.hip) in configuration `variant` of the
+// NTT plan: 1 = one limb per workgroup, 2 = two limbs per workgroup, 3 = one
+// limb with the LDS exchanges in 32-bit halves.
+void launch_plain_pass(const Context& c, bool fwd, bool rows, int variant, const PlainJob& job, int count,
+                       hipStream_t s);
+
+// One pass of a transform: in-place batches in the configuration the
+// context's tuned plan gives for the launch size, the fused jobs with one
+// limb per workgroup.
 template <bool FWD, bool ROWS, class Job>
 void launch_pass(const Context& c, const Job& job, int count, hipStream_t s) {
-    switch (c.ntt_variant(count)) {
-        case 2:
-            if constexpr (ROWS) launch_rows<FWD, 2, false>(c, job, count, s);
-            else launch_cols<FWD, 2, false>(c, job, count, s);
-            break;
-        case 3:
-            if constexpr (ROWS) launch_rows<FWD, 1, true>(c, job, count, s);
-            else launch_cols<FWD, 1, true>(c, job, count, s);
-            break;
-        default:
-            if constexpr (ROWS) launch_rows<FWD, 1, false>(c, job, count, s);
-            else launch_cols<FWD, 1, false>(c, job, count, s);
-    }
+    if constexpr (std::is_same_v<Job, PlainJob>) launch_plain_pass(c, FWD, ROWS, c.ntt_variant(count), job, count, s);
+    else if constexpr (ROWS) launch_rows<FWD, 1, false>(c, job, count, s);
+    else launch_cols<FWD, 1, false>(c, job, count, s);
 }
 
 // Forward NTT: first pass runs job `in` (load input, store intermediate),
-// second pass runs job `out` (load intermediate, store output), each in the
-// configuration the context's tuned plan gives for the launch size.
+// second pass runs job `out` (load intermediate, store output).
 template <class JobIn, class JobOut>
 void run_ntt_fwd(const Context& c, const JobIn& in, const JobOut& out, int count, hipStream_t s) {
     const long probe = c.probe_open(s, count);

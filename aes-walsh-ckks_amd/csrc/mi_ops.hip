@@ -345,10 +345,16 @@ struct RescaleInJob {
         const u64* top;
         u64* out;
         u64 p, half, q, mu_hi;
-        __device__ u64 load(int i) const {
-            u64 s = top[i] + half;
-            if (s >= p) s -= p;
-            return reduce64(s, q, mu_hi);
+        double qd, qinv;
+        __device__ u64 shifted(int i) const {
+            const u64 s = top[i] + half;
+            return s >= p ? s - p : s;
+        }
+        __device__ u64 load(int i) const { return reduce64(shifted(i), q, mu_hi); }
+        __device__ double load_fp(int i) const {
+            const FpMod m{qd, qinv};
+            if (p < (1ull << FP_BITS)) return m.centred(fp_from_u64(shifted(i)));  // uniform
+            return fp_from_u64(load(i));
         }
         __device__ void store(int i, u64 v) const { out[i] = v; }
     };
@@ -356,7 +362,7 @@ struct RescaleInJob {
         const int i = per_limb.div(k), poly = k - i * npolys;  // modulus-major
         const BasisConst b = bc[i];
         return View{i, polys[poly] + (long long)level * N, scratch + ((long long)poly * level + i) * N, p, half,
-                    b.q, b.mu_hi};
+                    b.q, b.mu_hi, b.qd, b.inv_d};
     }
     __device__ bool skip(int) const { return false; }
 };
@@ -378,14 +384,20 @@ struct RescaleOutJob {
         u64* x;
         const u64* half;
         u64 q, ip, ips;
+        double qd, qinv;
         __device__ u64 load(int i) const { return src[i]; }
         __device__ u64 pre(int i) const { return add_mod(x[i], half[i], q); }
         __device__ void store_pre(int i, u64 v, u64 num) const { x[i] = shoup(sub_mod(num, v, q), ip, ips, q); }
+        __device__ void store_fp(int i, double v, u64 num) const {
+            const FpMod m{qd, qinv};
+            const double w = fp_from_u64(ip);  // below q: the quotient is off by at most 1/2 + 6.2/4
+            x[i] = m.canonical(m.mul(fp_from_u64(num) - v, w, w * qinv));
+        }
     };
     __device__ View view(int k) const {
         const int i = per_limb.div(k), poly = k - i * npolys;  // modulus-major
         return View{i, scratch + ((long long)poly * level + i) * N, polys[poly] + (long long)i * N,
-                    half_ntt + (long long)i * N, bc[i].q, inv_p[i], inv_p_shoup[i]};
+                    half_ntt + (long long)i * N, bc[i].q, inv_p[i], inv_p_shoup[i], bc[i].qd, bc[i].inv_d};
     }
     __device__ bool skip(int) const { return false; }
 };

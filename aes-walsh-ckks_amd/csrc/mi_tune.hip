@@ -1,6 +1,6 @@
 // Autotuner for the launch shapes that have more than one configuration:
-//   * the NTT passes' limbs per workgroup (1 or 2), per ring dimension and
-//     launch size (six buckets of limbs per launch);
+//   * the in-place NTT passes' limbs per workgroup (1 or 2), per ring dimension
+//     and launch size (six buckets of limbs per launch);
 //   * the key-switch group size (items per launch sequence: 8, 16 or 32),
 //     per ring dimension.
 // Each candidate is timed with HIP events on a scratch batch (the timing of
@@ -83,12 +83,11 @@ void save_cache() {
 // launch-size buckets: limbs per launch below 4, 16, 64, 256, 1024, and above
 constexpr int kBucketCount[TUNE_BUCKETS] = {2, 8, 32, 128, 512, 2048};
 
-template <int LPB, bool HALF>
-void ntt_pair(const Context& c, const PlainJob& j, int count, hipStream_t s) {
-    launch_cols<true, LPB, HALF>(c, j, count, s);
-    launch_rows<true, LPB, HALF>(c, j, count, s);
-    launch_rows<false, LPB, HALF>(c, j, count, s);
-    launch_cols<false, LPB, HALF>(c, j, count, s);
+void ntt_pair(const Context& c, int variant, const PlainJob& j, int count, hipStream_t s) {
+    launch_plain_pass(c, true, false, variant, j, count, s);
+    launch_plain_pass(c, true, true, variant, j, count, s);
+    launch_plain_pass(c, false, true, variant, j, count, s);
+    launch_plain_pass(c, false, false, variant, j, count, s);
 }
 
 float time_ms(hipStream_t s, const std::function<void()>& f, int reps) {
@@ -124,9 +123,9 @@ TunePlan measure(Context& c) {
         const int npolys = count / lpp, n = npolys * lpp;
         const PlainJob j = plain_job(LimbBatch{buf, (long long)lpp * (long long)N, lpp, 0, n}, N);
         const int reps = n >= 512 ? 3 : 8;
-        const float t[NTT_VARIANTS] = {time_ms(s, [&] { ntt_pair<1, false>(c, j, n, s); }, reps),
-                                       time_ms(s, [&] { ntt_pair<2, false>(c, j, n, s); }, reps),
-                                       time_ms(s, [&] { ntt_pair<1, true>(c, j, n, s); }, reps)};
+        const float t[NTT_VARIANTS] = {time_ms(s, [&] { ntt_pair(c, 1, j, n, s); }, reps),
+                                       time_ms(s, [&] { ntt_pair(c, 2, j, n, s); }, reps),
+                                       time_ms(s, [&] { ntt_pair(c, 3, j, n, s); }, reps)};
         // the plain variant unless another is clearly faster
         int best = 0;
         for (int v = 1; v < NTT_VARIANTS; ++v)

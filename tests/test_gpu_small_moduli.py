@@ -1,0 +1,80 @@
+"""Moduli below 2^50 are computed in integer-valued doubles, larger ones in
+integers: both sides of that line, and the values that bring the doubles
+closest to 2^53, against the oracle (whose arithmetic is integer throughout).
+Residues are exact, so every comparison is equality."""
+import numpy as np
+import pytest
+
+import oracle as O
+from helpers import product, rand_residues
+
+pytestmark = pytest.mark.gpu
+
+# above and below 2^50 (integers / doubles) and 2^44 (reductions inside a pass)
+BITS = [50, 51, 49, 45, 44, 43, 36, 27, 61, 50, 38]
+
+
+def _pattern(kind, rng, moduli, N):
+    if kind == "random":
+        return rand_residues(rng, moduli, N)
+    out = []
+    for m in moduli:
+        m = int(m)
+        x = np.full(N, m - 1, dtype=np.uint64)
+        if kind == "alternating":
+            x[1::2] = 0
+        elif kind == "halves":
+            x[: N // 2], x[N // 2:] = m // 2, m // 2 + 1
+        out.append(x)
+    return np.concatenate(out)
+
+
+@pytest.mark.parametrize("kind", ["random", "largest", "alternating", "halves"])
+@pytest.mark.parametrize("logn", [10, 11, 12, 13, 14, 15, 16])
+def test_transforms_on_both_sides_of_the_line(logn, kind):
+    M = product()
+    N = 1 << logn
+    p, q = O.find_primes([61], BITS, N)
+    assert any(int(v) < 1 << 50 for v in q) and any(int(v) >= 1 << 50 for v in q)
+    ctx, octx = M.Context(N, q, p, 2), O.Ctx(N, q, p, 2)
+    host = _pattern(kind, np.random.default_rng(logn), q, N)
+    d = M.to_dev(host)
+    ctx.ntt_forward(d, 1, len(q))
+    assert np.array_equal(M.from_dev(d), octx.ntt_fwd(host, len(q)))
+    ctx.ntt_inverse(d, 1, len(q))
+    assert np.array_equal(M.from_dev(d), host)
+    # the inverse of extreme evaluations, and the forward one back
+    d = M.to_dev(host)
+    ctx.ntt_inverse(d, 1, len(q))
+    ctx.ntt_forward(d, 1, len(q))
+    assert np.array_equal(M.from_dev(d), host)
+
+
+@pytest.mark.parametrize("kind", ["random", "largest"])
+@pytest.mark.parametrize("p_bits,q_bits,dnum", [
+    ([50] * 3, [50] * 8, 3),                    # doubles throughout
+    ([61] * 4, [36, 61, 42, 42, 38, 38, 50], 2),  # both kinds in one digit
+    ([50], [50, 51, 50, 49], 4),                # one limb per digit
+])
+@pytest.mark.parametrize("mont", [True, False])
+def test_key_switch_and_rescale(p_bits, q_bits, dnum, kind, mont):
+    M = product()
+    N = 1 << 12
+    p, q = O.find_primes(p_bits, q_bits, N)
+    ctx, octx = M.Context(N, q, p, dnum), O.Ctx(N, q, p, dnum)
+    rng = np.random.default_rng(len(q_bits) + 10 * dnum)
+    basis = list(q) + list(p)
+    top = len(q) - 1
+    key = np.concatenate([_pattern(kind, rng, basis, N) for _ in range(2 * octx.parts(top))])
+    dkey = M.to_dev(key)
+    for level in (top, top // 2):
+        Q = q[: level + 1]
+        kt, b, a = (_pattern(kind, rng, Q, N) for _ in range(3))
+        ob, oa = octx.keyswitch(level, kt, key, b, a, 0, 1, montgomery=mont)
+        db, da = M.to_dev(b), M.to_dev(a)
+        ctx.keyswitch(level, M.to_dev(kt), dkey, db, da, 0, 1, montgomery=mont)
+        assert np.array_equal(M.from_dev(db), ob) and np.array_equal(M.from_dev(da), oa), level
+        x = M.to_dev(b)
+        ctx.rescale(level, x, 1)
+        want = octx.rescale(level, b.reshape(1, -1))
+        assert np.array_equal(M.from_dev(x)[: level * N], want[0]), level
