@@ -47,10 +47,34 @@ static u64 brev_u(u64 x, int bits) {
     return r;
 }
 
+static double centred(u64 w, u64 q) { return w > q / 2 ? -(double)(q - w) : (double)w; }
+// A constant w < q and its companion in the working form of the modulus:
+// (w, floor(w 2^64 / q)), or the centred w and w/q as doubles.
+static void put_const(const BasisConst& bc, u64 w, u64* out) {
+    if (bc.fp) {
+        const double c = centred(w, bc.q), cq = c / bc.qd;
+        std::memcpy(out, &c, 8);
+        std::memcpy(out + 1, &cq, 8);
+    } else {
+        out[0] = w;
+        out[1] = shoup_of(w, bc.q);
+    }
+}
+static ExtTerm ext_term(const BasisConst& bc, u64 c) {
+    ExtTerm t{};
+    if (bc.fp) {
+        put_const(bc, c, t.v);
+        put_const(bc, mulm(c, (1ull << 32) % bc.q, bc.q), t.v + 2);
+    } else {
+        t.v[0] = mulm(c, bc.r_mod_q, bc.q);
+    }
+    return t;
+}
+
 // Twiddles of one modulus: table[m + i] = psi^(step*(2*brev_m(i)+1)) with
 // step = N/(2m) (forward) and the same with psi^-1 (inverse).
 static void make_twiddles(u64 N, int logN, u64 q, u64* fwd, u64* fws, u64* inv, u64* ivs,
-                          BasisConst& bc) {
+                          BasisConst& bc, u64& inv1) {
     if ((q - 1) % (2 * N) != 0) throw Error(-1, "modulus is not 1 mod 2N");
     const u64 e = (q - 1) / (2 * N);
     u64 psi = 0;
@@ -86,29 +110,25 @@ static void make_twiddles(u64 N, int logN, u64 q, u64* fwd, u64* fws, u64* inv, 
     u64 inv_q = 1;
     for (int i = 0; i < 6; ++i) inv_q *= 2 - q * inv_q;
     bc.qninv = 0 - inv_q;
-    bc.n_inv = invm(N % q, q);
-    bc.n_inv_shoup = shoup_of(bc.n_inv, q);
     bc.r_mod_q = (u64)((((u128)1) << 64) % q);
     bc.inv_d = 1.0 / (double)q;
     bc.negq = (u64)0 - q;
-    bc.w1_ninv = (u64)(((u128)inv[1] * bc.n_inv) % q);
-    bc.w1_ninv_shoup = shoup_of(bc.w1_ninv, q);
+    inv1 = inv[1];
     bc.qd = (double)q;
     bc.fp = q < (1ull << FP_BITS) ? 1 : 0;
+    const u64 n_inv = invm(N % q, q);
+    put_const(bc, n_inv, bc.inv_last);
+    put_const(bc, mulm(inv[1], n_inv, q), bc.inv_last + 2);
     if (bc.fp) {
         // (w, companion) -> centred w and w/q as doubles, in place
-        auto centred = [q](u64 w) { return w > q / 2 ? -(double)(q - w) : (double)w; };
-        bc.n_inv_fp = centred(bc.n_inv);
-        bc.n_inv_fpq = bc.n_inv_fp / bc.qd;
-        bc.w1_ninv_fp = centred(bc.w1_ninv);
-        bc.w1_ninv_fpq = bc.w1_ninv_fp / bc.qd;
-        bc.rinv_fp = centred(invm(bc.r_mod_q, q));
+        bc.rinv_fp = centred(invm(bc.r_mod_q, q), q);
         bc.rinv_fpq = bc.rinv_fp / bc.qd;
         auto convert = [&](u64* w, u64* ws) {
             for (u64 i = 0; i < N; ++i) {
-                const double c = centred(w[i]), cq = c / bc.qd;
-                std::memcpy(&w[i], &c, 8);
-                std::memcpy(&ws[i], &cq, 8);
+                u64 k[2];
+                put_const(bc, w[i], k);
+                w[i] = k[0];
+                ws[i] = k[1];
             }
         };
         convert(fwd, fws);
@@ -236,6 +256,7 @@ Context* context_create(u64 N, const u64* q, int nq, const u64* p, int np, int d
     const int nb = nq + np;
     std::vector<u64> fwd(nb * N), fws(nb * N), inv(nb * N), ivs(nb * N);
     c->h_bc.resize(nb);
+    std::vector<u64> inv1(nb);  // inverse twiddle 1 of each modulus
     {
         std::vector<std::thread> th;
         unsigned hw = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
@@ -244,7 +265,7 @@ Context* context_create(u64 N, const u64* q, int nq, const u64* p, int np, int d
                 for (int b = (int)w; b < nb; b += (int)hw) {
                     u64 m = b < nq ? q[b] : p[b - nq];
                     make_twiddles(N, c->logN, m, &fwd[b * N], &fws[b * N], &inv[b * N],
-                                  &ivs[b * N], c->h_bc[b]);
+                                  &ivs[b * N], c->h_bc[b], inv1[b]);
                 }
             });
         for (auto& t : th) t.join();
@@ -266,62 +287,75 @@ Context* context_create(u64 N, const u64* q, int nq, const u64* p, int np, int d
 
     // ---- ModUp / ModDown / rescale tables packed in one blob ----
     Blob blob;
-    struct MU { size_t qi, qis, si, qmd, ac, db; int ns, nd, s0, s1; };
-    std::vector<std::vector<MU>> mu(nq);
+    struct EX { size_t terms, inv, corr, scale; int ns, nd, s0, s1; u64 wide; };
+    std::vector<std::vector<EX>> mu(nq);
     for (int level = 0; level < nq; ++level) {
         const int L = level + 1;
         const int parts = c->parts(level);
         for (int part = 0; part < parts; ++part) {
             const int s0 = part * c->alpha, s1 = std::min(s0 + c->alpha, L);
             const int ns = s1 - s0;
-            std::vector<u64> dst;
-            std::vector<int> dbasis;
-            for (int i = 0; i < s0; ++i) { dst.push_back(q[i]); dbasis.push_back(i); }
-            for (int i = s1; i < L; ++i) { dst.push_back(q[i]); dbasis.push_back(i); }
-            for (int i = 0; i < np; ++i) { dst.push_back(p[i]); dbasis.push_back(nq + i); }
+            std::vector<int> dst;
+            for (int i = 0; i < s0; ++i) dst.push_back(i);
+            for (int i = s1; i < L; ++i) dst.push_back(i);
+            for (int i = 0; i < np; ++i) dst.push_back(nq + i);
             const int nd = (int)dst.size();
-            std::vector<u64> qhi(ns), qhis(ns), qmd((size_t)nd * ns), ac((size_t)nd * (ns + 1));
+            std::vector<ExtTerm> terms((size_t)nd * ns);
+            std::vector<u64> corr((size_t)nd * 2), scale((size_t)ns * 4);
             std::vector<double> sinv(ns);
+            EX m{0, 0, 0, 0, ns, nd, s0, s1, 0};
             for (int i = 0; i < ns; ++i) {
                 const u64 qi = q[s0 + i];
+                const BasisConst& bs = c->h_bc[s0 + i];
                 sinv[i] = 1.0 / (double)qi;
+                if (!bs.fp && i < 64) m.wide |= 1ull << i;
                 u64 h = 1;
                 for (int j = 0; j < ns; ++j)
                     if (j != i) h = mulm(h, q[s0 + j] % qi, qi);
-                qhi[i] = invm(h, qi);
-                qhis[i] = shoup_of(qhi[i], qi);
+                const u64 y = mulm(invm(h, qi), invm(N % qi, qi), qi);
+                put_const(bs, y, &scale[(size_t)i * 4]);
+                put_const(bs, mulm(y, inv1[s0 + i], qi), &scale[(size_t)i * 4 + 2]);
                 for (int t = 0; t < nd; ++t) {
+                    const BasisConst& bd = c->h_bc[dst[t]];
                     u64 v = 1;
                     for (int j = 0; j < ns; ++j)
-                        if (j != i) v = mulm(v, q[s0 + j] % dst[t], dst[t]);
-                    // Montgomery form (x 2^64): the kernel's sum ends in one REDC
-                    qmd[(size_t)t * ns + i] = (u64)(((unsigned __int128)v << 64) % dst[t]);
+                        if (j != i) v = mulm(v, q[s0 + j] % bd.q, bd.q);
+                    terms[(size_t)t * ns + i] = ext_term(bd, v);
                 }
             }
             for (int t = 0; t < nd; ++t) {
+                const BasisConst& bd = c->h_bc[dst[t]];
                 u64 prod = 1;
-                for (int i = 0; i < ns; ++i) prod = mulm(prod, q[s0 + i] % dst[t], dst[t]);
-                for (int a = 0; a <= ns; ++a) ac[(size_t)t * (ns + 1) + a] = mulm(prod, (u64)a, dst[t]);
+                for (int i = 0; i < ns; ++i) prod = mulm(prod, q[s0 + i] % bd.q, bd.q);
+                put_const(bd, prod, &corr[(size_t)t * 2]);
             }
-            MU m;
-            m.ns = ns; m.nd = nd; m.s0 = s0; m.s1 = s1;
-            m.qi = blob.add(qhi.data(), 8 * ns);
-            m.qis = blob.add(qhis.data(), 8 * ns);
-            m.si = blob.add(sinv.data(), 8 * ns);
-            m.qmd = blob.add(qmd.data(), 8 * qmd.size());
-            m.ac = blob.add(ac.data(), 8 * ac.size());
-            m.db = blob.add(dbasis.data(), sizeof(int) * nd);
+            m.terms = blob.add(terms.data(), sizeof(ExtTerm) * terms.size());
+            m.inv = blob.add(sinv.data(), 8 * ns);
+            m.corr = blob.add(corr.data(), 8 * corr.size());
+            m.scale = blob.add(scale.data(), 8 * scale.size());
             mu[level].push_back(m);
         }
     }
-    std::vector<size_t> md_off(nq);
+    std::vector<EX> md(nq);
     for (int level = 0; level < nq; ++level) {
         const int L = level + 1;
-        std::vector<u64> pinv((size_t)L * np);
-        for (int i = 0; i < L; ++i)
-            for (int j = 0; j < np; ++j)  // Montgomery form, as above
-                pinv[(size_t)i * np + j] = (u64)(((unsigned __int128)invm(p[j] % q[i], q[i]) << 64) % q[i]);
-        md_off[level] = blob.add(pinv.data(), 8 * pinv.size());
+        std::vector<ExtTerm> terms((size_t)L * np);
+        std::vector<u64> corr((size_t)L * 2);
+        std::vector<double> pinv(np);
+        EX m{0, 0, 0, 0, np, L, 0, 0, 0};
+        for (int j = 0; j < np; ++j) {
+            pinv[j] = c->h_bc[nq + j].inv_d;
+            if (!c->h_bc[nq + j].fp && j < 64) m.wide |= 1ull << j;
+        }
+        for (int i = 0; i < L; ++i) {
+            for (int j = 0; j < np; ++j)
+                terms[(size_t)i * np + j] = ext_term(c->h_bc[i], invm(p[j] % q[i], q[i]));
+            put_const(c->h_bc[i], 1, &corr[(size_t)i * 2]);
+        }
+        m.terms = blob.add(terms.data(), sizeof(ExtTerm) * terms.size());
+        m.inv = blob.add(pinv.data(), 8 * np);
+        m.corr = blob.add(corr.data(), 8 * corr.size());
+        md[level] = m;
     }
     struct RS { size_t ip, ips, hm; };
     std::vector<RS> rs(nq);
@@ -342,21 +376,15 @@ Context* context_create(u64 N, const u64* q, int nq, const u64* p, int np, int d
     MI_HIP(hipMemcpy(c->d_blob, blob.host.data(), c->blob_bytes, hipMemcpyHostToDevice));
     c->table_bytes += c->blob_bytes;
     auto P = [&](size_t off) { return (const unsigned char*)c->d_blob + off; };
+    auto ext = [&](const EX& m) {
+        return ExtTables{m.ns, m.nd, m.wide, (const ExtTerm*)P(m.terms), (const double*)P(m.inv), (const u64*)P(m.corr)};
+    };
     c->modup.resize(nq);
-    for (int level = 0; level < nq; ++level)
-        for (const MU& m : mu[level]) {
-            ModUpTables t;
-            t.ns = m.ns; t.nd = m.nd; t.s0 = m.s0; t.s1 = m.s1;
-            t.qhat_inv = (const u64*)P(m.qi);
-            t.qhat_inv_shoup = (const u64*)P(m.qis);
-            t.src_inv = (const double*)P(m.si);
-            t.qhat_mod_dst = (const u64*)P(m.qmd);
-            t.alpha_corr = (const u64*)P(m.ac);
-            t.dst_basis = (const int*)P(m.db);
-            c->modup[level].push_back(t);
-        }
     c->moddown.resize(nq);
-    for (int level = 0; level < nq; ++level) c->moddown[level].pinv = (const u64*)P(md_off[level]);
+    for (int level = 0; level < nq; ++level) {
+        for (const EX& m : mu[level]) c->modup[level].push_back(ModUpTables{m.s0, m.s1, ext(m), (const u64*)P(m.scale)});
+        c->moddown[level] = ext(md[level]);
+    }
 
     // Rescale: NTT of the polynomial whose every coefficient is floor(q_d/2) mod q_i.
     c->rescale.resize(nq);

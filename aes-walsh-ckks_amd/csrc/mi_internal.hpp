@@ -20,39 +20,44 @@ struct BasisConst {
     u64 q;
     u64 mu_lo, mu_hi;   // floor((2^128-1)/q)
     u64 qninv;          // -q^-1 mod 2^64
-    u64 n_inv, n_inv_shoup;
+    u64 inv_last[4];    // N^-1 and inverse twiddle 1 times N^-1, each with its companion: the
+                        //   last inverse stage fused with the scaling
     u64 r_mod_q;        // 2^64 mod q
     double inv_d;       // 1.0 / (double)q (HPS estimates)
     u64 negq;           // 2^64 - q
-    u64 w1_ninv, w1_ninv_shoup;  // inverse twiddle 1 times N^-1: the last inverse
-                                 //   stage fused with the scaling
     // Moduli below 2^50 (fp != 0) are transformed in exact double arithmetic:
-    // their twiddle tables hold the centred w and w/q as doubles in place of w
-    // and its Shoup companion, and so do these.
+    // their twiddle tables and inv_last hold the centred w and w/q as doubles in
+    // place of w and its Shoup companion.
     int fp;
     double qd;                   // q
-    double n_inv_fp, n_inv_fpq;
-    double w1_ninv_fp, w1_ninv_fpq;
     double rinv_fp, rinv_fpq;    // 2^-64 mod q: a Montgomery-form factor's excess
 };
 constexpr int FP_BITS = 50;
 
-// HPS ModUp tables of one (level, digit): source limbs are the digit's chain
-// limbs [s0, s1); destinations are the remaining chain limbs of the level
-// followed by the P limbs, in the reference's order.
-struct ModUpTables {
-    int ns, nd, s0, s1;
-    const u64* qhat_inv;        // [ns]
-    const u64* qhat_inv_shoup;  // [ns]
-    const double* src_inv;      // [ns]
-    const u64* qhat_mod_dst;    // [nd][ns], Montgomery form (x 2^64 mod m_dst)
-    const u64* alpha_corr;      // [nd][ns+1]
-    const int* dst_basis;       // [nd]
+// Constant of one source of a base extension for one target modulus m: for m
+// below 2^50 the centred c and 2^32 c mod m and their quotients by m, as
+// doubles (c, c/m, 2^32 c, 2^32 c/m); else c in Montgomery form (and zeros).
+struct ExtTerm {
+    u64 v[4];
 };
-
-// Folded ModDown (ckks_keyswitch.cpp:521-607) tables at one level.
-struct ModDownTables {
-    const u64* pinv;            // [(level+1)][np] p_j^-1 mod q_i, Montgomery form
+// A base extension (mi_extend.hpp): sources -> targets.
+struct ExtTables {
+    int ns, nd;
+    u64 wide;               // bit i: source i has 50 bits or more
+    const ExtTerm* terms;   // [nd][ns]
+    const double* src_inv;  // [ns] 1/q_i
+    const u64* corr;        // [nd][2] the multiple taken off per unit of alpha, mod m:
+                            //   centred value and quotient as doubles, or value and Shoup companion
+};
+// HPS ModUp of one (level, digit): source limbs are the digit's chain limbs
+// [s0, s1); destinations are the remaining chain limbs of the level followed
+// by the P limbs, in the reference's order.  The sources enter as y_i = x_i
+// qhat_i^-1 mod q_i, a factor that the inverse NTT's last stage carries with
+// its N^-1.
+struct ModUpTables {
+    int s0, s1;
+    ExtTables ext;
+    const u64* inv_scale;  // [ns][4] BasisConst::inv_last times qhat_i^-1
 };
 
 struct RescaleTables {
@@ -96,7 +101,8 @@ struct Context {
     void* d_blob = nullptr;      // ModUp / ModDown / rescale tables
     size_t blob_bytes = 0;
     std::vector<std::vector<ModUpTables>> modup;  // [level][part]
-    std::vector<ModDownTables> moddown;           // [level]
+    std::vector<ExtTables> moddown;               // [level]: P limbs -> Q limbs with p_j^-1 (folded ModDown,
+                                                  //   ckks_keyswitch.cpp:521-607), alpha itself taken off
     std::vector<RescaleTables> rescale;           // [level] (level >= 1)
     u64* d_half = nullptr;                        // rescale half_ntt storage
     u64 q0p0_inv = 0, q0p0_inv_shoup = 0;         // p_0^-1 mod q_0 (level-0 switch)
@@ -332,7 +338,7 @@ MacArgs mac_args(const Context& c, int level, const u64* digits, const u64* key,
 //     (K*N words, destroyed); out[k] = base[k] - NTT(contribution_k), base
 //     may alias out; T = npoly*L*N words.
 void ks_modup_n(Context& c, int level, int n, const u64* const* key_terms, u64* D, long long dstride,
-                u64* C, hipStream_t s, bool cols_only = false);
+                u64* C, hipStream_t s);
 // ModDown of n key switches (one level and modes) with the key inner
 // product of their digits folded in (split form); at most 3 digits.
 void ks_moddown_mac(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,

@@ -16,6 +16,7 @@
 //                inner product folded in (mi_moddown_mac.hip).
 // Reordering "+ acc" before "- NTT(contribution)" leaves every canonical
 // residue unchanged.
+#include "mi_extend.hpp"
 #include "mi_moddown.hpp"
 
 #include <algorithm>
@@ -23,114 +24,95 @@
 
 namespace mi {
 
-constexpr int MODUP_DCH = 8;    // destination limbs per ModUp thread
-
-// ---- out-of-place inverse NTT of n key terms -> C (item-minor within a limb) ----
+// ---- inverse NTT of n key terms -> C (item-minor within a limb) ----
+// The first pass also copies each limb, as it is read, to its own place among
+// the digits.
 struct CopyListJob {
     const u64* src[KS_MAX_ITEMS];
     u64* dst;
     long long dstride;
-    int n;
+    u64* digits;  // item i's [parts][L+K][N] at digits + i * digit_stride
+    long long digit_stride;
+    int n, alpha, slots;
     u64 N;
-    FastDiv per_limb;  // n
+    FastDiv per_limb, per_digit;  // n, alpha
     struct View {
         int basis;
         const u64* s;
         u64* d;
-        __device__ u64 load(int i) const { return s[i]; }
+        u64* own;
+        __device__ u64 load(int i) const {
+            const u64 v = s[i];
+            own[i] = v;
+            return v;
+        }
         __device__ void store(int i, u64 v) const { d[i] = v; }
     };
     __device__ View view(int k) const {
         const int l = per_limb.div(k), it = k - l * n;
-        return View{l, src[it] + (long long)l * N, dst + it * dstride + (long long)l * N};
+        const long long o = (long long)l * N;
+        return View{l, src[it] + o, dst + it * dstride + o,
+                    digits + it * digit_stride + (long long)per_digit.div(l) * slots * N + o};
+    }
+    __device__ bool skip(int) const { return false; }
+};
+// Second pass: C holds y = x qhat^-1 mod q of the limb's digit, a factor that
+// rides in the last stage's N^-1.
+struct ScaledListJob {
+    u64* dst;
+    long long dstride;
+    int n, alpha;
+    const u64* inv_scale[16];  // per digit [ns][4]
+    u64 N;
+    FastDiv per_limb, per_digit;
+    struct View {
+        int basis;
+        u64* p;
+        const u64* inv_scale;
+        __device__ u64 load(int i) const { return p[i]; }
+        __device__ void store(int i, u64 v) const { p[i] = v; }
+    };
+    __device__ View view(int k) const {
+        const int l = per_limb.div(k), it = k - l * n, d = per_digit.div(l);
+        return View{l, dst + it * dstride + (long long)l * N, inv_scale[d] + 4 * (l - d * alpha)};
     }
     __device__ bool skip(int) const { return false; }
 };
 
-// ---- ModUp of all digits of n items ----
-struct ModUpArgs {
-    const u64* coeff;                   // C: item i's [L][N] at coeff + i*L*N
-    const u64* eval[KS_MAX_ITEMS];      // key terms [L][N]
-    u64* digits;                        // item i's D [parts][L+K][N] at digits + i*dstride
+// ---- ModUp of all digits of n items, fused with the forward column pass ----
+struct ModUpJob {
+    ExtGrid grid;
+    const u64* coeff;  // C: item i's [L][N] at coeff + i*L*N
+    u64* digits;       // item i's D [parts][L+K][N] at digits + i*dstride
     long long dstride;
-    int L, K, parts, chunks;
-    int logN;
-    ModUpTables t[16];
+    int L, K, nq, parts;
+    u64 N;
+    FastDiv per_item;  // parts
+    int s0[16];
+    ExtTables t[16];
     const BasisConst* bc;
+    // source: item-major (item, digit)
+    __device__ int targets(int source) const { return t[source - per_item.div(source) * parts].nd; }
+    __device__ ExtView view(int source, int target) const {
+        const int it = per_item.div(source), d = source - it * parts;
+        const ExtTables& e = t[d];
+        // targets in order: chain limbs before the digit, after it, P limbs
+        const int slot = target < s0[d] ? target : target + e.ns;
+        const int basis = slot < L ? slot : nq + (slot - L);
+        const BasisConst b = bc[basis];
+        return ExtView{basis,
+                       coeff + ((long long)it * L + s0[d]) * N,
+                       digits + it * dstride + ((long long)d * (L + K) + slot) * N,
+                       (long long)N,
+                       e.terms + (long long)target * e.ns,
+                       e.src_inv,
+                       e.corr + 2 * target,
+                       e.ns,
+                       e.wide,
+                       b.qninv,
+                       b.mu_hi};
+    }
 };
-
-// One block: 256 coefficients of one digit of one item, up to MODUP_DCH
-// destination limbs.  The digit's tables are staged in LDS first: every
-// thread reads the same entries, so they are LDS broadcasts instead of a
-// dependent global load per product.  NS = the digit's limb count.
-template <int NS>
-__global__ void __launch_bounds__(KS_THREADS) k_modup(ModUpArgs a) {
-    __shared__ u64 s_row[MODUP_DCH][NS];       // qhat_i mod m_j
-    __shared__ u64 s_corr[MODUP_DCH][NS + 1];  // alpha * Q_digit mod m_j
-    __shared__ u64 s_dq[MODUP_DCH], s_ninv[MODUP_DCH], s_muhi[MODUP_DCH];
-    __shared__ int s_slot[MODUP_DCH];
-    __shared__ u64 s_sq[NS], s_qinv[NS], s_qinvs[NS];
-    __shared__ double s_sinv[NS];
-    const int d = blockIdx.y;
-    const int it = blockIdx.z / a.chunks;
-    const int chunk = blockIdx.z - it * a.chunks;
-    const u64 N = (u64)1 << a.logN;
-    const ModUpTables& t = a.t[d];
-    const int j0 = chunk * MODUP_DCH;
-    if (j0 >= t.nd) return;  // uniform over the block
-    const int nj = j0 + MODUP_DCH < t.nd ? MODUP_DCH : t.nd - j0;
-    for (int e = threadIdx.x; e < nj * NS; e += KS_THREADS)
-        s_row[e / NS][e % NS] = t.qhat_mod_dst[(long long)(j0 + e / NS) * NS + e % NS];
-    for (int e = threadIdx.x; e < nj * (NS + 1); e += KS_THREADS)
-        s_corr[e / (NS + 1)][e % (NS + 1)] = t.alpha_corr[(long long)(j0 + e / (NS + 1)) * (NS + 1) + e % (NS + 1)];
-    if (threadIdx.x < nj) {
-        const int j = j0 + threadIdx.x;
-        const BasisConst b = a.bc[t.dst_basis[j]];
-        s_dq[threadIdx.x] = b.q;
-        s_ninv[threadIdx.x] = b.qninv;
-        s_muhi[threadIdx.x] = b.mu_hi;
-        s_slot[threadIdx.x] =
-            j < t.s0 ? j : (j < t.s0 + (a.L - t.s1) ? t.s1 + (j - t.s0) : a.L + (j - (a.L - NS)));
-    }
-    if (threadIdx.x >= 64 && threadIdx.x < 64 + NS) {
-        const int i = threadIdx.x - 64;
-        s_sq[i] = a.bc[t.s0 + i].q;
-        s_qinv[i] = t.qhat_inv[i];
-        s_qinvs[i] = t.qhat_inv_shoup[i];
-        s_sinv[i] = t.src_inv[i];
-    }
-    __syncthreads();
-    // N is a multiple of KS_THREADS: every thread has a coefficient
-    const int c = blockIdx.x * KS_THREADS + threadIdx.x;
-    const int slots = a.L + a.K;
-    const u64* coeff = a.coeff + (long long)it * a.L * N;
-    const u64* eval = a.eval[it];
-    u64* D = a.digits + it * a.dstride + (long long)d * slots * N;
-    u64 y[NS];
-    double est = 0.0;
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-        const int limb = t.s0 + i;
-        const u64 q = s_sq[i];
-        const u64 x = reduce_4q(coeff[(long long)limb * N + c], q);
-        y[i] = shoup(x, s_qinv[i], s_qinvs[i], q);
-        est = __dadd_rn(est, __dmul_rn((double)y[i], s_sinv[i]));
-        if (chunk == 0) D[(long long)limb * N + c] = eval[(long long)limb * N + c];
-    }
-    u64 al = (u64)__dadd_rn(est, 0.5);
-    if (al > (u64)NS) al = (u64)NS;
-    for (int jj = 0; jj < nj; ++jj) {
-        // sum of NS products < 16 * 2^124 fits in 128 bits; the rows are in
-        // Montgomery form, so one REDC gives sum y_i qhat_i mod m
-        U128 acc{0, 0};
-#pragma unroll
-        for (int i = 0; i < NS; ++i) mac128(acc, y[i], s_row[jj][i]);
-        const u64 q = s_dq[jj];
-        u64 v = redc128_any(acc.lo, acc.hi, q, s_ninv[jj], s_muhi[jj]);
-        v = sub_mod(v, s_corr[jj][al], q);
-        D[(long long)s_slot[jj] * N + c] = v;
-    }
-}
 
 // ---- forward NTT of the ModUp'd slots ----
 struct DigitJob {
@@ -166,66 +148,53 @@ struct DigitJob {
 };
 
 void ks_modup_n(Context& c, int level, int n, const u64* const* key_terms, u64* D, long long dstride,
-                u64* C, hipStream_t s, bool cols_only) {
+                u64* C, hipStream_t s) {
     const int L = level + 1, K = c.np, parts = c.parts(level);
     const u64 N = c.N;
     if (n < 1 || n > KS_MAX_ITEMS) throw Error(-1, "ModUp batch size out of range");
     if (parts > 16) throw Error(-1, "too many digits");
     for (int d = 0; d < parts; ++d)
-        if (c.modup[level][d].ns > MAX_ALPHA) throw Error(-1, "digit wider than 16 limbs");
+        if (c.modup[level][d].ext.ns > MAX_ALPHA) throw Error(-1, "digit wider than 16 limbs");
     {
         CopyListJob in{};
+        ScaledListJob out{};
         for (int i = 0; i < n; ++i) in.src[i] = key_terms[i];
-        in.dst = C;
-        in.dstride = (long long)L * (long long)N;
-        in.n = n;
-        in.N = N;
-        in.per_limb = fast_div(n);
-        const PlainJob out = plain_job(LimbBatch{C, (long long)L * (long long)N, L, 0, L * n}, N);
+        for (int d = 0; d < parts; ++d) out.inv_scale[d] = c.modup[level][d].inv_scale;
+        in.dst = out.dst = C;
+        in.dstride = out.dstride = (long long)L * (long long)N;
+        in.digits = D;
+        in.digit_stride = dstride;
+        in.slots = L + K;
+        in.n = out.n = n;
+        in.alpha = out.alpha = c.alpha;
+        in.N = out.N = N;
+        in.per_limb = out.per_limb = fast_div(n);
+        in.per_digit = out.per_digit = fast_div(c.alpha);
         run_ntt_inv(c, in, out, L * n, s);
     }
-    int maxnd = 0;
-    {
-        ModUpArgs a{};
-        a.coeff = C;
-        for (int i = 0; i < n; ++i) a.eval[i] = key_terms[i];
-        a.digits = D;
-        a.dstride = dstride;
-        a.L = L;
-        a.K = K;
-        a.parts = parts;
-        a.logN = c.logN;
-        a.bc = c.d_bc;
-        for (int d = 0; d < parts; ++d) {
-            a.t[d] = c.modup[level][d];
-            maxnd = a.t[d].nd > maxnd ? a.t[d].nd : maxnd;
-        }
-        a.chunks = (maxnd + MODUP_DCH - 1) / MODUP_DCH;
-        if (a.chunks < 1) a.chunks = 1;
-        // digits of one width go in one launch (all but the last have alpha limbs)
-        int d0 = 0;
-        while (d0 < parts) {
-            int d1 = d0 + 1;
-            while (d1 < parts && a.t[d1].ns == a.t[d0].ns) ++d1;
-            ModUpArgs b = a;
-            for (int d = d0; d < d1; ++d) b.t[d - d0] = a.t[d];
-            // the launch's digit index starts at 0: shift the digit outputs
-            b.digits = a.digits + (long long)d0 * (L + K) * (long long)N;
-            dim3 grid((unsigned)(N / KS_THREADS), d1 - d0, a.chunks * n);
-            switch (a.t[d0].ns) {
-#define MI_MODUP_CASE(NS) \
-                case NS: hipLaunchKernelGGL(k_modup<NS>, grid, dim3(KS_THREADS), 0, s, b); break;
-                MI_NS_CASES(MI_MODUP_CASE)
-#undef MI_MODUP_CASE
-                default: throw Error(-1, "digit wider than 16 limbs");
-            }
-            MI_HIP(hipGetLastError());
-            d0 = d1;
-        }
+    ModUpJob m{};
+    m.coeff = C;
+    m.digits = D;
+    m.dstride = dstride;
+    m.L = L;
+    m.K = K;
+    m.nq = c.nq;
+    m.parts = parts;
+    m.N = N;
+    m.per_item = fast_div(parts);
+    m.bc = c.d_bc;
+    int maxnd = 1;
+    for (int d = 0; d < parts; ++d) {
+        m.s0[d] = c.modup[level][d].s0;
+        m.t[d] = c.modup[level][d].ext;
+        maxnd = std::max(maxnd, m.t[d].nd);
     }
-    DigitJob j{D, dstride, L, K, c.nq, c.alpha, parts, n, N, fast_div(parts * n), fast_div(parts)};
-    if (cols_only) launch_pass<true, false>(c, j, parts * (L + K) * n, s);
-    else run_ntt_fwd(c, j, j, parts * (L + K) * n, s);
+    const DigitJob j{D, dstride, L, K, c.nq, c.alpha, parts, n, N, fast_div(parts * n), fast_div(parts)};
+    const int limbs = parts * (L + K) * n;
+    const long probe = c.probe_open(s, limbs);
+    launch_ext_cols(c, m, n * parts, maxnd, s);
+    launch_pass<true, true>(c, j, limbs, s);
+    c.probe_close(probe, s);
 }
 
 void ks_modup(Context& c, int level, const u64* key_term, u64* D, u64* C, hipStream_t s) {

@@ -179,7 +179,6 @@ void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64*
         moddown_p_cols(c, npoly, p, s);
         c.probe_close(probe, s);
     }
-    moddown_contrib(c, level, npoly, p, T, s);
     MdMacOutJob<PARTS> o{};
     o.kp = kp;
     o.tmp = T;
@@ -200,7 +199,7 @@ void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64*
     o.npoly = npoly;
     o.per_limb = fast_div(npoly);
     const long long probe = c.probe_open(s, npoly * L);
-    moddown_contrib_cols(c, level, npoly, T, s);
+    moddown_ext_cols(c, level, npoly, p, T, s);
     launch_rows_w4<true>(c, o, npoly * L, s);
     c.probe_close(probe, s);
 }

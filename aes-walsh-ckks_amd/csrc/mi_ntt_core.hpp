@@ -55,12 +55,12 @@ struct BfInt {
     template <int D>
     __device__ __forceinline__ void tame(u64 (&)[E], bool) const {}
     __device__ __forceinline__ u64 out_fwd(u64 x) const { return reduce_4q(x, q); }
-    // Last inverse stage (distance N/2) with the N^-1 scaling, canonical:
-    // x0 = (x0 + x1) N^-1, x1 = (x0 - x1) w_1 N^-1.
-    __device__ __forceinline__ void inv_last(u64& x0, u64& x1, const BasisConst& b) const {
+    // Last inverse stage (distance N/2) with a scaling, canonical: x0 = (x0 + x1)
+    // k[0], x1 = (x0 - x1) k[2] (BasisConst::inv_last).
+    __device__ __forceinline__ void inv_last(u64& x0, u64& x1, const u64* k) const {
         const u64 s = x0 + x1, d = x0 - x1 + q2;
-        x0 = shoup(s, b.n_inv, b.n_inv_shoup, q);
-        x1 = shoup(d, b.w1_ninv, b.w1_ninv_shoup, q);
+        x0 = shoup(s, k[0], k[1], q);
+        x1 = shoup(d, k[2], k[3], q);
     }
 };
 
@@ -108,10 +108,10 @@ struct BfFp {
             if ((j & D) == 0) x[j] = u(m.centred(d(x[j])));
     }
     __device__ __forceinline__ u64 out_fwd(u64 x) const { return m.canonical(d(x)); }
-    __device__ __forceinline__ void inv_last(u64& x0, u64& x1, const BasisConst& b) const {
+    __device__ __forceinline__ void inv_last(u64& x0, u64& x1, const u64* k) const {
         const double s = d(x0) + d(x1), t = d(x0) - d(x1);
-        x0 = m.canonical(m.mul(s, b.n_inv_fp, b.n_inv_fpq));
-        x1 = m.canonical(m.mul(t, b.w1_ninv_fp, b.w1_ninv_fpq));
+        x0 = m.canonical(m.mul(s, d(k[0]), d(k[1])));
+        x1 = m.canonical(m.mul(t, d(k[2]), d(k[3])));
     }
 };
 

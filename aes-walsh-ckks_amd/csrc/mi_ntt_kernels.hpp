@@ -18,6 +18,10 @@
 // `void store_fp(int i, double x, u64 pre) const` (`pre` as above, else 0),
 // which takes the transform's output x before it is made canonical
 // (|x| < 5.2q) and stores the canonical result.
+// A View with `static constexpr bool BLOCK` forms all E inputs of a thread in
+// one call, load_block(arithmetic, positions, x), in the working form.  A View
+// of an inverse transform's second pass may name its own `const u64* inv_scale`
+// in place of BasisConst::inv_last.
 // Forward column pass: load = job input, store = intermediate.
 // Forward row pass: load = intermediate, store = canonical output.
 // Inverse row pass: load = input (canonical), store = intermediate.
@@ -98,6 +102,14 @@ struct HasLoadFp : std::false_type {};
 template <class V>
 struct HasLoadFp<V, std::void_t<decltype(&V::load_fp)>> : std::true_type {};
 template <class V, class = void>
+struct HasBlock : std::false_type {};
+template <class V>
+struct HasBlock<V, std::void_t<decltype(V::BLOCK)>> : std::true_type {};
+template <class V, class = void>
+struct HasInvScale : std::false_type {};
+template <class V>
+struct HasInvScale<V, std::void_t<decltype(&V::inv_scale)>> : std::true_type {};
+template <class V, class = void>
 struct HasStoreFp : std::false_type {};
 template <class V>
 struct HasStoreFp<V, std::void_t<decltype(&V::store_fp)>> : std::true_type {};
@@ -151,7 +163,9 @@ __device__ __forceinline__ void pass_body(const NttTabs& tb, const V (&v)[LPB], 
 #pragma unroll
     for (int i = 0; i < LPB; ++i) {
         kq[i] = BF::of(tb.bc[v[i].basis]);
-        if (live[i]) {
+        if constexpr (HasBlock<V>::value) {
+            v[i].load_block(kq[i], at, x[i]);
+        } else if (live[i]) {
 #pragma unroll
             for (int j = 0; j < E; ++j) {
                 if constexpr (LOAD_FP) x[i][j] = BfFp::u(v[i].load_fp(at(j)));
@@ -193,9 +207,10 @@ __device__ __forceinline__ void pass_body(const NttTabs& tb, const V (&v)[LPB], 
             for (int j = 0; j < E; ++j) x[i][j] = kq[i].out_fwd(x[i][j]);
         }
         if constexpr (!FIRST && !FWD) {
-            const BasisConst b = tb.bc[v[i].basis];
+            const u64* k = tb.bc[v[i].basis].inv_last;
+            if constexpr (HasInvScale<V>::value) k = v[i].inv_scale;
 #pragma unroll
-            for (int j = 0; j < E / 2; ++j) kq[i].inv_last(x[i][j], x[i][j + E / 2], b);
+            for (int j = 0; j < E / 2; ++j) kq[i].inv_last(x[i][j], x[i][j + E / 2], k);
         }
 #pragma unroll
         for (int j = 0; j < E; ++j) {
