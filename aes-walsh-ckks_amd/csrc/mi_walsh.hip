@@ -14,6 +14,8 @@
 #include "mi_internal.hpp"
 #include "mi_arith.hpp"
 
+#include <cstring>
+
 namespace mi {
 
 constexpr int WALSH_MASKS = 16;
@@ -25,40 +27,39 @@ struct WalshArgs {
     const u64* high_a[WALSH_MASKS - 1];
     const u64* pt;                      // L limbs, evaluation domain
     u64 *acc_b, *acc_a, *raw_b, *raw_a, *raw_c2;
-    int cr[WALSH_MASKS][WALSH_MASKS];  // [h][m] (32-bit: scalar loads)
-    int ci[WALSH_MASKS][WALSH_MASKS];
+    // [h][m] as doubles: the high words (a 16-bit integer's low word is zero)
+    u32 cr[WALSH_MASKS][WALSH_MASKS];
+    u32 ci[WALSH_MASKS][WALSH_MASKS];
     u64 v_lo[2 * WALSH_MASKS], v_hi[2 * WALSH_MASKS];  // |V| of (h, real) at 2h, (h, imag) at 2h+1
     unsigned v_neg;                                     // sign bit per entry
+    u64 exact_fp;                                       // bit l: limb l takes the double path
     int logN, pt_mont;
     const BasisConst* bc;
 };
 
-// sum_m c[m] x_m mod q for |c| < 2^15, x_m = x1 2^31 + x0 given as 31-bit
-// halves: two signed 32x32+64 multiply-adds per term, |partial sums| < 2^50.
-// SMALL (q < 2^43, so x1 < 2^12 and |A1 2^31 + A0| < 2^62.1): the signed
-// 64-bit value A1 2^31 + A0 shifted non-negative by off (a multiple of q
-// near 2^63) and one 64-bit reduction.  Otherwise both halves shifted by off
-// (a multiple of q above 2^50) and one 128-bit reduction of
-// (A1 + off) 2^31 + (A0 + off).
-template <bool SMALL>
-__device__ __forceinline__ u64 walsh_lc(const int* c, const int (&x0)[WALSH_MASKS - 1],
-                                        const int (&x1)[WALSH_MASKS - 1], u64 off, const BasisConst& b) {
-    long long a0 = 0, a1 = 0;
+__device__ __forceinline__ double walsh_coef(u32 hi) { return __builtin_bit_cast(double, (u64)hi << 32); }
+
+// sum_m c[m] x_m for x_m below q as doubles: exact, the caller has checked
+// that the sum of the coefficients' magnitudes times q stays below 2^53.
+__device__ __forceinline__ double walsh_lc_fp(const u32* c, const double (&x)[WALSH_MASKS - 1]) {
+    double s = walsh_coef(c[1]) * x[0];
 #pragma unroll
-    for (int m = 1; m < WALSH_MASKS; ++m) {
-        const int cm = c[m];
-        a0 += (long long)cm * x0[m - 1];
-        a1 += (long long)cm * x1[m - 1];
-    }
-    if constexpr (SMALL) {
-        const u64 v = (u64)(a1 * (1LL << 31) + a0) + off;
-        return reduce64(v, b.q, b.mu_hi);
-    } else {
-        const u64 u = (u64)(a1 + (long long)off), w = (u64)(a0 + (long long)off);
-        const u64 lo = (u << 31) + w;
-        const u64 hi = (u >> 33) + (lo < w ? 1 : 0);
-        return reduce128(lo, hi, b.q, b.mu_lo, b.mu_hi);
-    }
+    for (int m = 2; m < WALSH_MASKS; ++m) s = __builtin_fma(walsh_coef(c[m]), x[m - 1], s);
+    return s;
+}
+
+// sum_m c[m] x_m mod q for |c| < 2^15 and any q < 2^62, x_m = x1 2^31 + x0
+// given as 31-bit halves: each half's sum is below 2^50, exact.  Their
+// quotient by q (below 2^19) is estimated in double, off by less than 1/2 and
+// a little, and the remainder taken modulo 2^64: in (-q, q), made canonical.
+__device__ __forceinline__ u64 walsh_lc(const u32* c, const double (&x0)[WALSH_MASKS - 1],
+                                        const double (&x1)[WALSH_MASKS - 1], const BasisConst& b) {
+    const double s0 = walsh_lc_fp(c, x0), s1 = walsh_lc_fp(c, x1);
+    const double k = __builtin_rint(__builtin_fma(s1, 0x1p31, s0) * b.inv_d);
+    // |v| < 2^51 as a 64-bit integer
+    auto integer = [](double v) { return __builtin_bit_cast(u64, v + 0x1.8p52) - 0x4338000000000000ull; };
+    const u64 r = (integer(s1) << 31) + integer(s0) - integer(k) * b.q;
+    return (long long)r < 0 ? r + b.q : r;
 }
 
 // A block holds 64 coefficients in 8 waves: side (b or a) x quarter of the
@@ -70,43 +71,68 @@ __device__ __forceinline__ u64 walsh_lc(const int* c, const int (&x0)[WALSH_MASK
 constexpr int WALSH_COEFFS = 64;
 constexpr int WALSH_BLOCK = 8 * WALSH_COEFFS;
 
-__global__ void __launch_bounds__(WALSH_BLOCK) k_walsh_product_sum(WalshArgs a) {
-    __shared__ u64 s_const[2 * WALSH_MASKS];
-    __shared__ u64 s_part[2][2][4][WALSH_COEFFS];  // [side][product][quarter][coefficient]
-    const int l = (int)(((long long)blockIdx.x * WALSH_COEFFS) >> a.logN);  // uniform: a block is in one limb
-    const int lane = threadIdx.x % WALSH_COEFFS;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WALSH_COEFFS);
-    const int side = wave >> 2, quarter = wave & 3;
-    const long long i = (long long)blockIdx.x * WALSH_COEFFS + lane;
-    const BasisConst b = a.bc[l];
-    if (threadIdx.x < 2 * WALSH_MASKS) {
-        const int t = threadIdx.x;
-        const u64 r = reduce128(a.v_lo[t], a.v_hi[t], b.q, b.mu_lo, b.mu_hi);
-        s_const[t] = ((a.v_neg >> t) & 1) && r ? b.q - r : r;
+// VALU-bound either way (a coefficient takes 64 linear combinations of 15
+// terms and 60 products per limb).  Doubles (moduli small enough for exact
+// sums, exact_fp): 15 fused multiply-adds per combination and no reduction,
+// six instructions per product.  Integers: the combinations as two sums of
+// halves and one double quotient, 128-bit lazy products.  Measured at N = 2^15
+// over 36-, 61- and 42-bit limbs, 16 output pairs and their relinearisations:
+// 739 us with integer multiply-adds throughout, 555 us.
+struct WalshShared {
+    u64 cst[2 * WALSH_MASKS];
+    u64 part[2][2][4][WALSH_COEFFS];  // [side][product][quarter][coefficient]
+};
+
+__device__ __forceinline__ void walsh_fp(const WalshArgs& a, const BasisConst& b, WalshShared& sh, int side,
+                                         int quarter, int lane, long long i) {
+    const FpMod q{b.qd, b.inv_d};
+    double x[WALSH_MASKS - 1];
+#pragma unroll
+    for (int m = 0; m < WALSH_MASKS - 1; ++m) x[m] = fp_from_u64((side ? a.low_a[m] : a.low_b[m])[i]);
+    double pt = q.centred(fp_from_u64(a.pt[i]));
+    if (a.pt_mont) pt = q.centred(q.mul(pt, b.rinv_fp, b.rinv_fpq));
+    // the rounded 1/q adds at most |x| 2^-53 to a quotient's error: products below 5/2 q
+    const double ptq = pt * b.inv_d;
+    double s0 = 0.0, s1 = 0.0;
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {
+        const int h = 4 * quarter + k;
+        double r = walsh_lc_fp(a.cr[h], x), im = walsh_lc_fp(a.ci[h], x);
+        if (side == 0) {
+            r += fp_from_u64(sh.cst[2 * h]);
+            im += fp_from_u64(sh.cst[2 * h + 1]);
+        }
+        const double z = q.centred(q.centred(r) + q.mul(im, pt, ptq));
+        if (h == 0) {
+            (side ? a.acc_a : a.acc_b)[i] = q.canonical(z);
+            continue;
+        }
+        s0 += q.mulq(z, fp_from_u64(a.high_b[h - 1][i]));
+        s1 += q.mulq(z, fp_from_u64(a.high_a[h - 1][i]));
     }
-    // a multiple of q above every partial sum's magnitude: q ceil(2^50 / q),
-    // or, for the one-word sum, q ceil(2^63 / q) (<= 2^63 + q < 2^64 - 2^62.1)
-    const bool small = b.q < (1ull << 43);  // uniform: one limb per block
-    const u64 off = small ? b.q * (((1ull << 63) + b.q - 1) / b.q) : b.q * (((1ull << 50) + b.q - 1) / b.q);
-    int x0[WALSH_MASKS - 1], x1[WALSH_MASKS - 1];
+    sh.part[side][0][quarter][lane] = q.canonical(s0);
+    sh.part[side][1][quarter][lane] = q.canonical(s1);
+}
+
+__device__ __forceinline__ void walsh_int(const WalshArgs& a, const BasisConst& b, WalshShared& sh, int side,
+                                          int quarter, int lane, long long i) {
+    double x0[WALSH_MASKS - 1], x1[WALSH_MASKS - 1];
 #pragma unroll
     for (int m = 0; m < WALSH_MASKS - 1; ++m) {
         const u64 x = (side ? a.low_a[m] : a.low_b[m])[i];
-        x0[m] = (int)(x & 0x7fffffffu);
-        x1[m] = (int)(x >> 31);
+        x0[m] = (double)(u32)(x & 0x7fffffffu);
+        x1[m] = (double)(u32)(x >> 31);
     }
     const u64 pt = a.pt[i];
-    __syncthreads();
     // at most 4 canonical products per 128-bit sum here
     U128 s_h0{0, 0}, s_h1{0, 0};  // side's Z times H_b, times H_a
 #pragma unroll 1
     for (int k = 0; k < 4; ++k) {
         const int h = 4 * quarter + k;
-        u64 r = small ? walsh_lc<true>(a.cr[h], x0, x1, off, b) : walsh_lc<false>(a.cr[h], x0, x1, off, b);
-        u64 im = small ? walsh_lc<true>(a.ci[h], x0, x1, off, b) : walsh_lc<false>(a.ci[h], x0, x1, off, b);
+        u64 r = walsh_lc(a.cr[h], x0, x1, b), im = walsh_lc(a.ci[h], x0, x1, b);
         if (side == 0) {
-            r = add_mod(r, s_const[2 * h], b.q);
-            im = add_mod(im, s_const[2 * h + 1], b.q);
+            r = add_mod(r, sh.cst[2 * h], b.q);
+            im = add_mod(im, sh.cst[2 * h + 1], b.q);
         }
         const u64 p = a.pt_mont ? mont_mul(im, pt, b.q, b.qninv) : mul_mod(im, pt, b.q, b.mu_lo, b.mu_hi);
         const u64 z = add_mod(r, p, b.q);
@@ -117,12 +143,30 @@ __global__ void __launch_bounds__(WALSH_BLOCK) k_walsh_product_sum(WalshArgs a) 
         mac128(s_h0, z, a.high_b[h - 1][i]);
         mac128(s_h1, z, a.high_a[h - 1][i]);
     }
-    s_part[side][0][quarter][lane] = reduce128(s_h0.lo, s_h0.hi, b.q, b.mu_lo, b.mu_hi);
-    s_part[side][1][quarter][lane] = reduce128(s_h1.lo, s_h1.hi, b.q, b.mu_lo, b.mu_hi);
+    sh.part[side][0][quarter][lane] = reduce128(s_h0.lo, s_h0.hi, b.q, b.mu_lo, b.mu_hi);
+    sh.part[side][1][quarter][lane] = reduce128(s_h1.lo, s_h1.hi, b.q, b.mu_lo, b.mu_hi);
+}
+
+__global__ void __launch_bounds__(WALSH_BLOCK) k_walsh_product_sum(WalshArgs a) {
+    __shared__ WalshShared sh;
+    const int l = (int)(((long long)blockIdx.x * WALSH_COEFFS) >> a.logN);  // uniform: a block is in one limb
+    const int lane = threadIdx.x % WALSH_COEFFS;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WALSH_COEFFS);
+    const int side = wave >> 2, quarter = wave & 3;
+    const long long i = (long long)blockIdx.x * WALSH_COEFFS + lane;
+    const BasisConst b = a.bc[l];
+    if (threadIdx.x < 2 * WALSH_MASKS) {
+        const int t = threadIdx.x;
+        const u64 r = reduce128(a.v_lo[t], a.v_hi[t], b.q, b.mu_lo, b.mu_hi);
+        sh.cst[t] = ((a.v_neg >> t) & 1) && r ? b.q - r : r;
+    }
+    __syncthreads();
+    if (l < 64 && ((a.exact_fp >> l) & 1)) walsh_fp(a, b, sh, side, quarter, lane, i);
+    else walsh_int(a, b, sh, side, quarter, lane, i);
     __syncthreads();
     auto sum4 = [&](int sd, int pr) {
-        return add_mod(add_mod(s_part[sd][pr][0][lane], s_part[sd][pr][1][lane], b.q),
-                       add_mod(s_part[sd][pr][2][lane], s_part[sd][pr][3][lane], b.q), b.q);
+        return add_mod(add_mod(sh.part[sd][pr][0][lane], sh.part[sd][pr][1][lane], b.q),
+                       add_mod(sh.part[sd][pr][2][lane], sh.part[sd][pr][3][lane], b.q), b.q);
     };
     if (wave == 0) a.raw_b[i] = sum4(0, 0);                                  // Z_b H_b
     else if (wave == 1) a.raw_a[i] = add_mod(sum4(0, 1), sum4(1, 0), b.q);   // Z_b H_a + Z_a H_b
@@ -142,12 +186,30 @@ void walsh_product_sum(const Context& c, int level, const u64* const* low_b, con
         a.high_b[m] = high_b[m];
         a.high_a[m] = high_a[m];
     }
-    for (int h = 0; h < WALSH_MASKS; ++h)
+    auto high_word = [](short v) {
+        const double d = v;
+        u64 bits;
+        std::memcpy(&bits, &d, 8);
+        return (u32)(bits >> 32);
+    };
+    long long widest = 0;  // largest sum of magnitudes over a row's masks
+    for (int h = 0; h < WALSH_MASKS; ++h) {
+        long long sr = 0, si = 0;
         for (int m = 0; m < WALSH_MASKS; ++m) {
-            a.cr[h][m] = cr[h * WALSH_MASKS + m];
-            a.ci[h][m] = ci[h * WALSH_MASKS + m];
-            if (a.cr[h][m] == -32768 || a.ci[h][m] == -32768) throw Error(-1, "coefficient out of range");
+            const short r = cr[h * WALSH_MASKS + m], im = ci[h * WALSH_MASKS + m];
+            if (r == -32768 || im == -32768) throw Error(-1, "coefficient out of range");
+            a.cr[h][m] = high_word(r);
+            a.ci[h][m] = high_word(im);
+            if (m) {
+                sr += r < 0 ? -r : r;
+                si += im < 0 ? -im : im;
+            }
         }
+        widest = std::max(widest, std::max(sr, si));
+    }
+    // a combination and its constant stay below (widest + 1) q
+    for (int l = 0; l <= level && l < 64; ++l)
+        if (c.h_bc[l].fp && (u64)(widest + 1) <= (1ull << 53) / c.h_bc[l].q) a.exact_fp |= 1ull << l;
     for (int t = 0; t < 2 * WALSH_MASKS; ++t) {
         a.v_lo[t] = v_abs[2 * t];
         a.v_hi[t] = v_abs[2 * t + 1];

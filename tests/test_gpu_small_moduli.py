@@ -78,3 +78,37 @@ def test_key_switch_and_rescale(p_bits, q_bits, dnum, kind, mont):
         ctx.rescale(level, x, 1)
         want = octx.rescale(level, b.reshape(1, -1))
         assert np.array_equal(M.from_dev(x)[: level * N], want[0]), level
+
+
+@pytest.mark.parametrize("bits", [50, 49, 43, 38])
+@pytest.mark.parametrize("over", [False, True])
+@pytest.mark.parametrize("mont", [True, False])
+def test_walsh_sum_at_the_line_of_exact_doubles(bits, over, mont):
+    """A row of Walsh coefficients whose magnitudes sum to the largest value
+    that keeps a combination and its constant below 2^53 (doubles), and to one
+    more (integers), over residues all q - 1."""
+    M = product()
+    N = 1 << 10
+    p, q = O.find_primes([61], [bits, bits], N)
+    ctx, octx = M.Context(N, q, p, 1), O.Ctx(N, q, p, 1)
+    rng = np.random.default_rng(bits)
+    Q = [int(v) for v in q]
+    most = (1 << 53) // max(Q) - 1 + (1 if over else 0)
+    row = np.zeros(16, dtype=np.int64)
+    row[1:] = most // 15
+    row[1: 1 + most % 15] += 1
+    cr = np.stack([row if h % 2 == 0 else -row for h in range(16)])
+    ci = np.stack([-row if h % 3 == 0 else row for h in range(16)])
+    big = _pattern("largest", rng, Q, N)
+    low = [np.stack([big, big]) for _ in range(15)]
+    high = [np.stack([big, rand_residues(rng, Q, N)]) for _ in range(15)]
+    pt = _pattern("largest", rng, Q, N)
+    consts = [(-1, (1 << 90) + h) for h in range(16)]  # constants of q - 1 and of many words
+    acc_o, raw_o = octx.walsh_product_sum(1, low, high, cr, ci, consts, pt, mont)
+    dev = lambda x: [M.to_dev(x[0]), M.to_dev(x[1])]  # noqa: E731
+    new = lambda: M.to_dev(np.zeros(2 * N, np.uint64))  # noqa: E731
+    acc, raw = [new(), new()], [new(), new(), new()]
+    ctx.walsh_product_sum(1, [dev(x) for x in low], [dev(x) for x in high], cr, ci, consts, M.to_dev(pt), acc, raw,
+                          pt_montgomery=mont)
+    assert all(np.array_equal(M.from_dev(a), o) for a, o in zip(acc, acc_o))
+    assert all(np.array_equal(M.from_dev(r), o) for r, o in zip(raw, raw_o))
