@@ -203,15 +203,6 @@ void ks_modup(Context& c, int level, const u64* key_term, u64* D, u64* C, hipStr
 }
 
 // ---- key inner product ----
-// Evaluation-domain source index of output index i under Galois element g:
-// dst[brev(d)] = src[brev(((2d+1) g mod 2N - 1) / 2)].
-__device__ __forceinline__ u32 galois_src(u32 i, u64 g, int logN) {
-    const u32 mask2n = (2u << logN) - 1;
-    const u32 d = __brev(i) >> (32 - logN);
-    const u32 e = (u32)(((u64)(2 * d + 1) * g) & mask2n);
-    return __brev((e - 1) >> 1) >> (32 - logN);
-}
-
 __global__ void __launch_bounds__(KS_THREADS) k_mac(MacArgs a) {
     const u64 N = (u64)1 << a.logN;
     const int slots = a.L + a.K;
@@ -223,7 +214,7 @@ __global__ void __launch_bounds__(KS_THREADS) k_mac(MacArgs a) {
     const int basis = slot < a.L ? slot : a.nq + (slot - a.L);
     const int key_limbs = a.nq + a.K;
     const BasisConst b = a.bc[basis];
-    const long long src = a.galois ? (long long)galois_src((u32)i, a.galois, a.logN) : i;
+    const long long src = a.galois ? (long long)galois_index((u32)i, a.galois, a.logN) : i;
     const u64* digits = a.digits + it * a.digits_stride;
     const u64* key = a.key[it];
     u64 acc_b, acc_a;
@@ -525,7 +516,7 @@ __global__ void __launch_bounds__(KS_THREADS) k_automorphism_items(AutoItemsArgs
     const int tile = blockIdx.x % tps, rest = blockIdx.x / tps;
     const int l = rest % a.L, poly = (rest / a.L) & 1, it = rest / (2 * a.L);
     const u32 i = (u32)tile * KS_THREADS + threadIdx.x;
-    const u32 sidx = galois_src(i, a.galois[it], a.logN);
+    const u32 sidx = galois_index(i, a.galois[it], a.logN);
     const u64* src = a.src + ((long long)it * 2 + poly) * a.L * N + (long long)l * N;
     u64* dst = (poly == 0 ? a.dst_a[it] : a.dst_b[it]) + (long long)l * N;
     dst[i] = src[sidx];
@@ -672,7 +663,7 @@ __global__ void __launch_bounds__(KS_THREADS) k_automorphism_list(AutoListArgs a
     const int l = rest % a.L, k = rest / a.L;
     const u32 i = (u32)tile * KS_THREADS + threadIdx.x;
     const long long off = (long long)l * N;
-    a.dst[k][off + i] = a.src[k][off + galois_src(i, a.galois, a.logN)];
+    a.dst[k][off + i] = a.src[k][off + galois_index(i, a.galois, a.logN)];
 }
 
 void conjugate_batch(Context& c, int level, int n, u64* const* b, u64* const* a, const u64* key, bool montgomery,

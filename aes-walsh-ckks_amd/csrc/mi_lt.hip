@@ -10,8 +10,8 @@
 //              out.a += rot_{g*bs}(KS.a), out.b += rot_{g*bs}(KS.b + inner_g.b)
 //              (automorphism_qp_pair_accumulate, :373-416)
 //   result   = folded ModDown of out                  (moddown_qp_pair_to_q_eval, :641-718)
-// The automorphism is folded into the inner-product kernel's loads, so the
-// rotated baby steps and giant-step accumulations never exist unpermuted.
+// The baby steps exist only inside the fused inner-product kernel, which reads
+// the digits through each rotation's map.
 #include "mi_ntt_kernels.hpp"
 
 #include <algorithm>
@@ -97,6 +97,210 @@ __global__ void __launch_bounds__(LT_THREADS) k_lt_inner_all(LtAllArgs a) {
     u64* pb = pa + TN;
     *pa = a.accumulate ? add_mod(*pa, ra, b.q) : ra;
     *pb = a.accumulate ? add_mod(*pb, rb, b.q) : rb;
+}
+
+// Baby steps and inner products of the QP evaluator in one pass.  A thread
+// forms, for one coefficient of one limb, the baby step of each rotation (the
+// key product of the hoisted digits, read through the rotation's map, with the
+// b term) and adds its product with every giant step's diagonal, so no baby
+// step is written or read: at N = 2^16, 35 limbs, 15 rotations, 32 ciphertexts
+// the separate passes moved 70 GB of babies and re-read digits.  IT ciphertexts
+// share the loaded keys and diagonals and NG giant steps share the baby step;
+// IT * NG = 16 keeps the sums in 64 registers.  The blocks of one tile for all
+// ciphertexts follow each other on one XCD (map_tile): keys and diagonals come
+// from memory once per launch, the digits of a limb's ciphertexts (2 MB each)
+// stay in the Infinity Cache while its tiles run.
+struct LtFusedArgs {
+    const u64* diag[LT_NG * LT_NB];  // [giant][baby slot], null: no term
+    const u64* key[LT_NB];           // baby slot slot0 + r
+    u64 galois[LT_NB];
+    const u64* in_a[KS_MAX_ITEMS];
+    const u64* in_b[KS_MAX_ITEMS];
+    const u64* digits;               // item i's [parts][T][N] at digits + i*digit_stride
+    long long digit_stride;
+    u64* out[LT_NG];                 // giant g of item i: a at out[g] + i*out_stride[g], b T*N later
+    long long out_stride[LT_NG];
+    int slot0, nb, ng, accumulate;
+    int items, L, K, nq, logN, parts, mont, pt_mont;
+    const BasisConst* bc;
+};
+
+template <int NG, int IT>
+__device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisConst& b, int it0, int slot, long long i) {
+    const u64 N = (u64)1 << a.logN;
+    const int T = a.L + a.K, basis = slot < a.L ? slot : a.nq + (slot - a.L);
+    const long long o = (long long)slot * N, to_a = (long long)(a.nq + a.K) * N;
+    const FpMod m{b.qd, b.inv_d};
+    double sa[IT][NG], sb[IT][NG];
+#pragma unroll
+    for (int t = 0; t < IT; ++t)
+#pragma unroll
+        for (int g = 0; g < NG; ++g) sa[t][g] = sb[t][g] = 0.0;
+    int item[IT];
+#pragma unroll
+    for (int t = 0; t < IT; ++t) item[t] = it0 + t < a.items ? it0 + t : a.items - 1;  // past the end: a repeat, not stored
+    for (int r = 0; r < a.nb; ++r) {
+        double xa[IT], xb[IT];
+        if (a.slot0 + r == 0) {
+            if (slot >= a.L) continue;  // the input's P limbs are zero
+#pragma unroll
+            for (int t = 0; t < IT; ++t) {
+                xa[t] = fp_from_u64(a.in_a[item[t]][o + i]);
+                xb[t] = fp_from_u64(a.in_b[item[t]][o + i]);
+            }
+        } else {
+            const u32 src = galois_index((u32)i, a.galois[r], a.logN);
+            const u64* k = a.key[r] + (long long)basis * N + src;
+            const u64* d = a.digits + o + src;
+#pragma unroll
+            for (int t = 0; t < IT; ++t) xa[t] = xb[t] = 0.0;
+            // operands below 4q: each product at most 9/2 q, centred (as in k_mac)
+            for (int e = 0; e < a.parts; ++e) {
+                const double kb = fp_from_u64(k[2LL * e * to_a]), ka = fp_from_u64(k[(2LL * e + 1) * to_a]);
+#pragma unroll
+                for (int t = 0; t < IT; ++t) {
+                    const double x = fp_from_u64(d[item[t] * a.digit_stride + (long long)e * T * N]);
+                    xb[t] += m.centred(m.mulq(x, kb));
+                    xa[t] += m.centred(m.mulq(x, ka));
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < IT; ++t) {
+                if (a.mont) {
+                    xb[t] = m.mul(xb[t], b.rinv_fp, b.rinv_fpq);
+                    xa[t] = m.mul(xa[t], b.rinv_fp, b.rinv_fpq);
+                }
+                if (slot < a.L) xb[t] += fp_from_u64(a.in_b[item[t]][o + src]);
+                xb[t] = m.centred(xb[t]);
+                xa[t] = m.centred(xa[t]);
+            }
+        }
+        // |x| < q, diagonals below 4q: products at most 3/2 q; four of them
+        // between two reductions
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const u64* dp = a.diag[g * LT_NB + r];
+            if (!dp) continue;
+            const double d = fp_from_u64(dp[o + i]);
+#pragma unroll
+            for (int t = 0; t < IT; ++t) {
+                sa[t][g] += m.mulq(xa[t], d);
+                sb[t][g] += m.mulq(xb[t], d);
+            }
+        }
+        if ((r & 3) == 3) {
+#pragma unroll
+            for (int t = 0; t < IT; ++t)
+#pragma unroll
+                for (int g = 0; g < NG; ++g) {
+                    sa[t][g] = m.centred(sa[t][g]);
+                    sb[t][g] = m.centred(sb[t][g]);
+                }
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g >= a.ng) continue;
+#pragma unroll
+        for (int t = 0; t < IT; ++t) {
+            if (it0 + t >= a.items) continue;
+            double ra = sa[t][g], rb = sb[t][g];
+            if (a.pt_mont) {
+                ra = m.mul(ra, b.rinv_fp, b.rinv_fpq);
+                rb = m.mul(rb, b.rinv_fp, b.rinv_fpq);
+            }
+            u64* pa = a.out[g] + (it0 + t) * a.out_stride[g] + o + i;
+            u64* pb = pa + (long long)T * N;
+            const u64 va = m.canonical(ra), vb = m.canonical(rb);
+            *pa = a.accumulate ? add_mod(*pa, va, b.q) : va;
+            *pb = a.accumulate ? add_mod(*pb, vb, b.q) : vb;
+        }
+    }
+}
+
+// Any modulus: canonical baby steps, exact 128-bit sums (at most 16 products
+// of residues below 2^62), one ciphertext and the NG giant steps from g0 on at
+// a time (a sum takes four registers).
+template <int NG>
+__device__ __forceinline__ void lt_fused_int(const LtFusedArgs& a, const BasisConst& b, int it, int g0, int slot,
+                                             long long i) {
+    const u64 N = (u64)1 << a.logN;
+    const int T = a.L + a.K, basis = slot < a.L ? slot : a.nq + (slot - a.L);
+    const long long o = (long long)slot * N, to_a = (long long)(a.nq + a.K) * N;
+    U128 sa[NG], sb[NG];
+#pragma unroll
+    for (int g = 0; g < NG; ++g) sa[g] = sb[g] = U128{0, 0};
+    const bool lazy = a.parts <= 3 && b.q < (1ull << 61);  // as in k_mac
+    for (int r = 0; r < a.nb; ++r) {
+        u64 xa, xb;
+        if (a.slot0 + r == 0) {
+            if (slot >= a.L) continue;
+            xa = a.in_a[it][o + i];
+            xb = a.in_b[it][o + i];
+        } else {
+            const u32 src = galois_index((u32)i, a.galois[r], a.logN);
+            const u64* k = a.key[r] + (long long)basis * N + src;
+            const u64* d = a.digits + it * a.digit_stride + o + src;
+            U128 pa{0, 0}, pb{0, 0};
+            for (int e = 0; e < a.parts; ++e) {
+                u64 x = d[(long long)e * T * N], kb = k[2LL * e * to_a], ka = k[(2LL * e + 1) * to_a];
+                if (!lazy) {
+                    x = reduce_4q(x, b.q);
+                    kb = reduce_4q(kb, b.q);
+                    ka = reduce_4q(ka, b.q);
+                }
+                mac128(pb, x, kb);
+                mac128(pa, x, ka);
+            }
+            pb.hi = reduce64(pb.hi, b.q, b.mu_hi);
+            pa.hi = reduce64(pa.hi, b.q, b.mu_hi);
+            xb = a.mont ? redc128(pb.lo, pb.hi, b.q, b.qninv) : barrett128(pb.lo, pb.hi, b.q, b.mu_lo, b.mu_hi);
+            xa = a.mont ? redc128(pa.lo, pa.hi, b.q, b.qninv) : barrett128(pa.lo, pa.hi, b.q, b.mu_lo, b.mu_hi);
+            if (slot < a.L) xb = add_mod(xb, a.in_b[it][o + src], b.q);
+        }
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            const u64* dp = a.diag[(g0 + g) * LT_NB + r];
+            if (!dp) continue;
+            const u64 d = reduce_4q(dp[o + i], b.q);
+            mac128(sa[g], xa, d);
+            mac128(sb[g], xb, d);
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+        if (g0 + g >= a.ng) continue;
+        u64 va, vb;
+        if (a.pt_mont) {
+            va = redc128_any(sa[g].lo, sa[g].hi, b.q, b.qninv, b.mu_hi);
+            vb = redc128_any(sb[g].lo, sb[g].hi, b.q, b.qninv, b.mu_hi);
+        } else {
+            va = reduce128(sa[g].lo, sa[g].hi, b.q, b.mu_lo, b.mu_hi);
+            vb = reduce128(sb[g].lo, sb[g].hi, b.q, b.mu_lo, b.mu_hi);
+        }
+        u64* pa = a.out[g0 + g] + it * a.out_stride[g0 + g] + o + i;
+        u64* pb = pa + (long long)T * N;
+        *pa = a.accumulate ? add_mod(*pa, va, b.q) : va;
+        *pb = a.accumulate ? add_mod(*pb, vb, b.q) : vb;
+    }
+}
+
+template <int NG, int IT>
+__global__ void __launch_bounds__(LT_THREADS) k_lt_fused(LtFusedArgs a) {
+    const int tps = (1 << a.logN) / LT_THREADS;
+    const TileMap tm = map_tile(blockIdx.x, (a.items + IT - 1) / IT, tps, a.L + a.K);
+    if (!tm.valid) return;
+    const long long i = (long long)tm.tile * LT_THREADS + threadIdx.x;
+    const BasisConst b = a.bc[tm.slot < a.L ? tm.slot : a.nq + (tm.slot - a.L)];
+    const int it0 = tm.item * IT;
+    if (b.fp) {
+        lt_fused_fp<NG, IT>(a, b, it0, tm.slot, i);
+    } else {
+#pragma unroll 1
+        for (int t = 0; t < IT && it0 + t < a.items; ++t)
+#pragma unroll 1
+            for (int g0 = 0; g0 < a.ng; g0 += 8) lt_fused_int<(NG < 8 ? NG : 8)>(a, b, it0 + t, g0, tm.slot, i);
+    }
 }
 
 static u64 powmod_u64(u64 a, u64 e, u64 m) {
@@ -245,6 +449,58 @@ void launch_inner(Context& c, const Compiled& k, const LtStage& st, int m, int K
     }
 }
 
+// Baby steps and inner products of m items from their hoisted digits; outputs
+// as launch_inner.
+void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const u64* const* a, const u64* const* b,
+                  const u64* digits, long long dstride, u64* out0, long long out0_stride, u64* outg,
+                  long long outg_giant, long long outg_item, hipStream_t s) {
+    const int L = st.level + 1, T = L + c.np;
+    const int tps = (int)(c.N / LT_THREADS);
+    for (int s0 = 0; s0 < k.nslots; s0 += LT_NB) {
+        for (size_t gk0 = 0; gk0 < k.glist.size(); gk0 += LT_NG) {
+            LtFusedArgs f{};
+            f.nb = std::min(LT_NB, k.nslots - s0);
+            f.ng = (int)std::min<size_t>(LT_NG, k.glist.size() - gk0);
+            f.slot0 = s0;
+            for (int r = 0; r < f.nb; ++r) {
+                f.key[r] = k.baby_key[s0 + r];
+                f.galois[r] = k.baby_gal[s0 + r];
+            }
+            for (int g = 0; g < f.ng; ++g) {
+                const size_t gk = gk0 + g;
+                for (int r = 0; r < f.nb; ++r) f.diag[g * LT_NB + r] = k.table[gk * k.nslots + s0 + r];
+                const bool first = k.glist[gk] == 0;
+                f.out[g] = first ? out0 : outg + (long long)(gk - (k.g0 ? 1 : 0)) * outg_giant;
+                f.out_stride[g] = first ? out0_stride : outg_item;
+            }
+            for (int it = 0; it < m; ++it) {
+                f.in_a[it] = a[it];
+                f.in_b[it] = b[it];
+            }
+            f.digits = digits;
+            f.digit_stride = dstride;
+            f.accumulate = s0 > 0 ? 1 : 0;
+            f.items = m;
+            f.L = L;
+            f.K = c.np;
+            f.nq = c.nq;
+            f.logN = c.logN;
+            f.parts = c.parts(st.level);
+            f.mont = st.montgomery ? 1 : 0;
+            f.pt_mont = st.pt_montgomery ? 1 : 0;
+            f.bc = c.d_bc;
+            // the fewest giant steps that hold f.ng, and with them as many items
+#define MI_LT_FUSED(NG, IT)                                                                            \
+    hipLaunchKernelGGL((k_lt_fused<NG, IT>), dim3(tile_grid((m + IT - 1) / IT, tps, T)), dim3(LT_THREADS), 0, s, f)
+            if (f.ng <= 4 && m > 1) MI_LT_FUSED(4, 4);
+            else if (f.ng <= 8 && m > 1) MI_LT_FUSED(8, 2);
+            else MI_LT_FUSED(16, 1);
+#undef MI_LT_FUSED
+            MI_HIP(hipGetLastError());
+        }
+    }
+}
+
 void check_batch(int n, const u64* const* a, const u64* const* b, u64* const* a_out, u64* const* b_out) {
     if (n < 1 || !a || !b || !a_out || !b_out) throw Error(-1, "null pointer argument");
     for (int i = 0; i < n; ++i)
@@ -263,9 +519,9 @@ void linear_transform_qp_batch(Context& c, const LtStage& st, int n, const u64* 
     const long long W = (long long)T * (long long)N, LN = (long long)L * (long long)N;
     const int nbaby = k.nslots - 1, ngp = k.ngp;
 
-    // per-item scratch: digits | C | babies (a, b) | out (a, b) | giant inners (a, b) | ModDown temp
+    // per-item scratch: digits | C | out (a, b) | giant inners (a, b) | ModDown temp
     const long long dw = (long long)parts * W;
-    const long long item_words = dw + LN + 2 * (long long)nbaby * W + 2 * W + 2 * (long long)ngp * W + 2 * LN;
+    const long long item_words = dw + LN + 2 * W + 2 * (long long)ngp * W + 2 * LN;
     const long long budget_words = (32LL << 30) / 8;
     int chunk = (int)std::min<long long>(KS_MAX_ITEMS, std::max<long long>(1, budget_words / item_words));
     chunk = std::min(chunk, n);
@@ -275,39 +531,16 @@ void linear_transform_qp_batch(Context& c, const LtStage& st, int n, const u64* 
         const int m = std::min(chunk, n - i0);
         u64* D = ws;
         u64* C = D + m * dw;
-        u64* BAB = C + m * LN;
-        u64* OAB = BAB + m * 2 * (long long)nbaby * W;
+        u64* OAB = C + m * LN;
         u64* IAB = OAB + m * 2 * W;
         u64* Tm = IAB + m * 2 * (long long)ngp * W;
-        auto baby = [&](int it, int sl) { return BAB + it * 2LL * nbaby * W + (long long)(sl - 1) * 2 * W; };
         auto inner = [&](int it, int gp) { return IAB + it * 2LL * ngp * W + (long long)gp * 2 * W; };
         auto outp = [&](int it) { return OAB + it * 2 * W; };
 
-        // baby steps: one hoisted ModUp, then one key product per baby step
-        // (hoisted QP rotations, :675-852), b added in the Q limbs
-        if (nbaby > 0) {
-            ks_modup_n(c, level, m, a + i0, D, dw, C, s);
-            // the baby steps' key products are independent (each writes its
-            // own baby slots from the shared digits): spread over the streams
-            over_streams(c, s, k.nslots - 1, 0, [&](hipStream_t bst, u64*, int i) {
-                const int sl = i + 1;
-                MacArgs ma = mac_args(c, level, D, k.baby_key[sl], st.montgomery != 0);
-                ma.items = m;
-                ma.digits_stride = dw;
-                ma.qp_out = 1;
-                ma.galois = k.baby_gal[sl];
-                for (int it = 0; it < m; ++it) {
-                    ma.key[it] = k.baby_key[sl];
-                    ma.a_out[it] = baby(it, sl);
-                    ma.b_out[it] = baby(it, sl) + W;
-                    ma.init_b[it] = b[i0 + it];
-                }
-                ks_mac(c, ma, level, bst);
-            });
-        }
-
-        launch_inner(c, k, st, m, K, a + i0, b + i0, BAB, 2LL * nbaby * W, 2 * W, OAB, 2 * W, IAB, 2 * W,
-                     2LL * ngp * W, s);
+        // one hoisted ModUp, then the baby steps (hoisted QP rotations, :675-852,
+        // b added in the Q limbs) and every giant step's inner product
+        if (nbaby > 0) ks_modup_n(c, level, m, a + i0, D, dw, C, s);
+        launch_fused(c, k, st, m, a + i0, b + i0, D, dw, OAB, 2 * W, IAB, 2 * W, 2LL * ngp * W, s);
 
         // giant steps > 0: key term = ModDown(inner.a); QP switch; rotate-accumulate
         // with inner.b (automorphism_qp_pair_accumulate, :373-416)

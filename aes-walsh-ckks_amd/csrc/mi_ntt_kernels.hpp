@@ -355,6 +355,15 @@ void run_ntt_inv(const Context& c, const JobIn& in, const JobOut& out, int count
     c.probe_close(probe, s);
 }
 
+// Evaluation-domain source index of output index i under Galois element g:
+// dst[brev(d)] = src[brev(((2d+1) g mod 2N - 1) / 2)].
+__device__ __forceinline__ u32 galois_index(u32 i, u64 g, int logN) {
+    const u32 mask2n = (2u << logN) - 1;
+    const u32 d = __brev(i) >> (32 - logN);
+    const u32 e = (u32)(((u64)(2 * d + 1) * g) & mask2n);
+    return __brev((e - 1) >> 1) >> (32 - logN);
+}
+
 // Block -> (item, slot, tile) with the blocks of one (slot, tile) for all
 // items consecutive on one XCD: workgroups are dealt to the 8 XCDs round
 // robin, so block b runs on XCD b % 8.  The key (or diagonal) tile that all
