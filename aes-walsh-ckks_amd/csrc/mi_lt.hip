@@ -111,7 +111,8 @@ __global__ void __launch_bounds__(LT_THREADS) k_lt_inner_all(LtAllArgs a) {
 // from memory once per launch, the digits of a limb's ciphertexts (2 MB each)
 // stay in the Infinity Cache while its tiles run.
 struct LtFusedArgs {
-    const u64* diag[LT_NG * LT_NB];  // [giant][baby slot], null: no term
+    const u64* diag[LT_NG * LT_NB];  // [giant][baby slot]; no term: a row of N zeros
+    unsigned term[LT_NB];            // bit g: baby slot slot0 + r has a term of giant g
     const u64* key[LT_NB];           // baby slot slot0 + r
     u64 galois[LT_NB];
     const u64* in_a[KS_MAX_ITEMS];
@@ -125,7 +126,10 @@ struct LtFusedArgs {
     const BasisConst* bc;
 };
 
-template <int NG, int IT>
+// All words of a rotation are loaded before any is used, the diagonals without
+// a branch (a missing term reads zeros): one wait per rotation instead of one
+// per digit and giant step.
+template <int NG, int IT, int PARTS>
 __device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisConst& b, int it0, int slot, long long i) {
     const u64 N = (u64)1 << a.logN;
     const int T = a.L + a.K, basis = slot < a.L ? slot : a.nq + (slot - a.L);
@@ -140,6 +144,10 @@ __device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisCon
 #pragma unroll
     for (int t = 0; t < IT; ++t) item[t] = it0 + t < a.items ? it0 + t : a.items - 1;  // past the end: a repeat, not stored
     for (int r = 0; r < a.nb; ++r) {
+        u64 dw[NG];
+        const unsigned term = a.term[r];
+#pragma unroll
+        for (int g = 0; g < NG; ++g) dw[g] = a.diag[g * LT_NB + r][((term >> g) & 1) ? o + i : i];
         double xa[IT], xb[IT];
         if (a.slot0 + r == 0) {
             if (slot >= a.L) continue;  // the input's P limbs are zero
@@ -152,16 +160,40 @@ __device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisCon
             const u32 src = galois_index((u32)i, a.galois[r], a.logN);
             const u64* k = a.key[r] + (long long)basis * N + src;
             const u64* d = a.digits + o + src;
+            u64 bw[IT];
 #pragma unroll
-            for (int t = 0; t < IT; ++t) xa[t] = xb[t] = 0.0;
-            // operands below 4q: each product at most 9/2 q, centred (as in k_mac)
-            for (int e = 0; e < a.parts; ++e) {
-                const double kb = fp_from_u64(k[2LL * e * to_a]), ka = fp_from_u64(k[(2LL * e + 1) * to_a]);
+            for (int t = 0; t < IT; ++t) {
+                bw[t] = slot < a.L ? a.in_b[item[t]][o + src] : 0;
+                xa[t] = xb[t] = 0.0;
+            }
+            // digits canonical, keys below 4q: each product at most 3/2 q, the
+            // sum of up to five below 8q
+            if constexpr (PARTS > 0) {
+                u64 kw[PARTS][2], xw[PARTS][IT];
 #pragma unroll
-                for (int t = 0; t < IT; ++t) {
-                    const double x = fp_from_u64(d[item[t] * a.digit_stride + (long long)e * T * N]);
-                    xb[t] += m.centred(m.mulq(x, kb));
-                    xa[t] += m.centred(m.mulq(x, ka));
+                for (int e = 0; e < PARTS; ++e) {
+                    kw[e][0] = k[2LL * e * to_a];
+                    kw[e][1] = k[(2LL * e + 1) * to_a];
+#pragma unroll
+                    for (int t = 0; t < IT; ++t) xw[e][t] = d[item[t] * a.digit_stride + (long long)e * T * N];
+                }
+#pragma unroll
+                for (int e = 0; e < PARTS; ++e)
+#pragma unroll
+                    for (int t = 0; t < IT; ++t) {
+                        const double x = fp_from_u64(xw[e][t]);
+                        xb[t] += m.mulq(x, fp_from_u64(kw[e][0]));
+                        xa[t] += m.mulq(x, fp_from_u64(kw[e][1]));
+                    }
+            } else {
+                for (int e = 0; e < a.parts; ++e) {
+                    const double kb = fp_from_u64(k[2LL * e * to_a]), ka = fp_from_u64(k[(2LL * e + 1) * to_a]);
+#pragma unroll
+                    for (int t = 0; t < IT; ++t) {
+                        const double x = fp_from_u64(d[item[t] * a.digit_stride + (long long)e * T * N]);
+                        xb[t] += m.centred(m.mulq(x, kb));
+                        xa[t] += m.centred(m.mulq(x, ka));
+                    }
                 }
             }
 #pragma unroll
@@ -170,8 +202,7 @@ __device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisCon
                     xb[t] = m.mul(xb[t], b.rinv_fp, b.rinv_fpq);
                     xa[t] = m.mul(xa[t], b.rinv_fp, b.rinv_fpq);
                 }
-                if (slot < a.L) xb[t] += fp_from_u64(a.in_b[item[t]][o + src]);
-                xb[t] = m.centred(xb[t]);
+                xb[t] = m.centred(xb[t] + fp_from_u64(bw[t]));
                 xa[t] = m.centred(xa[t]);
             }
         }
@@ -179,9 +210,7 @@ __device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisCon
         // between two reductions
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
-            const u64* dp = a.diag[g * LT_NB + r];
-            if (!dp) continue;
-            const double d = fp_from_u64(dp[o + i]);
+            const double d = fp_from_u64(dw[g]);
 #pragma unroll
             for (int t = 0; t < IT; ++t) {
                 sa[t][g] += m.mulq(xa[t], d);
@@ -260,9 +289,8 @@ __device__ __forceinline__ void lt_fused_int(const LtFusedArgs& a, const BasisCo
         }
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
-            const u64* dp = a.diag[(g0 + g) * LT_NB + r];
-            if (!dp) continue;
-            const u64 d = reduce_4q(dp[o + i], b.q);
+            if (!((a.term[r] >> (g0 + g)) & 1)) continue;
+            const u64 d = reduce_4q(a.diag[(g0 + g) * LT_NB + r][o + i], b.q);
             mac128(sa[g], xa, d);
             mac128(sb[g], xb, d);
         }
@@ -285,7 +313,8 @@ __device__ __forceinline__ void lt_fused_int(const LtFusedArgs& a, const BasisCo
     }
 }
 
-template <int NG, int IT>
+// PARTS = the digits (1 to 5), or 0: any number, one after the other.
+template <int NG, int IT, int PARTS>
 __global__ void __launch_bounds__(LT_THREADS) k_lt_fused(LtFusedArgs a) {
     const int tps = (1 << a.logN) / LT_THREADS;
     const TileMap tm = map_tile(blockIdx.x, (a.items + IT - 1) / IT, tps, a.L + a.K);
@@ -294,7 +323,7 @@ __global__ void __launch_bounds__(LT_THREADS) k_lt_fused(LtFusedArgs a) {
     const BasisConst b = a.bc[tm.slot < a.L ? tm.slot : a.nq + (tm.slot - a.L)];
     const int it0 = tm.item * IT;
     if (b.fp) {
-        lt_fused_fp<NG, IT>(a, b, it0, tm.slot, i);
+        lt_fused_fp<NG, IT, PARTS>(a, b, it0, tm.slot, i);
     } else {
 #pragma unroll 1
         for (int t = 0; t < IT && it0 + t < a.items; ++t)
@@ -466,9 +495,14 @@ void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const
                 f.key[r] = k.baby_key[s0 + r];
                 f.galois[r] = k.baby_gal[s0 + r];
             }
+            for (const u64*& d : f.diag) d = c.d_zero;
             for (int g = 0; g < f.ng; ++g) {
                 const size_t gk = gk0 + g;
-                for (int r = 0; r < f.nb; ++r) f.diag[g * LT_NB + r] = k.table[gk * k.nslots + s0 + r];
+                for (int r = 0; r < f.nb; ++r) {
+                    const u64* d = k.table[gk * k.nslots + s0 + r];
+                    f.diag[g * LT_NB + r] = d ? d : c.d_zero;
+                    if (d) f.term[r] |= 1u << g;
+                }
                 const bool first = k.glist[gk] == 0;
                 f.out[g] = first ? out0 : outg + (long long)(gk - (k.g0 ? 1 : 0)) * outg_giant;
                 f.out_stride[g] = first ? out0_stride : outg_item;
@@ -490,11 +524,22 @@ void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const
             f.pt_mont = st.pt_montgomery ? 1 : 0;
             f.bc = c.d_bc;
             // the fewest giant steps that hold f.ng, and with them as many items
-#define MI_LT_FUSED(NG, IT)                                                                            \
-    hipLaunchKernelGGL((k_lt_fused<NG, IT>), dim3(tile_grid((m + IT - 1) / IT, tps, T)), dim3(LT_THREADS), 0, s, f)
-            if (f.ng <= 4 && m > 1) MI_LT_FUSED(4, 4);
-            else if (f.ng <= 8 && m > 1) MI_LT_FUSED(8, 2);
-            else MI_LT_FUSED(16, 1);
+#define MI_LT_FUSED(NG, IT, PARTS)                                                                     \
+    hipLaunchKernelGGL((k_lt_fused<NG, IT, PARTS>), dim3(tile_grid((m + IT - 1) / IT, tps, T)),        \
+                       dim3(LT_THREADS), 0, s, f)
+#define MI_LT_FUSED_P(PARTS)                                                                           \
+    if (f.ng <= 4 && m > 1) MI_LT_FUSED(4, 4, PARTS);                                                  \
+    else if (f.ng <= 8 && m > 1) MI_LT_FUSED(8, 2, PARTS);                                             \
+    else MI_LT_FUSED(16, 1, PARTS);
+            switch (f.parts) {
+                case 1: MI_LT_FUSED_P(1) break;
+                case 2: MI_LT_FUSED_P(2) break;
+                case 3: MI_LT_FUSED_P(3) break;
+                case 4: MI_LT_FUSED_P(4) break;
+                case 5: MI_LT_FUSED_P(5) break;
+                default: MI_LT_FUSED_P(0)
+            }
+#undef MI_LT_FUSED_P
 #undef MI_LT_FUSED
             MI_HIP(hipGetLastError());
         }
@@ -687,11 +732,15 @@ void linear_transform_q_batch(Context& c, const LtStage& st, int n, const u64* c
                              have_out, s);
             have_out = true;
         }
+        u64* dst[2 * KS_MAX_ITEMS];
+        const u64* src[2 * KS_MAX_ITEMS];
         for (int it = 0; it < m; ++it) {
-            MI_HIP(hipMemcpyAsync(a_out[i0 + it], OQ + it * 2 * LN, sizeof(u64) * LN, hipMemcpyDeviceToDevice, s));
-            MI_HIP(hipMemcpyAsync(b_out[i0 + it], OQ + it * 2 * LN + LN, sizeof(u64) * LN,
-                                  hipMemcpyDeviceToDevice, s));
+            dst[2 * it] = a_out[i0 + it];
+            dst[2 * it + 1] = b_out[i0 + it];
+            src[2 * it] = OQ + it * 2 * LN;
+            src[2 * it + 1] = src[2 * it] + LN;
         }
+        pair_list_op(c, 0, level, dst, src, 2 * m, nullptr, s);  // copy
     }
 }
 
