@@ -590,15 +590,11 @@ int mi_rotate(mi_context* ctx, int level, uint64_t* b, uint64_t* a, uint64_t gal
         check_ctx(ctx);
         check_level(*ctx->c, level);
         check_ptr(b); check_ptr(a); check_ptr(key);
+        check_galois(galois, false);
         mi::Context& c = *ctx->c;
-        const int L = level + 1;
-        const long long words = (long long)L * (long long)c.N;
-        mi::keyswitch(c, mi::KsItem{a, key, b, a, level, 0, 1}, montgomery != 0, S(stream));
-        uint64_t* tmp = (uint64_t*)c.workspace(S(stream), sizeof(uint64_t) * 2 * words);
-        mi::automorphism(c, L, galois, b, tmp, 1, words, words, S(stream));
-        mi::automorphism(c, L, galois, a, tmp + words, 1, words, words, S(stream));
-        MI_HIP(hipMemcpyAsync(b, tmp, sizeof(uint64_t) * words, hipMemcpyDeviceToDevice, S(stream)));
-        MI_HIP(hipMemcpyAsync(a, tmp + words, sizeof(uint64_t) * words, hipMemcpyDeviceToDevice, S(stream)));
+        // switch into staging (b added in the same pass), one automorphism
+        // launch for both polys back into the ciphertext
+        mi::rotate_batch(c, level, 1, &b, &a, &galois, &key, montgomery != 0, S(stream));
     });
 }
 
@@ -609,15 +605,7 @@ int mi_conjugate(mi_context* ctx, int level, uint64_t* b, uint64_t* a, const uin
         check_level(*ctx->c, level);
         check_ptr(b); check_ptr(a); check_ptr(key);
         mi::Context& c = *ctx->c;
-        const int L = level + 1;
-        const long long words = (long long)L * (long long)c.N;
-        const uint64_t g = 2 * c.N - 1;
-        uint64_t* tmp = (uint64_t*)c.workspace(S(stream), sizeof(uint64_t) * 2 * words);
-        mi::automorphism(c, L, g, b, tmp, 1, words, words, S(stream));
-        mi::automorphism(c, L, g, a, tmp + words, 1, words, words, S(stream));
-        MI_HIP(hipMemcpyAsync(b, tmp, sizeof(uint64_t) * words, hipMemcpyDeviceToDevice, S(stream)));
-        MI_HIP(hipMemcpyAsync(a, tmp + words, sizeof(uint64_t) * words, hipMemcpyDeviceToDevice, S(stream)));
-        mi::keyswitch(c, mi::KsItem{a, key, b, a, level, 0, 1}, montgomery != 0, S(stream));
+        mi::conjugate(c, level, b, a, key, montgomery != 0, S(stream));
     });
 }
 

@@ -362,6 +362,7 @@ void keyswitch_batch(Context& c, const KsItem* items, int n, bool montgomery, hi
 // In-place conjugations of independent ciphertexts at one level: one
 // automorphism launch per KS_MAX_ITEMS ciphertexts into scratch, then their
 // key switches as one batch (the conjugated b enters as the switch's init_b).
+void conjugate(Context& c, int level, u64* b, u64* a, const u64* key, bool montgomery, hipStream_t s);
 void conjugate_batch(Context& c, int level, int n, u64* const* b, u64* const* a, const u64* key, bool montgomery,
                      hipStream_t s);
 // One key switch with its scratch in the library's fixed device array

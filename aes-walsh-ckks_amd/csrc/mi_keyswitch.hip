@@ -666,6 +666,27 @@ __global__ void __launch_bounds__(KS_THREADS) k_automorphism_list(AutoListArgs a
     a.dst[k][off + i] = a.src[k][off + galois_index(i, a.galois, a.logN)];
 }
 
+// One conjugation: both automorphisms in one launch into the workspace, from
+// which the key switch reads its term and the b it adds.
+void conjugate(Context& c, int level, u64* b, u64* a, const u64* key, bool montgomery, hipStream_t s) {
+    if (level < 0 || level >= c.nq) throw Error(-1, "invalid ciphertext level");
+    const int L = level + 1;
+    const long long LN = (long long)L * (long long)c.N;
+    u64* tmp = (u64*)c.workspace(s, sizeof(u64) * (2 * (size_t)LN + ks_item_words(c, level)));
+    AutoListArgs al{};
+    al.src[0] = a;
+    al.src[1] = b;
+    al.dst[0] = tmp;
+    al.dst[1] = tmp + LN;
+    al.galois = 2 * c.N - 1;
+    al.L = L;
+    al.logN = c.logN;
+    hipLaunchKernelGGL(k_automorphism_list, dim3((unsigned)(2 * L * (c.N / KS_THREADS))), dim3(KS_THREADS), 0, s, al);
+    MI_HIP(hipGetLastError());
+    const KsItem it{tmp, key, b, a, level, 1, 1, tmp + LN};
+    keyswitch_items_with(c, &it, 1, montgomery, tmp + 2 * LN, s);
+}
+
 void conjugate_batch(Context& c, int level, int n, u64* const* b, u64* const* a, const u64* key, bool montgomery,
                      hipStream_t s) {
     if (level < 0 || level >= c.nq) throw Error(-1, "invalid ciphertext level");
