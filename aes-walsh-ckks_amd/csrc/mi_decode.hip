@@ -15,6 +15,7 @@
 //   * the FFT stages in double with the host's operation order (complex
 //     product (ac - bd, ad + bc), then t + u and t - u; no contraction).
 #include "mi_arith.hpp"
+#include "mi_fft.hpp"
 #include "mi_internal.hpp"
 
 namespace mi {
@@ -155,27 +156,12 @@ __global__ void __launch_bounds__(DEC_THREADS) k_dec_crt(CrtArgs a) {
     m[2 * j + 1] = 0.0;
 }
 
-// one radix-2 stage of fft_dit: m groups of span 2k (tw[m + i] for group i)
-__global__ void __launch_bounds__(DEC_THREADS)
-k_dec_fft_stage(double* __restrict__ x, const double* __restrict__ tw, int logN, int m, int k, long long total) {
-    const long long t = (long long)blockIdx.x * DEC_THREADS + threadIdx.x;
-    if (t >= total) return;
-    const long long N = 1ll << logN;
-    const long long half = N >> 1;
-    const long long ct = t / half, b = t - ct * half;
-    const long long i = b / k, j = b - i * k;
-    double* v = x + ct * 2 * N;
-    const long long i0 = (i << 1) * k + j, i1 = i0 + k;
-    const double wr = tw[2 * (m + i)], wi = tw[2 * (m + i) + 1];
-    const double tr = v[2 * i0], ti = v[2 * i0 + 1];
-    const double ar = v[2 * i1], ai = v[2 * i1 + 1];
-    const double ur = __dsub_rn(__dmul_rn(ar, wr), __dmul_rn(ai, wi));
-    const double ui = __dadd_rn(__dmul_rn(ar, wi), __dmul_rn(ai, wr));
-    v[2 * i0] = __dadd_rn(tr, ur);
-    v[2 * i0 + 1] = __dadd_rn(ti, ui);
-    v[2 * i1] = __dsub_rn(tr, ur);
-    v[2 * i1 + 1] = __dsub_rn(ti, ui);
-}
+// the column pass's result as the block pass's input
+struct DecPoints {
+    const C64* x;
+    int logN;
+    __device__ C64 operator()(int b, int j) const { return x[((long long)b << logN) + j]; }
+};
 
 // slots: out[i] = m[perm[i]]; coefficients: out[i] = (m[brev i].re, m[N/2 + brev i].re)
 __global__ void __launch_bounds__(DEC_THREADS)
@@ -263,12 +249,11 @@ void decode_batch(Context& c, int count, const u64* const* coeffs, int limbs, co
         hipLaunchKernelGGL(k_dec_crt, dim3((unsigned)(N / DEC_THREADS), n), dim3(DEC_THREADS), 0, s, a);
         MI_HIP(hipGetLastError());
         const long long total = (long long)n * (long long)(N >> 1);
-        if (!coeff_domain)
-            for (int m = 1, k = (int)(N >> 1); m < (int)N; m <<= 1, k >>= 1) {
-                hipLaunchKernelGGL(k_dec_fft_stage, dim3(dec_blocks(total)), dim3(DEC_THREADS), 0, s, work,
-                                   c.d_dec_tw, c.logN, m, k, total);
-                MI_HIP(hipGetLastError());
-            }
+        if (!coeff_domain) {
+            const C64* tw = (const C64*)c.d_dec_tw;
+            launch_fft_cols<false>((C64*)work, tw, c.logN, n, s);
+            launch_fft_block<false>(DecPoints{(const C64*)work, c.logN}, (C64*)work, tw, c.logN, n, s);
+        }
         hipLaunchKernelGGL(k_dec_out, dim3(dec_blocks(total)), dim3(DEC_THREADS), 0, s, work, c.d_dec_perm,
                            out + (size_t)c0 * N, c.logN, coeff_domain ? 1 : 0, total);
         MI_HIP(hipGetLastError());

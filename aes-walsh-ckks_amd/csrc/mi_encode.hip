@@ -7,6 +7,7 @@
 // Every double operation is a separately rounded IEEE multiply, add or
 // subtract in the reference's order (no contraction), so the rounded
 // integers - and hence the residues - equal the host restatement's bit for bit.
+#include "mi_fft.hpp"
 #include "mi_ntt_kernels.hpp"
 
 #include <cmath>
@@ -17,46 +18,19 @@ namespace mi {
 
 constexpr int ENC_THREADS = 256;
 
-// inv[j] = i + 1: ev[j] = z_i; -(i + 1): ev[j] = conj(z_i); 0: ev[j] = 0
-__global__ void __launch_bounds__(ENC_THREADS)
-k_enc_place(const double* __restrict__ z, const int* __restrict__ inv, double* __restrict__ ev, int N,
-            long long total) {
-    const long long t = (long long)blockIdx.x * ENC_THREADS + threadIdx.x;
-    if (t >= total) return;
-    const long long b = t / N;
-    const int j = (int)(t - b * N);
-    const int s = inv[j];
-    double re = 0.0, im = 0.0;
-    if (s != 0) {
-        const int i = (s > 0 ? s : -s) - 1;
-        const double* zi = z + (b * (N >> 1) + i) * 2;
-        re = zi[0];
-        im = s > 0 ? zi[1] : -zi[1];
+// Slot placement as the FFT's input: inv[j] = i + 1: ev[j] = z_i; -(i + 1):
+// ev[j] = conj(z_i); 0: ev[j] = 0
+struct EncPlace {
+    const C64* z;
+    const int* inv;
+    int logN;
+    __device__ C64 operator()(int b, int j) const {
+        const int s = inv[j];
+        if (s == 0) return C64{0.0, 0.0};
+        const C64 v = z[((long long)b << (logN - 1)) + (s > 0 ? s : -s) - 1];
+        return C64{v.re, s > 0 ? v.im : -v.im};
     }
-    ev[t * 2] = re;
-    ev[t * 2 + 1] = im;
-}
-
-// One decimation-in-frequency stage: block pairs (2i k + j, 2i k + j + k)
-// with twiddle tw[m + i]; x0 = u + v, x1 = (u - v) w.
-__global__ void __launch_bounds__(ENC_THREADS)
-k_fft_dif_stage(double* __restrict__ ev, const double* __restrict__ tw, int N, int m, int k, long long total) {
-    const long long t = (long long)blockIdx.x * ENC_THREADS + threadIdx.x;
-    if (t >= total) return;
-    const int half = N >> 1;
-    const long long b = t / half;
-    const int r = (int)(t - b * half);
-    const int i = r / k, j = r - i * k;
-    double* x0 = ev + (b * N + 2LL * i * k + j) * 2;
-    double* x1 = x0 + 2LL * k;
-    const double ur = x0[0], ui = x0[1], vr = x1[0], vi = x1[1];
-    const double wr = tw[2 * (m + i)], wi = tw[2 * (m + i) + 1];
-    x0[0] = __dadd_rn(ur, vr);
-    x0[1] = __dadd_rn(ui, vi);
-    const double dr = __dsub_rn(ur, vr), di = __dsub_rn(ui, vi);
-    x1[0] = __dsub_rn(__dmul_rn(dr, wr), __dmul_rn(di, wi));
-    x1[1] = __dadd_rn(__dmul_rn(dr, wi), __dmul_rn(di, wr));
-}
+};
 
 // Rounded real parts as signed residues of every limb.
 __global__ void __launch_bounds__(ENC_THREADS)
@@ -109,15 +83,12 @@ void encode_slots(Context& c, const double* values, int count, double scale, int
     double* z = (double*)c.workspace(s, sizeof(double) * (zwords + evwords));
     double* ev = z + zwords;
     MI_HIP(hipMemcpyAsync(z, values, sizeof(double) * zwords, hipMemcpyHostToDevice, s));
-    const long long total = (long long)count * N;
-    hipLaunchKernelGGL(k_enc_place, dim3(enc_blocks(total)), dim3(ENC_THREADS), 0, s, z, c.d_enc_inv, ev, N,
-                       total);
-    MI_HIP(hipGetLastError());
-    const long long bf = (long long)count * (N >> 1);
-    for (int m = N >> 1, k = 1; m > 0; m >>= 1, k <<= 1) {
-        hipLaunchKernelGGL(k_fft_dif_stage, dim3(enc_blocks(bf)), dim3(ENC_THREADS), 0, s, ev, c.d_enc_tw, N, m,
-                           k, bf);
-        MI_HIP(hipGetLastError());
+    const C64* tw = (const C64*)c.d_enc_tw;
+    for (int c0 = 0; c0 < count; c0 += 32768) {  // transforms are blockIdx.y
+        const int n = std::min(32768, count - c0);
+        C64* x = (C64*)ev + (size_t)c0 * N;
+        launch_fft_block<true>(EncPlace{(const C64*)z + (size_t)c0 * (N / 2), c.d_enc_inv, c.logN}, x, tw, c.logN, n, s);
+        launch_fft_cols<true>(x, tw, c.logN, n, s);
     }
     const long long rt = (long long)count * limbs * N;
     hipLaunchKernelGGL(k_enc_round, dim3(enc_blocks(rt)), dim3(ENC_THREADS), 0, s, ev, c.d_bc, out, N, limbs,
