@@ -175,14 +175,16 @@ CKKSCiphertext ckks_encrypt(const CKKSContext& c, const CKKSEncoding& encd, bool
         mi_check(mi_memcpy(mi, b, one.data(), L * N * 8, MI_COPY_D2D, c.stream()), "ckks_encrypt(ptxt)");
         mi_check(mi_stream_synchronize(mi, c.stream()), "ckks_encrypt(ptxt)");
     }
-    if (!eval) mi_check(mi_ntt_forward(mi, b, 1, (int)L, W, 0, c.stream()), "ckks_encrypt(ptxt)");
-    // a uniform (evaluation domain) and e Gaussian, drawn on the device
+    // a uniform (evaluation domain) and e Gaussian, drawn on the device; a
+    // plaintext in coefficients takes e before its transform (the transform is
+    // linear, residues exact)
     const uint64_t seed = c.nextRandomnessSeed();
     mi_check(mi_sample_uniform(mi, a, (int)L, 0, seed, 0, c.stream()), "ckks_encrypt(ptxt)");
     DeviceBuffer tmp(mi, L * N);
     mi_check(mi_sample_gaussian(mi, tmp.data(), (int)L, P.getSigma(), seed, 1, c.stream()), "ckks_encrypt(ptxt)");
-    mi_check(mi_ntt_forward(mi, tmp.data(), 1, (int)L, W, 0, c.stream()), "ckks_encrypt(ptxt)");
+    if (eval) mi_check(mi_ntt_forward(mi, tmp.data(), 1, (int)L, W, 0, c.stream()), "ckks_encrypt(ptxt)");
     mi_check(mi_poly_op(mi, MI_OP_ADD, b, tmp.data(), (int)L, 0, 1, W, c.stream()), "ckks_encrypt(ptxt)");
+    if (!eval) mi_check(mi_ntt_forward(mi, b, 1, (int)L, W, 0, c.stream()), "ckks_encrypt(ptxt)");
     mi_check(mi_memcpy(mi, tmp.data(), a, L * N * 8, MI_COPY_D2D, c.stream()), "ckks_encrypt(ptxt)");
     mi_check(mi_poly_op(mi, MI_OP_MUL, tmp.data(), c.secretKeyDevice(), (int)L, 0, 1, W, c.stream()), "ckks_encrypt(ptxt)");
     mi_check(mi_poly_op(mi, MI_OP_SUB, b, tmp.data(), (int)L, 0, 1, W, c.stream()), "ckks_encrypt(ptxt)");
