@@ -14,6 +14,12 @@
 namespace mi {
 
 namespace {
+template <bool FWD, bool ROWS, Arith A>
+void one_limb(const Context& c, const PlainJob& job, int count, hipStream_t s) {
+    if constexpr (ROWS) launch_rows<FWD, 1, false, A>(c, job, count, s);
+    else launch_cols<FWD, 1, false, A>(c, job, count, s);
+}
+
 template <bool FWD, bool ROWS>
 void plain_pass(const Context& c, int variant, const PlainJob& job, int count, hipStream_t s) {
     switch (variant) {
@@ -25,9 +31,13 @@ void plain_pass(const Context& c, int variant, const PlainJob& job, int count, h
             if constexpr (ROWS) launch_rows<FWD, 1, true>(c, job, count, s);
             else launch_cols<FWD, 1, true>(c, job, count, s);
             break;
-        default:
-            if constexpr (ROWS) launch_rows<FWD, 1, false>(c, job, count, s);
-            else launch_cols<FWD, 1, false>(c, job, count, s);
+        default: {
+            int fp = 0;
+            for (int l = 0; l < job.b.lpp; ++l) fp += c.h_bc[job.b.basis0 + l].fp ? 1 : 0;
+            if (fp == 0) one_limb<FWD, ROWS, Arith::Int>(c, job, count, s);
+            else if (fp == job.b.lpp) one_limb<FWD, ROWS, Arith::Fp>(c, job, count, s);
+            else one_limb<FWD, ROWS, Arith::Both>(c, job, count, s);
+        }
     }
 }
 }  // namespace

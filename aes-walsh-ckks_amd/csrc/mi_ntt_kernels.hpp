@@ -220,9 +220,15 @@ __device__ __forceinline__ void pass_body(const NttTabs& tb, const V (&v)[LPB], 
     }
 }
 
+// The arithmetics a kernel holds.  With both, the compiler shares address
+// registers across them and a pass takes up to 134 registers where either
+// alone takes 100 to 106 (the integer forward column pass loses a wave per
+// SIMD), so in-place batches whose moduli are of one kind get a kernel of their own.
+enum class Arith { Both, Int, Fp };
+
 // A workgroup's limbs (limb_views) through one pass in the arithmetic of their
 // moduli; two limbs are interleaved only if both are integer limbs.
-template <int LOGN, bool FWD, bool ROWS, int LPB, bool HALF, class Job>
+template <int LOGN, bool FWD, bool ROWS, int LPB, bool HALF, Arith A, class Job>
 __device__ __forceinline__ void ntt_pass(const NttTabs& tb, const Job& job, int count) {
     constexpr int n1 = LOGN / 2, n2 = LOGN - n1;
     constexpr int wpl = ROWS ? pass_wpl(n2, n1) : pass_wpl(n1, n2);
@@ -236,7 +242,11 @@ __device__ __forceinline__ void ntt_pass(const NttTabs& tb, const Job& job, int 
     int fp = 0;
 #pragma unroll
     for (int i = 0; i < LPB; ++i) fp += tb.fp(v[i].basis) ? 1 : 0;
-    if constexpr (LPB == 1) {
+    if constexpr (A == Arith::Int) {
+        pass_body<LOGN, FWD, ROWS, LPB, BfInt>(tb, v, live, w, lds);
+    } else if constexpr (A == Arith::Fp) {
+        pass_body<LOGN, FWD, ROWS, LPB, BfFp>(tb, v, live, w, lds);
+    } else if constexpr (LPB == 1) {
         if (fp) pass_body<LOGN, FWD, ROWS, 1, BfFp>(tb, v, live, w, lds);
         else pass_body<LOGN, FWD, ROWS, 1, BfInt>(tb, v, live, w, lds);
     } else if (fp == 0) {
@@ -255,13 +265,13 @@ __device__ __forceinline__ void ntt_pass(const NttTabs& tb, const Job& job, int 
     }
 }
 
-template <int LOGN, bool FWD, int LPB, bool HALF, class Job>
+template <int LOGN, bool FWD, int LPB, bool HALF, Arith A, class Job>
 __global__ void __launch_bounds__(NTT_THREADS) k_ntt_cols(NttTabs tb, Job job, int count) {
-    ntt_pass<LOGN, FWD, false, LPB, HALF>(tb, job, count);
+    ntt_pass<LOGN, FWD, false, LPB, HALF, A>(tb, job, count);
 }
-template <int LOGN, bool FWD, int LPB, bool HALF, class Job>
+template <int LOGN, bool FWD, int LPB, bool HALF, Arith A, class Job>
 __global__ void __launch_bounds__(NTT_THREADS) k_ntt_rows(NttTabs tb, Job job, int count) {
-    ntt_pass<LOGN, FWD, true, LPB, HALF>(tb, job, count);
+    ntt_pass<LOGN, FWD, true, LPB, HALF, A>(tb, job, count);
 }
 // The same pass held to 128 VGPRs (four waves per SIMD, the LDS limit), for
 // jobs whose load or store does enough work of its own that the scheduler
@@ -269,7 +279,7 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ntt_rows(NttTabs tb, Job job, i
 template <int LOGN, bool FWD, class Job>
 __global__ void __launch_bounds__(NTT_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 k_ntt_rows_w4(NttTabs tb, Job job, int count) {
-    ntt_pass<LOGN, FWD, true, 1, false>(tb, job, count);
+    ntt_pass<LOGN, FWD, true, 1, false, Arith::Both>(tb, job, count);
 }
 
 #define MI_NTT_LOGN_CASES(K)                                                                          \
@@ -284,26 +294,26 @@ k_ntt_rows_w4(NttTabs tb, Job job, int count) {
         default: throw Error(-1, "ntt: unsupported ring dimension");                                  \
     }
 
-template <bool FWD, int LPB, bool HALF, class Job>
+template <bool FWD, int LPB, bool HALF, Arith A = Arith::Both, class Job>
 void launch_cols(const Context& c, const Job& job, int count, hipStream_t s) {
     if (count >= (1 << 20)) throw Error(-1, "ntt: more than 2^20 limbs in one launch");
     const NttTabs tb = tabs_of(c);
     const unsigned blocks = (unsigned)((count + LPB - 1) / LPB);
 #define MI_COLS(LN)                                                                                   \
-    hipLaunchKernelGGL((k_ntt_cols<LN, FWD, LPB, HALF, Job>), dim3(blocks * pass_wpl(LN / 2, LN - LN / 2)), \
+    hipLaunchKernelGGL((k_ntt_cols<LN, FWD, LPB, HALF, A, Job>), dim3(blocks * pass_wpl(LN / 2, LN - LN / 2)), \
                        dim3(pass_threads(LN / 2, LN - LN / 2)), 0, s, tb, job, count)
     MI_NTT_LOGN_CASES(MI_COLS)
 #undef MI_COLS
     MI_HIP(hipGetLastError());
 }
 
-template <bool FWD, int LPB, bool HALF, class Job>
+template <bool FWD, int LPB, bool HALF, Arith A = Arith::Both, class Job>
 void launch_rows(const Context& c, const Job& job, int count, hipStream_t s) {
     if (count >= (1 << 20)) throw Error(-1, "ntt: more than 2^20 limbs in one launch");
     const NttTabs tb = tabs_of(c);
     const unsigned blocks = (unsigned)((count + LPB - 1) / LPB);
 #define MI_ROWS(LN)                                                                                   \
-    hipLaunchKernelGGL((k_ntt_rows<LN, FWD, LPB, HALF, Job>), dim3(blocks * pass_wpl(LN - LN / 2, LN / 2)), \
+    hipLaunchKernelGGL((k_ntt_rows<LN, FWD, LPB, HALF, A, Job>), dim3(blocks * pass_wpl(LN - LN / 2, LN / 2)), \
                        dim3(pass_threads(LN - LN / 2, LN / 2)), 0, s, tb, job, count)
     MI_NTT_LOGN_CASES(MI_ROWS)
 #undef MI_ROWS
