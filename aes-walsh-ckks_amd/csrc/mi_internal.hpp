@@ -299,6 +299,8 @@ struct KsItem {
     u64* a_out;
     int level, b_mode, a_mode;
     const u64* init_b = nullptr;  // optional L-limb term added to the switched b before it is combined
+    u64 galois = 0;               // folded ModDown, Assign modes: the outputs through this automorphism
+                                  //   (they must not overlap init_b then)
 };
 void keyswitch(Context& c, const KsItem& it, bool montgomery, hipStream_t s);
 
@@ -340,9 +342,10 @@ MacArgs mac_args(const Context& c, int level, const u64* digits, const u64* key,
 void ks_modup_n(Context& c, int level, int n, const u64* const* key_terms, u64* D, long long dstride,
                 u64* C, hipStream_t s);
 // ModDown of n key switches (one level and modes) with the key inner
-// product of their digits folded in (split form); at most 3 digits.
+// product of their digits folded in (split form); at most 3 digits.  Item i
+// reads the digits at D + ((first + i) mod period) * dstride (period 0: its own).
 void ks_moddown_mac(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,
-                    u64* T, bool montgomery, hipStream_t s);
+                    u64* T, bool montgomery, hipStream_t s, int first = 0, int period = 0);
 void ks_modup(Context& c, int level, const u64* key_term, u64* D, u64* C, hipStream_t s);
 void ks_mac(const Context& c, const MacArgs& a, int level, hipStream_t s);
 void ks_moddown_n(Context& c, int level, int npoly, u64* const* p, const u64* const* base, u64* const* out,

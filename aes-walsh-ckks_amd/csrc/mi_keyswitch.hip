@@ -537,27 +537,30 @@ void rotate_hoisted_items(Context& c, int level, const u64* digits, long long ds
     const int per_block = (period + chunk - 1) / chunk;
     const int nblocks = (n + period - 1) / period;
     const bool fold = c.parts(level) <= 3 && c.fuse_mac;
-    // per rotation: P accumulators (a, b) | switched pair (a, b) | ModDown temp
-    const size_t ws_bytes = sizeof(u64) * (size_t)chunk * (2 * KN + 4 * LN);
+    // per rotation: P accumulators (a, b) | ModDown temp | switched pair (a, b; not folded)
+    const size_t ws_bytes = sizeof(u64) * (size_t)chunk * (2 * KN + (fold ? 2 : 4) * LN);
     over_streams(c, s, nblocks * per_block, ws_bytes, [&](hipStream_t st, u64* ws, int ci) {
         const int blk = ci / per_block, cb = ci - blk * per_block;
         const int i0 = blk * period + cb * chunk;
         if (i0 >= n) return;
         const int m = std::min(std::min(chunk, period - cb * chunk), n - i0);
         u64* AP = ws;
-        u64* SW = AP + chunk * 2 * KN;
-        u64* Tm = SW + chunk * 2 * LN;
+        u64* Tm = AP + chunk * 2 * KN;
+        u64* SW = Tm + chunk * 2 * LN;
         const u64* dig = digits + (long long)(cb * chunk) * dstride;
         // key products of the hoisted digits, b added in the Q limbs
-        // (ckks_hybrid_key_switch_hoisted_inplace with b Add, a Assign),
-        // into the staging pairs
+        // (ckks_hybrid_key_switch_hoisted_inplace with b Add, a Assign): folded,
+        // the last pass stores through the rotation's map; else into staging
+        // pairs, permuted by a pass of their own
         if (fold) {
             KsItem items[KS_MAX_ITEMS];
             for (int it = 0; it < m; ++it)
-                items[it] = KsItem{nullptr, keys[i0 + it], SW + it * 2 * LN + LN, SW + it * 2 * LN, level, 1, 1,
-                                   b[i0 + it]};
+                items[it] = KsItem{nullptr, keys[i0 + it], b_out[i0 + it], a_out[i0 + it], level, 1, 1, b[i0 + it],
+                                   galois[i0 + it] % (2 * N)};
             ks_moddown_mac(c, level, m, items, dig, dstride, AP, Tm, montgomery, st);
-        } else {
+            return;
+        }
+        {
             MacArgs ma = mac_args(c, level, dig, keys[i0], montgomery);
             ma.items = m;
             ma.digits_stride = dstride;

@@ -650,16 +650,23 @@ void linear_transform_q_batch(Context& c, const LtStage& st, int n, const u64* c
     const long long budget_words = (32LL << 30) / 8;
     int chunk = (int)std::min<long long>(KS_MAX_ITEMS, std::max<long long>(1, budget_words / item_words));
     chunk = std::min(chunk, n);
-    u64* ws = (u64*)c.workspace(s, sizeof(u64) * (size_t)(item_words * chunk));
+    // Folded, the baby steps of all ciphertexts are one batch and so are the
+    // giant steps' switches, KS_MAX_ITEMS at a time: a few ciphertexts' single
+    // steps leave most of the chip idle.
+    const bool fold = parts <= 3 && c.fuse_mac;
+    const int ck = fold ? (int)std::min<long long>(KS_MAX_ITEMS, (long long)chunk * std::max(1, std::max(nbaby, ngp)))
+                        : chunk;
+    const long long step_words = dw + LN + 2 * KN + 2 * LN + 2 * LN;  // digits | C | P accumulators | temp | switched
+    u64* ws = (u64*)c.workspace(s, sizeof(u64) * (size_t)(step_words * ck + (item_words - step_words) * chunk));
 
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int m = std::min(chunk, n - i0);
         u64* D = ws;
-        u64* C = D + m * dw;
-        u64* AP = C + m * LN;
-        u64* Tm = AP + m * 2 * KN;
-        u64* SW = Tm + m * 2 * LN;
-        u64* BQ = SW + m * 2 * LN;
+        u64* C = D + ck * dw;
+        u64* AP = C + ck * LN;
+        u64* Tm = AP + ck * 2 * KN;
+        u64* SW = Tm + ck * 2 * LN;
+        u64* BQ = SW + ck * 2 * LN;
         u64* OQ = BQ + m * 2 * (long long)nbaby * LN;
         u64* IQ = OQ + m * 2 * LN;
         u64* p[2 * KS_MAX_ITEMS];
@@ -670,14 +677,6 @@ void linear_transform_q_batch(Context& c, const LtStage& st, int n, const u64* c
         // starting from b_init), modes Assign: the hoisted or full switch
         // of ckks_hybrid_key_switch_(hoisted_)inplace
         auto mac_moddown = [&](const u64* key, const u64* const* b_init) {
-            if (parts <= 3 && c.fuse_mac) {
-                // the key product folded into ModDown's NTT passes
-                KsItem items[KS_MAX_ITEMS];
-                for (int it = 0; it < m; ++it)
-                    items[it] = KsItem{nullptr, key, SW + it * 2 * LN + LN, SW + it * 2 * LN, level, 1, 1, b_init[it]};
-                ks_moddown_mac(c, level, m, items, D, dw, AP, Tm, st.montgomery != 0, s);
-                return;
-            }
             MacArgs ma = mac_args(c, level, D, key, st.montgomery != 0);
             ma.items = m;
             ma.digits_stride = dw;
@@ -705,7 +704,18 @@ void linear_transform_q_batch(Context& c, const LtStage& st, int n, const u64* c
         // with b Add and a Assign, then the automorphism), [slot][item] layout
         if (nbaby > 0) {
             ks_modup_n(c, level, m, a + i0, D, dw, C, s);
-            for (int sl = 1; sl < k.nslots; ++sl) {
+            // (slot, ciphertext) pairs in order, each stored through its rotation's map
+            for (int j0 = 0; fold && j0 < nbaby * m; j0 += ck) {
+                const int n1 = std::min(ck, nbaby * m - j0);
+                KsItem items[KS_MAX_ITEMS];
+                for (int e = 0; e < n1; ++e) {
+                    const int sl = (j0 + e) / m + 1, it = (j0 + e) % m;
+                    u64* o = BQ + ((long long)(sl - 1) * m + it) * 2 * LN;
+                    items[e] = KsItem{nullptr, k.baby_key[sl], o + LN, o, level, 1, 1, b[i0 + it], k.baby_gal[sl]};
+                }
+                ks_moddown_mac(c, level, n1, items, D, dw, AP, Tm, st.montgomery != 0, s, j0, m);
+            }
+            for (int sl = 1; !fold && sl < k.nslots; ++sl) {
                 mac_moddown(k.baby_key[sl], b + i0);
                 automorphism(c, L, k.baby_gal[sl], SW, BQ + (long long)(sl - 1) * m * 2 * LN, 2 * m, LN, LN, s);
             }
@@ -717,7 +727,35 @@ void linear_transform_q_batch(Context& c, const LtStage& st, int n, const u64* c
         // giant steps > 0: rotate each inner sum by a full key switch
         // (ckks_rotate_inplace: switch a, then the automorphism) and add
         bool have_out = k.g0;
-        for (int gp = 0; gp < ngp; ++gp) {
+        for (int j0 = 0; fold && j0 < ngp * m; j0 += ck) {
+            const int n1 = std::min(ck, ngp * m - j0);
+            const u64* kt[KS_MAX_ITEMS];
+            KsItem items[KS_MAX_ITEMS];
+            for (int e = 0; e < n1; ++e) {
+                const size_t gk = (size_t)((j0 + e) / m) + (k.g0 ? 1 : 0);
+                const u64* in = IQ + (long long)(j0 + e) * 2 * LN;
+                u64* o = SW + (long long)e * 2 * LN;
+                kt[e] = in;
+                items[e] = KsItem{nullptr, k.giant_key[gk], o + LN, o, level, 1, 1, in + LN,
+                                  rotation_galois(N, (long long)k.glist[gk] * k.bs)};
+            }
+            ks_modup_n(c, level, n1, kt, D, dw, C, s);
+            ks_moddown_mac(c, level, n1, items, D, dw, AP, Tm, st.montgomery != 0, s);
+            // the switched sums of one giant step at a time onto the ciphertexts
+            for (int e = 0; e < n1;) {
+                const int it0 = (j0 + e) % m, run = std::min(n1 - e, m - it0);
+                u64* dst[2 * KS_MAX_ITEMS];
+                const u64* src[2 * KS_MAX_ITEMS];
+                for (int r = 0; r < 2 * run; ++r) {
+                    dst[r] = OQ + ((long long)it0 * 2 + r) * LN;
+                    src[r] = SW + ((long long)e * 2 + r) * LN;
+                }
+                const bool first = !k.g0 && (j0 + e) / m == 0;
+                pair_list_op(c, first ? 0 : 1, level, dst, src, 2 * run, nullptr, s);  // copy or add
+                e += run;
+            }
+        }
+        for (int gp = 0; !fold && gp < ngp; ++gp) {
             const size_t gk = (size_t)gp + (k.g0 ? 1 : 0);
             u64* in = IQ + (long long)gp * m * 2 * LN;
             const u64* kt[KS_MAX_ITEMS];

@@ -43,8 +43,10 @@ __device__ __forceinline__ double key_product_fp(const u64* dig, long long dstep
 }
 
 struct KeyProductLists {
-    const u64* digits;  // item i's digits at digits + i * dstride: [parts][L+K][N]
+    const u64* digits;  // item i's digits at digits + ((first + i) mod period) * dstride: [parts][L+K][N]
     long long dstride;
+    int first, period;
+    FastDiv per_period;
     const u64* key[KS_MAX_ITEMS];
     int L, K, nq;
     u64 N;
@@ -52,8 +54,8 @@ struct KeyProductLists {
     const BasisConst* bc;
     // slot `slot` of poly k (even: a, odd: b) of item k / 2
     __device__ void at(int k, int slot, int basis, const u64*& dig, const u64*& key_p) const {
-        const int item = k >> 1;
-        dig = digits + item * dstride + (long long)slot * N;
+        const int item = k >> 1, j = first + item;
+        dig = digits + (j - per_period.div(j) * period) * dstride + (long long)slot * N;
         key_p = key[item] + ((long long)((k & 1) ? 0 : nq + K) + basis) * N;
     }
 };
@@ -96,7 +98,10 @@ struct MacPJob {
 // forward NTT last (row) pass over the Q slots: out = combine(old, key
 // product + b term) - NTT(contribution); old and the b term read from a zero
 // row where the mode assigns / there is no b term
-template <int PARTS>
+// MAPPED: items may store through an automorphism.  A form of its own: with the
+// map in every switch the 128 switches took 14.8 ms instead of 14.3 and the
+// Walsh pairs' relinearisations 40 us more.
+template <int PARTS, bool MAPPED>
 struct MdMacOutJob {
     KeyProductLists kp;
     const u64* tmp;                        // [npoly][L][N] NTT'd contributions
@@ -105,10 +110,13 @@ struct MdMacOutJob {
     const u64* add[2 * KS_MAX_ITEMS];      // the b term or the zero row
     long long old_step[2 * KS_MAX_ITEMS];  // limb step of old / add: N, or 0 for the zero row
     long long add_step[2 * KS_MAX_ITEMS];
-    int npoly;
+    u32 to[KS_MAX_ITEMS];                  // item's output map: inverse Galois element, or 0
+    int npoly, logN;
     FastDiv per_limb;  // npoly
     struct View {
         int basis;
+        u32 to;
+        int logN;
         const u64* src;
         u64* out;
         const u64* old;
@@ -120,20 +128,25 @@ struct MdMacOutJob {
         BasisConst b;
         __device__ u64 load(int i) const { return src[i]; }
         __device__ u64 pre(int i) const { return add_mod(old[i], add[i], b.q); }
+        // An automorphism permutes each row block of the evaluation order into
+        // one other block, so mapped stores still fill whole lines.
+        __device__ u32 place(int i) const { return MAPPED && to ? galois_index((u32)i, to, logN) : (u32)i; }
         __device__ void store_pre(int i, u64 v, u64 base) const {
             const u64 acc = add_mod(key_product<PARTS>(dig, dstep, key, kstep, i, b, mont), base, b.q);
-            out[i] = sub_mod(acc, v, b.q);
+            out[place(i)] = sub_mod(acc, v, b.q);
         }
         __device__ void store_fp(int i, double x, u64 base) const {
             // at most 3/4 q + 5.2q + q < 8q
             const double p = key_product_fp<PARTS>(dig, dstep, key, kstep, i, b, mont);
-            out[i] = FpMod{b.qd, b.inv_d}.canonical(p - x + fp_from_u64(base));
+            out[place(i)] = FpMod{b.qd, b.inv_d}.canonical(p - x + fp_from_u64(base));
         }
     };
     __device__ View view(int k) const {
         const int t = per_limb.div(k), poly = k - t * npoly;
         View v;
         v.basis = t;
+        v.to = to[poly >> 1];
+        v.logN = logN;
         v.src = tmp + ((long long)poly * kp.L + t) * kp.N;
         v.out = out[poly] + (long long)t * kp.N;
         v.old = old[poly] + (long long)t * old_step[poly];
@@ -148,16 +161,57 @@ struct MdMacOutJob {
     __device__ bool skip(int) const { return false; }
 };
 
+template <int PARTS, bool MAPPED>
+void moddown_mac_out(Context& c, int level, int n, const KsItem* items, const KeyProductLists& kp, u64* const* p,
+                     u64* T, hipStream_t s) {
+    const int L = level + 1, npoly = 2 * n;
+    const u64 N = c.N;
+    MdMacOutJob<PARTS, MAPPED> o{};
+    o.kp = kp;
+    o.tmp = T;
+    for (int i = 0; i < n; ++i) {
+        const KsItem& it = items[i];
+        if (it.galois && (it.a_mode == 0 || it.b_mode == 0)) throw Error(-1, "a mapped key switch assigns its outputs");
+        if (it.galois) {
+            // inverse modulo a power of two, by Newton's iteration
+            u64 x = it.galois;
+            for (int k = 0; k < 5; ++k) x *= 2 - it.galois * x;
+            o.to[i] = (u32)(x & (2 * N - 1));
+        }
+        // poly 2i: a, poly 2i+1: b
+        o.out[2 * i] = it.a_out;
+        o.out[2 * i + 1] = it.b_out;
+        o.old[2 * i] = it.a_mode == 0 ? it.a_out : c.d_zero;
+        o.old_step[2 * i] = it.a_mode == 0 ? (long long)N : 0;
+        o.old[2 * i + 1] = it.b_mode == 0 ? it.b_out : c.d_zero;
+        o.old_step[2 * i + 1] = it.b_mode == 0 ? (long long)N : 0;
+        o.add[2 * i] = c.d_zero;
+        o.add_step[2 * i] = 0;
+        o.add[2 * i + 1] = it.init_b ? it.init_b : c.d_zero;
+        o.add_step[2 * i + 1] = it.init_b ? (long long)N : 0;
+    }
+    o.npoly = npoly;
+    o.logN = c.logN;
+    o.per_limb = fast_div(npoly);
+    const long long probe = c.probe_open(s, npoly * L);
+    moddown_ext_cols(c, level, npoly, p, T, s);
+    launch_rows_w4<true>(c, o, npoly * L, s);
+    c.probe_close(probe, s);
+}
+
 template <int PARTS>
 void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,
-                   u64* T, bool montgomery, hipStream_t s) {
-    const int L = level + 1, K = c.np, npoly = 2 * n;
+                   u64* T, bool montgomery, hipStream_t s, int first, int period) {
+    const int K = c.np, npoly = 2 * n;
     const u64 N = c.N;
     KeyProductLists kp{};
     kp.digits = D;
     kp.dstride = dstride;
+    kp.first = first;
+    kp.period = period;
+    kp.per_period = fast_div(period);
     for (int i = 0; i < n; ++i) kp.key[i] = items[i].key;
-    kp.L = L;
+    kp.L = level + 1;
     kp.K = K;
     kp.nq = c.nq;
     kp.N = N;
@@ -179,40 +233,22 @@ void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64*
         moddown_p_cols(c, npoly, p, s);
         c.probe_close(probe, s);
     }
-    MdMacOutJob<PARTS> o{};
-    o.kp = kp;
-    o.tmp = T;
-    for (int i = 0; i < n; ++i) {
-        const KsItem& it = items[i];
-        // poly 2i: a, poly 2i+1: b
-        o.out[2 * i] = it.a_out;
-        o.out[2 * i + 1] = it.b_out;
-        o.old[2 * i] = it.a_mode == 0 ? it.a_out : c.d_zero;
-        o.old_step[2 * i] = it.a_mode == 0 ? (long long)N : 0;
-        o.old[2 * i + 1] = it.b_mode == 0 ? it.b_out : c.d_zero;
-        o.old_step[2 * i + 1] = it.b_mode == 0 ? (long long)N : 0;
-        o.add[2 * i] = c.d_zero;
-        o.add_step[2 * i] = 0;
-        o.add[2 * i + 1] = it.init_b ? it.init_b : c.d_zero;
-        o.add_step[2 * i + 1] = it.init_b ? (long long)N : 0;
-    }
-    o.npoly = npoly;
-    o.per_limb = fast_div(npoly);
-    const long long probe = c.probe_open(s, npoly * L);
-    moddown_ext_cols(c, level, npoly, p, T, s);
-    launch_rows_w4<true>(c, o, npoly * L, s);
-    c.probe_close(probe, s);
+    bool mapped = false;
+    for (int i = 0; i < n; ++i) mapped = mapped || items[i].galois != 0;
+    if (mapped) moddown_mac_out<PARTS, true>(c, level, n, items, kp, p, T, s);
+    else moddown_mac_out<PARTS, false>(c, level, n, items, kp, p, T, s);
 }
 
 void ks_moddown_mac(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,
-                    u64* T, bool montgomery, hipStream_t s) {
+                    u64* T, bool montgomery, hipStream_t s, int first, int period) {
+    if (period < 1) period = first + n;
     if (n < 1 || n > KS_MAX_ITEMS) throw Error(-1, "key switch batch size out of range");
     if (c.np > MAX_ALPHA) throw Error(-1, "more than 16 special moduli");
     const int parts = c.parts(level);
     switch (parts) {
-        case 1: moddown_mac_t<1>(c, level, n, items, D, dstride, AP, T, montgomery, s); break;
-        case 2: moddown_mac_t<2>(c, level, n, items, D, dstride, AP, T, montgomery, s); break;
-        case 3: moddown_mac_t<3>(c, level, n, items, D, dstride, AP, T, montgomery, s); break;
+        case 1: moddown_mac_t<1>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period); break;
+        case 2: moddown_mac_t<2>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period); break;
+        case 3: moddown_mac_t<3>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period); break;
         default: throw Error(-1, "folded key product takes at most 3 digits");
     }
 }
