@@ -71,8 +71,8 @@ int mi_memory_stats(mi_context* ctx, int64_t* stats);
 int mi_set_memory_limit(mi_context* ctx, int64_t bytes);
 /* Autotuned launch plan (no counterpart in the reference): at context
  * creation the library times the candidate configurations of its tunable
- * launches on the device (the NTT kernel variant per launch-size bucket of
- * 0-3, 4-15, 16-63, 64-255, 256-1023 and 1024+ limbs: 1 = one limb per
+ * launches on the device (the kernel variant of in-place NTTs per launch-size
+ * bucket of 0-3, 4-15, 16-63, 64-255, 256-1023 and 1024+ limbs: 1 = one limb per
  * workgroup, 2 = two limbs per workgroup, 3 = one limb with 32-bit LDS
  * exchanges; key switches per launch group, 8/16/32) and keeps the fastest,
  * cached per device and ring dimension in memory and in $MICKKS_TUNE_CACHE
