@@ -321,7 +321,10 @@ size_t ks_item_words(const Context& c, int level) {
 
 void keyswitch_items(Context& c, const KsItem* items, int n, bool montgomery, hipStream_t s) {
     if (n < 1 || n > KS_MAX_ITEMS) throw Error(-1, "key switch batch size out of range");
-    u64* ws = (u64*)c.workspace(s, sizeof(u64) * ks_item_words(c, items[0].level) * (size_t)n);
+    // A single switch (a relinearisation, say) sizes the workspace for a rotation
+    // at its level too: growing it later would stop the stream for a new allocation.
+    const size_t staging = n == 1 ? 2 * (size_t)(items[0].level + 1) * c.N : 0;
+    u64* ws = (u64*)c.workspace(s, sizeof(u64) * (ks_item_words(c, items[0].level) * (size_t)n + staging));
     keyswitch_items_with(c, items, n, montgomery, ws, s);
 }
 
