@@ -525,6 +525,24 @@ __global__ void __launch_bounds__(KS_THREADS) k_automorphism_items(AutoItemsArgs
     dst[i] = src[sidx];
 }
 
+// Whether an output pair of hoisted rotations overlaps the digits or a key.
+static bool outputs_overlap_reads(const Context& c, int level, const u64* digits, long long dstride, int period, int n,
+                                  const u64* const* keys, u64* const* b_out, u64* const* a_out) {
+    const long long N = (long long)c.N, W = (level + 1) * N, parts = c.parts(level);
+    const long long digit_words = (period - 1) * dstride + parts * (level + 1 + c.np) * N;
+    const long long key_words = parts * 2 * c.nb() * N;
+    std::vector<const u64*> ks(keys, keys + n);
+    std::sort(ks.begin(), ks.end());
+    ks.erase(std::unique(ks.begin(), ks.end()), ks.end());
+    for (int i = 0; i < n; ++i)
+        for (const u64* o : {(const u64*)b_out[i], (const u64*)a_out[i]}) {
+            if (overlaps(Span{o, o + W}, Span{digits, digits + digit_words})) return true;
+            const auto k = std::lower_bound(ks.begin(), ks.end(), o + W);  // the last key that starts below the output's end
+            if (k != ks.begin() && *(k - 1) + key_words > o) return true;
+        }
+    return false;
+}
+
 void rotate_hoisted_items(Context& c, int level, const u64* digits, long long dstride, int period,
                           const u64* const* b, int n, const u64* galois, const u64* const* keys, u64* const* b_out,
                           u64* const* a_out, bool montgomery, hipStream_t s) {
@@ -540,8 +558,12 @@ void rotate_hoisted_items(Context& c, int level, const u64* digits, long long ds
     const int per_block = (period + chunk - 1) / chunk;
     const int nblocks = (n + period - 1) / period;
     const bool fold = c.parts(level) <= 3 && c.fuse_mac;
-    // per rotation: P accumulators (a, b) | ModDown temp | switched pair (a, b; not folded)
-    const size_t ws_bytes = sizeof(u64) * (size_t)chunk * (2 * KN + (fold ? 2 : 4) * LN);
+    // Folded, the last pass stores through the rotation's map while other
+    // workgroups still read the digits and keys: outputs on their memory (an
+    // output may take a buffer that the chunk no longer needs) go through staging.
+    const bool mapped = fold && !outputs_overlap_reads(c, level, digits, dstride, period, n, keys, b_out, a_out);
+    // per rotation: P accumulators (a, b) | ModDown temp | switched pair (a, b; not mapped)
+    const size_t ws_bytes = sizeof(u64) * (size_t)chunk * (2 * KN + (mapped ? 2 : 4) * LN);
     over_streams(c, s, nblocks * per_block, ws_bytes, [&](hipStream_t st, u64* ws, int ci) {
         const int blk = ci / per_block, cb = ci - blk * per_block;
         const int i0 = blk * period + cb * chunk;
@@ -552,18 +574,22 @@ void rotate_hoisted_items(Context& c, int level, const u64* digits, long long ds
         u64* SW = Tm + chunk * 2 * LN;
         const u64* dig = digits + (long long)(cb * chunk) * dstride;
         // key products of the hoisted digits, b added in the Q limbs
-        // (ckks_hybrid_key_switch_hoisted_inplace with b Add, a Assign): folded,
+        // (ckks_hybrid_key_switch_hoisted_inplace with b Add, a Assign): mapped,
         // the last pass stores through the rotation's map; else into staging
         // pairs, permuted by a pass of their own
         if (fold) {
             KsItem items[KS_MAX_ITEMS];
-            for (int it = 0; it < m; ++it)
+            for (int it = 0; it < m; ++it) {
                 items[it] = KsItem{nullptr, keys[i0 + it], b_out[i0 + it], a_out[i0 + it], level, 1, 1, b[i0 + it],
                                    galois[i0 + it] % (2 * N)};
+                if (mapped) continue;
+                items[it].a_out = SW + it * 2 * LN;
+                items[it].b_out = SW + it * 2 * LN + LN;
+                items[it].galois = 0;
+            }
             ks_moddown_mac(c, level, m, items, dig, dstride, AP, Tm, montgomery, st);
-            return;
-        }
-        {
+            if (mapped) return;
+        } else {
             MacArgs ma = mac_args(c, level, dig, keys[i0], montgomery);
             ma.items = m;
             ma.digits_stride = dstride;

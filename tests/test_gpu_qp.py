@@ -170,6 +170,35 @@ def test_hoisted_and_qp_switches_match_oracle(N, nq, np_, dnum, mont):
         assert np.array_equal(M.from_dev(dx)[: L * N], octx.moddown_qp_to_q(level, x)), level
 
 
+@pytest.mark.parametrize("fuse", ["1", "0"])
+@pytest.mark.parametrize("level,where", [(7, "digits"), (4, "digits"), (1, "digits"), (7, "key")])
+def test_rotate_hoisted_batch_into_what_it_reads(level, where, fuse, monkeypatch):
+    """Outputs in the digits' own memory, or in the key of another rotation of
+    the chunk: both are read to the end before the outputs are written."""
+    monkeypatch.setenv("MICKKS_FUSE_MAC", fuse)
+    M, ctx, octx, q, p, rng = _setup(1 << 13, 9, 3, 3, seed=31)
+    N, W = 1 << 13, (level + 1) * (1 << 13)
+    words = ctx.parts(level) * ctx.qp_limbs(level) * N
+    host_keys = [_key(rng, q, p, N, octx.parts(len(q) - 1)) for _ in range(2)]
+    keys = [M.to_dev(k) for k in host_keys]
+    a, b = M.to_dev(rand_residues(rng, q[:level + 1], N)), M.to_dev(rand_residues(rng, q[:level + 1], N))
+    gal = [O.galois_rotation(N, r) for r in (1, 5)]
+    dig = _zeros(M, words)
+    ctx.hoist(level, a, dig)
+    want = [(_zeros(M, W), _zeros(M, W)) for _ in gal]
+    ctx.rotate_hoisted_batch(level, dig, b, gal, keys, want)
+    if where == "digits":
+        flat = M.to_dev(np.zeros(max(words, 4 * W), np.uint64))
+        ctx.hoist(level, a, flat)
+        outs = [(flat[:W], flat[W:2 * W]), (flat[2 * W:3 * W], flat[3 * W:4 * W])]
+        dig = flat
+    else:
+        outs = [(keys[1][:W], _zeros(M, W)), (_zeros(M, W), _zeros(M, W))]
+    ctx.rotate_hoisted_batch(level, dig, b, gal, keys, outs)
+    for (wb, wa), (ob, oa) in zip(want, outs):
+        assert np.array_equal(M.from_dev(wb), M.from_dev(ob)) and np.array_equal(M.from_dev(wa), M.from_dev(oa))
+
+
 def test_rotate_hoisted_batch_matches_single_rotations_and_reference():
     """mi_rotate_hoisted_batch equals one mi_keyswitch_hoisted (b Add, a
     Assign, galois) per rotation, bit for bit, for 37 rotations (more than
