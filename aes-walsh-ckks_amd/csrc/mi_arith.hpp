@@ -145,9 +145,10 @@ struct FpMod {
         const double k = __builtin_rint(x * wq);
         return __builtin_fma(-k, q, h) + l;
     }
-    // x y mod q for two variables: the quotient estimate is off by at most
-    // 1/2 + |x y / q| 2^-52, so the result is at most 3/4 q for canonical
-    // operands and 9/2 q for operands up to 4q.
+    // x y mod q for two variables: the quotient estimate takes three roundings
+    // (x y, 1/q and their product) before rint, so it is off by at most 1/2 +
+    // 3 |x y / q| 2^-53 and the result at most 7/8 q for canonical operands, 2q
+    // if one of them is below 4q and 13/2 q if both are.
     __device__ __forceinline__ double mulq(double x, double y) const {
         const double h = x * y, l = __builtin_fma(x, y, -h);
         const double k = __builtin_rint(h * qinv);

@@ -223,7 +223,7 @@ __global__ void __launch_bounds__(KS_THREADS) k_mac(MacArgs a) {
     const long long dstep = (long long)slots * N, kstep = 2LL * key_limbs * N, to_a = (long long)key_limbs * N;
     // Operands are residues below 4q.
     if (b.fp) {  // uniform over the block
-        // each product at most 9/2 q (FpMod::mulq), centred; 16 of them stay at 8q
+        // each product at most 13/2 q (FpMod::mulq), centred; 16 of them stay at 8q
         const FpMod m{b.qd, b.inv_d};
         double sb = 0.0, sa = 0.0;
         for (int d = 0; d < a.parts; ++d) {

@@ -166,8 +166,8 @@ __device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisCon
                 bw[t] = slot < a.L ? a.in_b[item[t]][o + src] : 0;
                 xa[t] = xb[t] = 0.0;
             }
-            // digits canonical, keys below 4q: each product at most 3/2 q, the
-            // sum of up to five below 8q
+            // digits canonical, keys below 4q: each product at most 2q; three of
+            // them (6q) between two reductions
             if constexpr (PARTS > 0) {
                 u64 kw[PARTS][2], xw[PARTS][IT];
 #pragma unroll
@@ -184,6 +184,10 @@ __device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisCon
                         const double x = fp_from_u64(xw[e][t]);
                         xb[t] += m.mulq(x, fp_from_u64(kw[e][0]));
                         xa[t] += m.mulq(x, fp_from_u64(kw[e][1]));
+                        if (e == 2 && PARTS > 3) {
+                            xb[t] = m.centred(xb[t]);
+                            xa[t] = m.centred(xa[t]);
+                        }
                     }
             } else {
                 for (int e = 0; e < a.parts; ++e) {
@@ -201,13 +205,15 @@ __device__ __forceinline__ void lt_fused_fp(const LtFusedArgs& a, const BasisCon
                 if (a.mont) {
                     xb[t] = m.mul(xb[t], b.rinv_fp, b.rinv_fpq);
                     xa[t] = m.mul(xa[t], b.rinv_fp, b.rinv_fpq);
+                } else if (PARTS == 0) {
+                    xb[t] = m.centred(xb[t]);  // 16 digits reach 8q: no room for b
                 }
                 xb[t] = m.centred(xb[t] + fp_from_u64(bw[t]));
                 xa[t] = m.centred(xa[t]);
             }
         }
-        // |x| < q, diagonals below 4q: products at most 3/2 q; four of them
-        // between two reductions
+        // |x| < q (the input) or q/2 (the others), diagonals below 4q: products
+        // at most 2q or 5/4 q; four of them between two reductions, below 6q
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
             const double d = fp_from_u64(dw[g]);

@@ -30,7 +30,7 @@ __device__ __forceinline__ u64 key_product(const u64* dig, long long dstep, cons
     return mont ? redc128(s.lo, s.hi, b.q, b.qninv) : barrett128(s.lo, s.hi, b.q, b.mu_lo, b.mu_hi);
 }
 // The same as an integer-valued double of magnitude below 3/4 q (Montgomery
-// keys; else 9/4 q for canonical operands): moduli below 2^50.
+// keys; else q/2): moduli below 2^50.
 template <int PARTS>
 __device__ __forceinline__ double key_product_fp(const u64* dig, long long dstep, const u64* key, long long kstep,
                                                  int i, const BasisConst& b, int mont) {

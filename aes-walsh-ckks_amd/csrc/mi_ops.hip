@@ -390,7 +390,7 @@ struct RescaleOutJob {
         __device__ void store_pre(int i, u64 v, u64 num) const { x[i] = shoup(sub_mod(num, v, q), ip, ips, q); }
         __device__ void store_fp(int i, double v, u64 num) const {
             const FpMod m{qd, qinv};
-            const double w = fp_from_u64(ip);  // below q: the quotient is off by at most 1/2 + 6.2/4
+            const double w = fp_from_u64(ip);  // below q: the quotient is off by at most 1/2 + 6.2 * 3/8
             x[i] = m.canonical(m.mul(fp_from_u64(num) - v, w, w * qinv));
         }
     };

@@ -112,3 +112,50 @@ def test_walsh_sum_at_the_line_of_exact_doubles(bits, over, mont):
                           pt_montgomery=mont)
     assert all(np.array_equal(M.from_dev(a), o) for a, o in zip(acc, acc_o))
     assert all(np.array_equal(M.from_dev(r), o) for r, o in zip(raw, raw_o))
+
+
+# A prime below 2^50 whose rounded inverse is a little below 1/q by almost half
+# a unit in the last place, a residue x and a word y in [3q, 4q) for which the
+# products of the double path leave x y - k q = 1.4956 q, odd: five of them and
+# q - 1 are an odd number above 2^53.
+WORST_Q, WORST_X, WORST_Y = 1125899894996993, 1122752751754747, 4501000844983853
+
+
+@pytest.mark.parametrize("mont", [True, False])
+@pytest.mark.parametrize("keys", ["largest", "worst"])
+@pytest.mark.parametrize("parts", [1, 3, 4, 5, 6])
+def test_fused_baby_steps_at_their_largest(parts, keys, mont):
+    """QP linear transforms whose key products are the largest that the double
+    path meets: digits of q - 1 (a polynomial that is a small negative constant
+    is one in every digit) against keys of 4q - 1, and the digits and keys above,
+    whose sum over five digits is not a double.  Diagonals of 4q - 1, b of q - 1,
+    against the oracle on the reduced values."""
+    M = product()
+    N = 1 << 11
+    p, q = O.find_primes([50], [50] * 5, N)
+    q = [WORST_Q] + [int(v) for v in q]
+    p = [int(v) for v in p]
+    assert len(set(q + p)) == 7 and (WORST_Q - 1) % (2 * N) == 0
+    ctx, octx = M.Context(N, q, p, 6), O.Ctx(N, q, p, 6)
+    level = parts - 1
+    assert ctx.parts(level) == parts
+    minus = 1 if keys == "largest" else WORST_Q - WORST_X
+    full = lambda moduli, value: np.concatenate([np.full(N, value(int(m)), np.uint64) for m in moduli])  # noqa: E731
+    Q, basis, T = q[: level + 1], q + p, q[: level + 1] + p
+    a, b = full(Q, lambda m: m - minus), full(Q, lambda m: m - 1)
+    raw = full(basis, lambda m: WORST_Y if keys == "worst" and m == WORST_Q else 4 * m - 1)
+    raw = np.concatenate([raw] * (2 * octx.parts(len(q) - 1)))
+    mods = np.repeat(np.array(basis, np.uint64), N)
+    key = raw % np.concatenate([mods] * (2 * octx.parts(len(q) - 1)))
+    index = [0, 1, 2, 3, 5, 6]
+    lifted = full(T, lambda m: 4 * m - 1)
+    diags = [lifted % np.repeat(np.array(T, np.uint64), N)] * len(index)
+    rots = [1, 2, 3, 4]
+    wa, wb = octx.lt_stage_qp(level, a, b, index, np.concatenate(diags), 4, {r: key for r in rots}, montgomery=mont)
+    dkey, ddiag = M.to_dev(raw), M.to_dev(lifted)
+    for count in (1, 3):
+        outs = [(M.to_dev(np.zeros(len(a), np.uint64)), M.to_dev(np.zeros(len(a), np.uint64))) for _ in range(count)]
+        ctx.linear_transform_qp_batch(level, [(M.to_dev(a), M.to_dev(b))] * count, index, [ddiag] * len(index), 4,
+                                      {r: dkey for r in rots}, outs, montgomery=mont)
+        for oa, ob in outs:
+            assert np.array_equal(M.from_dev(oa), wa) and np.array_equal(M.from_dev(ob), wb), count
