@@ -171,6 +171,17 @@ void* Context::workspace(hipStream_t s, size_t bytes) {
     return w.ptr;
 }
 
+void* Context::workspace_up_to(hipStream_t s, size_t want, size_t need, bool* whole) {
+    *whole = true;
+    if (want > need) try {
+            return workspace(s, want);
+        } catch (const Error&) {
+            (void)hipGetLastError();
+            *whole = false;
+        }
+    return workspace(s, need);
+}
+
 int Context::ntt_variant(int count) const {
     if (ntt_forced) return ntt_forced;
     return tune.ntt_variant[tune_bucket(count)];

@@ -180,6 +180,9 @@ struct Context {
         return pp < dnum ? pp : dnum;
     }
     void* workspace(hipStream_t s, size_t bytes);
+    // `want` bytes, or at least `need` where those cannot be had (device memory, or a
+    // capture, in which the buffer cannot grow); *whole says which.
+    void* workspace_up_to(hipStream_t s, size_t want, size_t need, bool* whole);
     const std::vector<hipStream_t>& side_streams();
     void* pool_alloc(size_t bytes);
     void pool_release(void* p);

@@ -324,7 +324,9 @@ void keyswitch_items(Context& c, const KsItem* items, int n, bool montgomery, hi
     // A single switch (a relinearisation, say) sizes the workspace for a rotation
     // at its level too: growing it later would stop the stream for a new allocation.
     const size_t staging = n == 1 ? 2 * (size_t)(items[0].level + 1) * c.N : 0;
-    u64* ws = (u64*)c.workspace(s, sizeof(u64) * (ks_item_words(c, items[0].level) * (size_t)n + staging));
+    const size_t need = sizeof(u64) * ks_item_words(c, items[0].level) * (size_t)n;
+    bool whole;
+    u64* ws = (u64*)c.workspace_up_to(s, need + sizeof(u64) * staging, need, &whole);
     keyswitch_items_with(c, items, n, montgomery, ws, s);
 }
 

@@ -657,13 +657,26 @@ void linear_transform_q_batch(Context& c, const LtStage& st, int n, const u64* c
     int chunk = (int)std::min<long long>(KS_MAX_ITEMS, std::max<long long>(1, budget_words / item_words));
     chunk = std::min(chunk, n);
     // Folded, the baby steps of all ciphertexts are one batch and so are the
-    // giant steps' switches, KS_MAX_ITEMS at a time: a few ciphertexts' single
-    // steps leave most of the chip idle.
-    const bool fold = parts <= 3 && c.fuse_mac;
-    const int ck = fold ? (int)std::min<long long>(KS_MAX_ITEMS, (long long)chunk * std::max(1, std::max(nbaby, ngp)))
-                        : chunk;
+    // giant steps' switches, ck (step, ciphertext) pairs at a time: a few
+    // ciphertexts' single steps leave most of the chip idle.  Each pair takes
+    // step_words of scratch, so ck ends where a pass over its two polynomials
+    // has 2^25 words (8192 workgroups, 32 per CU) and where the budget does:
+    // 16 pairs of 13 limbs at N = 2^15 (3328 workgroups) took 5 % longer than
+    // 32, 8 pairs of 30 limbs at N = 2^16 (7680) 1 %, and 32 of those would
+    // hold 4.9 GB.
     const long long step_words = dw + LN + 2 * KN + 2 * LN + 2 * LN;  // digits | C | P accumulators | temp | switched
-    u64* ws = (u64*)c.workspace(s, sizeof(u64) * (size_t)(step_words * ck + (item_words - step_words) * chunk));
+    const bool fold = parts <= 3 && c.fuse_mac;
+    int ck = chunk;
+    if (fold) {
+        const long long pairs = (long long)chunk * std::max(1, std::max(nbaby, ngp));
+        const long long fill = ((1LL << 25) + 2 * LN - 1) / (2 * LN);
+        const long long fit = chunk + std::max(0LL, budget_words - item_words * chunk) / step_words;
+        ck = std::max(chunk, (int)std::min({(long long)KS_MAX_ITEMS, pairs, fill, fit}));
+    }
+    auto bytes = [&](int k) { return sizeof(u64) * (size_t)(step_words * k + (item_words - step_words) * chunk); };
+    bool whole = true;
+    u64* ws = (u64*)c.workspace_up_to(s, bytes(ck), bytes(chunk), &whole);
+    if (!whole) ck = chunk;
 
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int m = std::min(chunk, n - i0);

@@ -53,3 +53,73 @@ def test_stage_batches_match_the_oracle(evaluator, dnum, count, bs, index, monke
         for (a, b), (oa, ob) in zip(cts[:2], outs[:2]):
             wa, wb = octx.lt_stage_qp(level, a, b, index, np.concatenate(diags), bs, keys)
             assert np.array_equal(M.from_dev(oa), wa) and np.array_equal(M.from_dev(ob), wb)
+
+
+def _sequential(M, N, q, p, dnum, monkeypatch):
+    """A context that runs the Q evaluator's steps one after the other."""
+    monkeypatch.setenv("MICKKS_FUSE_MAC", "0")
+    ctx = M.Context(N, q, p, dnum)
+    monkeypatch.delenv("MICKKS_FUSE_MAC")
+    return ctx
+
+
+def test_one_ciphertext_keeps_its_scratch_small(monkeypatch):
+    """31 baby steps of one ciphertext at N = 2^16, 30 + 10 limbs: the steps run
+    in batches of nine pairs (2^25 words of two polynomials), not of 31 with
+    152 MB of scratch each; the result is the sequential form's."""
+    M = product()
+    N, level, bs = 1 << 16, 29, 32
+    p, q = O.find_primes([50] * 10, [50] * 30, N)
+    ctx = M.Context(N, q, p, 3)
+    rng = np.random.default_rng(5)
+    key = np.tile(rand_residues(rng, list(q) + list(p), N), 2 * ctx.parts(level))
+    ct, diag = [rand_residues(rng, q, N) for _ in range(2)], M.to_dev(rand_residues(rng, q, N))
+    dkey, index = M.to_dev(key), list(range(bs))
+    results = []
+    for c in (ctx, _sequential(M, N, q, p, 3, monkeypatch)):
+        out = [M.to_dev(np.zeros((level + 1) * N, np.uint64)) for _ in range(2)]
+        before = c.device_bytes()
+        c.linear_transform_q(level, M.to_dev(ct[0]), M.to_dev(ct[1]), index, [diag] * bs, bs,
+                             {r: dkey for r in range(1, bs)}, out[0], out[1])
+        results.append([M.from_dev(o) for o in out])
+        if c is ctx:
+            LN, pair = 30 * N, (3 * 40 + 30 + 20 + 120) * N
+            babies = 2 * (bs - 1) * LN
+            assert c.device_bytes() - before <= 8 * (9 * pair + babies + 2 * LN)
+    assert all(np.array_equal(x, y) for x, y in zip(*results))
+
+
+def test_steps_fit_the_workspace_of_a_capture(monkeypatch):
+    """A captured transform whose stream holds enough for one ciphertext's steps
+    one at a time, but not for a batch of them, runs them one at a time."""
+    import torch
+    M = product()
+    N, level, bs = 1 << 12, 5, 13
+    p, q = O.find_primes([50] * 3, [50] * 6, N)
+    ctx = M.Context(N, q, p, 3)
+    rng = np.random.default_rng(6)
+    key = M.to_dev(np.concatenate([rand_residues(rng, list(q) + list(p), N) for _ in range(6)]))
+    a, b, diag = (M.to_dev(rand_residues(rng, q, N)) for _ in range(3))
+    new = lambda: M.to_dev(np.zeros(6 * N, np.uint64))  # noqa: E731
+    out, want, st = [new(), new()], [new(), new()], torch.cuda.Stream()
+    args = (list(range(bs)), [diag] * bs, bs, {r: key for r in range(1, bs)})
+    _sequential(M, N, q, p, 3, monkeypatch).linear_transform_q(level, a, b, *args, want[0], want[1])
+    torch.cuda.synchronize()
+    # eight key switches at once: 408 limbs of workspace, where the transform's
+    # steps take 219 one at a time and 900 as one batch
+    ctx.keyswitch_batch([(level, a, key, new(), new(), 0, 1) for _ in range(8)], stream=st)
+    st.synchronize()
+    ctx.graph_begin(st)
+    ctx.linear_transform_q(level, a, b, *args, out[0], out[1], stream=st)
+    graph = ctx.graph_end(st)
+    try:
+        for r in range(3):
+            out[0].zero_(), out[1].zero_()
+            torch.cuda.synchronize()
+            graph.launch(st)
+            st.synchronize()
+            assert all(np.array_equal(M.from_dev(o), M.from_dev(w)) for o, w in zip(out, want)), r
+            ctx.keyswitch_batch([(level, a, key, new(), new(), 0, 1)], stream=st)
+            st.synchronize()
+    finally:
+        graph.destroy()
