@@ -248,7 +248,7 @@ Context* context_create(u64 N, const u64* q, int nq, const u64* p, int np, int d
 void set_decoding_tables(Context& c, const double* twiddles, const u64* perm);
 void decode_batch(Context& c, int count, const u64* const* coeffs, int limbs, const u64* scale_mant,
                   const int* scale_exp, bool coeff_domain, double* out, hipStream_t s);
-// Installs the tuned plan for the context's device and ring dimension,
+// Installs the tuned plan for the context's device, arithmetics and ring dimension,
 // measuring it first when neither this process nor the cache file has it.
 void tune_context(Context& c);
 int tune_bucket(int count);

@@ -1,12 +1,15 @@
 // Autotuner for the launch shapes that have more than one configuration:
-//   * the in-place NTT passes' limbs per workgroup (1 or 2), per ring dimension
-//     and launch size (six buckets of limbs per launch);
-//   * the key-switch group size (items per launch sequence: 8, 16 or 32),
-//     per ring dimension.
+//   * the in-place NTT passes' limbs per workgroup (1 or 2), per launch size
+//     (six buckets of limbs per launch);
+//   * the key-switch group size (items per launch sequence: 8, 16 or 32).
 // Each candidate is timed with HIP events on a scratch batch (the timing of
-// these kernels does not depend on the residues), the fastest kept.  Results
-// are cached per device (GPU architecture and compute-unit count) and ring
-// dimension, in memory for the process and in a text file
+// these kernels does not depend on the residues), the fastest kept.  Which is
+// depends on the arithmetics that the moduli take: variant 1 has a kernel for
+// each, variant 2 runs two integer limbs together but double ones in turn.
+// Results are cached per device (GPU architecture and compute-unit count),
+// arithmetic (all integer, all double, both) and ring dimension, in memory for
+// the process and, with the version of the kernels they were timed on, in a
+// text file
 // ($MICKKS_TUNE_CACHE, else $HOME/.cache/mickks/tune.txt) across processes.
 // MICKKS_TUNE=0 skips tuning (the defaults: 1 limb per workgroup, groups of
 // 32).  Every configuration computes the same residues: the choice changes
@@ -27,7 +30,10 @@ namespace mi {
 namespace {
 
 std::mutex g_mu;
-std::map<std::string, TunePlan> g_plans;  // "<arch> <cus> <logN>" -> plan
+std::map<std::string, TunePlan> g_plans;  // "<arch> <cus> <arithmetic> <logN>" -> plan
+// First field of a cache line; goes up when the tuned kernels change, so that
+// plans timed on earlier ones are not used.
+constexpr const char* kCacheVersion = "v2";
 bool g_loaded = false;
 
 std::string cache_path() {
@@ -35,6 +41,10 @@ std::string cache_path() {
     const char* h = std::getenv("HOME");
     if (!h) return "";
     return std::string(h) + "/.cache/mickks/tune.txt";
+}
+
+std::string plan_key(const std::string& arch, int cus, const std::string& kind, int logN) {
+    return arch + " " + std::to_string(cus) + " " + kind + " " + std::to_string(logN);
 }
 
 void load_cache() {
@@ -46,17 +56,17 @@ void load_cache() {
     std::string line;
     while (std::getline(f, line)) {
         std::istringstream in(line);
-        std::string arch;
+        std::string version, arch, kind;
         int cus, logN;
         TunePlan p;
-        if (!(in >> arch >> cus >> logN)) continue;
+        if (!(in >> version >> arch >> cus >> kind >> logN) || version != kCacheVersion) continue;
         bool ok = true;
         for (int b = 0; b < TUNE_BUCKETS; ++b) ok = ok && (in >> p.ntt_variant[b]) && p.ntt_variant[b] >= 1 && p.ntt_variant[b] <= NTT_VARIANTS;
         ok = ok && (in >> p.ks_group) && (p.ks_group == 8 || p.ks_group == 16 || p.ks_group == 32);
         if (ok) {
             p.tuned = true;
             p.from_cache = true;
-            g_plans[arch + " " + std::to_string(cus) + " " + std::to_string(logN)] = p;
+            g_plans[plan_key(arch, cus, kind, logN)] = p;
         }
     }
 }
@@ -74,7 +84,7 @@ void save_cache() {
     std::ofstream f(path, std::ios::trunc);
     if (!f) return;  // read-only home: the plans stay per process
     for (const auto& kv : g_plans) {
-        f << kv.first;
+        f << kCacheVersion << ' ' << kv.first;
         for (int b = 0; b < TUNE_BUCKETS; ++b) f << ' ' << kv.second.ntt_variant[b];
         f << ' ' << kv.second.ks_group << '\n';
     }
@@ -188,8 +198,11 @@ void tune_context(Context& c) {
         if (std::string(e) == "0") return;  // defaults
     hipDeviceProp_t prop;
     MI_HIP(hipGetDeviceProperties(&prop, c.device));
-    const std::string key = std::string(prop.gcnArchName).substr(0, std::string(prop.gcnArchName).find(':')) + " " +
-                            std::to_string(prop.multiProcessorCount) + " " + std::to_string(c.logN);
+    const std::string arch = prop.gcnArchName;
+    int fp = 0;
+    for (const BasisConst& b : c.h_bc) fp += b.fp;
+    const std::string key = plan_key(arch.substr(0, arch.find(':')), prop.multiProcessorCount,
+                                     fp == 0 ? "integer" : fp == c.nb() ? "double" : "both", c.logN);
     std::lock_guard<std::mutex> g(g_mu);
     load_cache();
     auto f = g_plans.find(key);

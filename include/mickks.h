@@ -75,8 +75,9 @@ int mi_set_memory_limit(mi_context* ctx, int64_t bytes);
  * bucket of 0-3, 4-15, 16-63, 64-255, 256-1023 and 1024+ limbs: 1 = one limb per
  * workgroup, 2 = two limbs per workgroup, 3 = one limb with 32-bit LDS
  * exchanges; key switches per launch group, 8/16/32) and keeps the fastest,
- * cached per device and ring dimension in memory and in $MICKKS_TUNE_CACHE
- * (else $HOME/.cache/mickks/tune.txt); MICKKS_TUNE=0 keeps the defaults and
+ * cached per device, arithmetic of the moduli (all below 2^50, none, or both)
+ * and ring dimension in memory and in $MICKKS_TUNE_CACHE (else
+ * $HOME/.cache/mickks/tune.txt); MICKKS_TUNE=0 keeps the defaults and
  * MICKKS_NTT_VARIANT=v forces one NTT variant.  Every plan computes the same
  * residues.  mi_tune_report writes the context's plan as a JSON object into
  * buf; mi_tune_set replaces it (six variants, each 1, 2 or 3, and a group

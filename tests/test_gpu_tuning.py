@@ -3,11 +3,15 @@ variants 1 = one limb per workgroup, 2 = two limbs per workgroup, 3 = one
 limb with 32-bit LDS exchanges, in every launch-size bucket; key-switch
 groups of 8, 16 and 32) gives the same residues as the oracle, and the
 context reports the plan it runs with."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 import oracle as O
-from helpers import product, rand_residues
+from helpers import ROOT, product, rand_residues
 
 pytestmark = pytest.mark.gpu
 
@@ -116,3 +120,38 @@ def test_folded_key_product_matches_the_oracle(fuse, mont, monkeypatch):
         db, da = M.to_dev(b), M.to_dev(a)
         ctx.keyswitch(level, M.to_dev(kt), dkey, db, da, bm, am, montgomery=mont)
         assert np.array_equal(M.from_dev(db), ob) and np.array_equal(M.from_dev(da), oa), (level, bm, am)
+
+
+_PLANS = """
+import sys
+sys.path[:0] = [{root!r} + "/tests", {root!r} + "/oracle"]
+import oracle as O
+from helpers import product
+M = product()
+for bits in ([60] * 4, [45] * 4, [60, 45, 60, 45]):
+    p, q = O.find_primes(bits[:1], bits, 1 << 12)
+    r = M.Context(1 << 12, q, p, 2).tune_report()
+    print("plan", r["device"].split()[2], r["from_cache"], *r["ntt_variant"], r["keyswitch_group"], flush=True)
+"""
+
+
+def test_plans_are_kept_per_arithmetic_and_kernel_version(tmp_path):
+    """A plan is measured for each kind of moduli (integers, doubles, both) of a
+    ring dimension, and lines of a cache file without the present version (an
+    earlier form, and an earlier version) are not used; a second process finds
+    all three plans."""
+    cache = tmp_path / "tune.txt"
+    kinds = ["integer", "double", "both"]
+    stale = ["gfx950 256 12 3 3 3 3 3 3 8"] + [f"v1 gfx950 256 {k} 12 3 3 3 3 3 3 8" for k in kinds]
+    cache.write_text("\n".join(stale) + "\n")
+
+    def plans():
+        env = {k: v for k, v in os.environ.items() if not k.startswith("MICKKS_")}
+        out = subprocess.run([sys.executable, "-c", _PLANS.format(root=ROOT)], capture_output=True, text=True,
+                             timeout=100, env=dict(env, MICKKS_TUNE_CACHE=str(cache)))
+        assert out.returncode == 0, out.stderr
+        return [ln.split()[1:] for ln in out.stdout.splitlines() if ln.startswith("plan ")]
+
+    first, second = plans(), plans()
+    assert [r[0] for r in first] == kinds and [r[1] for r in first] == ["False"] * 3
+    assert [r[1] for r in second] == ["True"] * 3 and [r[2:] for r in first] == [r[2:] for r in second]
