@@ -35,26 +35,34 @@ struct LiftJob {
         const u64* c0;
         u64* o;
         u64 q0, q, mu_hi;
-        double qd, qinv;
-        __device__ double load_fp(int i) const {
-            if (q0 >= (1ull << FP_BITS)) return fp_from_u64(load(i));  // uniform
-            const u64 v = c0[i];
-            const double x = v > (q0 >> 1) ? -fp_from_u64(q0 - v) : fp_from_u64(v);
-            return FpMod{qd, qinv}.centred(x);
-        }
-        __device__ u64 load(int i) const {
-            const u64 v = c0[i];
-            if (v > (q0 >> 1)) {
-                const u64 m = reduce64(q0 - v, q, mu_hi);
-                return m == 0 ? 0 : q - m;
+        static constexpr bool BLOCK = true;
+        // all loads before the choice on q_0
+        template <class BF, class AT>
+        __device__ __forceinline__ void load_block(const BF& bf, AT at, u64 (&x)[E]) const {
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = c0[at(j)];
+            if constexpr (std::is_same_v<BF, BfFp>) {
+                if (q0 < (1ull << FP_BITS)) {  // uniform
+#pragma unroll
+                    for (int j = 0; j < E; ++j) {
+                        const u64 v = x[j];
+                        x[j] = BfFp::u(bf.m.centred(v > (q0 >> 1) ? -fp_from_u64(q0 - v) : fp_from_u64(v)));
+                    }
+                    return;
+                }
             }
-            return reduce64(v, q, mu_hi);
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                const bool neg = x[j] > (q0 >> 1);
+                const u64 m = reduce64(neg ? q0 - x[j] : x[j], q, mu_hi);
+                x[j] = bf.in(neg && m ? q - m : m);
+            }
         }
         __device__ void store(int i, u64 v) const { o[i] = v; }
     };
     __device__ View view(int k) const {
         const BasisConst b = bc[k];
-        return View{k, coeff0, out + (long long)k * N, q0, b.q, b.mu_hi, b.qd, b.inv_d};
+        return View{k, coeff0, out + (long long)k * N, q0, b.q, b.mu_hi};
     }
     __device__ bool skip(int) const { return false; }
 };
@@ -101,7 +109,7 @@ struct LiftListJob {
     __device__ LiftJob::View view(int k) const {
         const int l = per_limb.div(k), it = k - l * n;
         const BasisConst b = bc[l];
-        return LiftJob::View{l, coeff0 + (long long)it * N, out[it] + (long long)l * N, q0, b.q, b.mu_hi, b.qd, b.inv_d};
+        return LiftJob::View{l, coeff0 + (long long)it * N, out[it] + (long long)l * N, q0, b.q, b.mu_hi};
     }
     __device__ bool skip(int) const { return false; }
 };

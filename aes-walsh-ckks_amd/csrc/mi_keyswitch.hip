@@ -26,7 +26,8 @@ namespace mi {
 
 // ---- inverse NTT of n key terms -> C (item-minor within a limb) ----
 // The first pass also copies each limb, as it is read, to its own place among
-// the digits.
+// the digits: all words loaded before the first is stored (a later load may
+// not pass a store that it might overlap, and each would wait for its own).
 struct CopyListJob {
     const u64* src[KS_MAX_ITEMS];
     u64* dst;
@@ -41,10 +42,16 @@ struct CopyListJob {
         const u64* s;
         u64* d;
         u64* own;
-        __device__ u64 load(int i) const {
-            const u64 v = s[i];
-            own[i] = v;
-            return v;
+        static constexpr bool BLOCK = true;
+        template <class BF, class AT>
+        __device__ __forceinline__ void load_block(const BF& bf, AT at, u64 (&x)[E]) const {
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = s[at(j)];
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                own[at(j)] = x[j];
+                x[j] = bf.in(x[j]);
+            }
         }
         __device__ void store(int i, u64 v) const { d[i] = v; }
     };

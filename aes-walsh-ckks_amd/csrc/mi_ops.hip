@@ -345,16 +345,25 @@ struct RescaleInJob {
         const u64* top;
         u64* out;
         u64 p, half, q, mu_hi;
-        double qd, qinv;
-        __device__ u64 shifted(int i) const {
-            const u64 s = top[i] + half;
-            return s >= p ? s - p : s;
-        }
-        __device__ u64 load(int i) const { return reduce64(shifted(i), q, mu_hi); }
-        __device__ double load_fp(int i) const {
-            const FpMod m{qd, qinv};
-            if (p < (1ull << FP_BITS)) return m.centred(fp_from_u64(shifted(i)));  // uniform
-            return fp_from_u64(load(i));
+        static constexpr bool BLOCK = true;
+        // The choice on p comes after all loads: made per word, each word waited
+        // for its own load (10.6 us instead of 8.0 at N = 2^14, 14 limbs).
+        template <class BF, class AT>
+        __device__ __forceinline__ void load_block(const BF& bf, AT at, u64 (&x)[E]) const {
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                const u64 s = top[at(j)] + half;
+                x[j] = s >= p ? s - p : s;
+            }
+            if constexpr (std::is_same_v<BF, BfFp>) {
+                if (p < (1ull << FP_BITS)) {  // uniform
+#pragma unroll
+                    for (int j = 0; j < E; ++j) x[j] = BfFp::u(bf.m.centred(fp_from_u64(x[j])));
+                    return;
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < E; ++j) x[j] = bf.in(reduce64(x[j], q, mu_hi));
         }
         __device__ void store(int i, u64 v) const { out[i] = v; }
     };
@@ -362,7 +371,7 @@ struct RescaleInJob {
         const int i = per_limb.div(k), poly = k - i * npolys;  // modulus-major
         const BasisConst b = bc[i];
         return View{i, polys[poly] + (long long)level * N, scratch + ((long long)poly * level + i) * N, p, half,
-                    b.q, b.mu_hi, b.qd, b.inv_d};
+                    b.q, b.mu_hi};
     }
     __device__ bool skip(int) const { return false; }
 };

@@ -159,3 +159,21 @@ def test_fused_baby_steps_at_their_largest(parts, keys, mont):
                                       {r: dkey for r in rots}, outs, montgomery=mont)
         for oa, ob in outs:
             assert np.array_equal(M.from_dev(oa), wa) and np.array_equal(M.from_dev(ob), wb), count
+
+
+@pytest.mark.parametrize("kind", ["random", "largest", "halves"])
+@pytest.mark.parametrize("first", [49, 50, 51, 60])
+def test_modraise_from_either_side(first, kind):
+    """The q_0 limb, below or above 2^50, centred and lifted to limbs of both
+    sides; values around q_0 / 2, where the sign changes, among them."""
+    M = product()
+    N = 1 << 11
+    p, q = O.find_primes([61], [first, 50, 51, 36, 61, 27], N)
+    ctx, octx = M.Context(N, q, p, 2), O.Ctx(N, q, p, 2)
+    coeff = _pattern(kind, np.random.default_rng(first), q[:1], N)
+    x = M.to_dev(coeff)
+    ctx.ntt_forward(x, 1, 1)
+    host = M.from_dev(x)
+    out = M.to_dev(np.zeros(len(q) * N, np.uint64))
+    ctx.modraise(len(q) - 1, x, out)
+    assert np.array_equal(M.from_dev(out), octx.modraise(len(q) - 1, host))
