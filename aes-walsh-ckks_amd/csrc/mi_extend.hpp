@@ -82,7 +82,9 @@ struct ExtView {
 
     // Any target: exact 128-bit sums of at most 16 products (< 2^128), the
     // constants in Montgomery form, one REDC.  Eight positions at a time: a
-    // sum takes four registers.
+    // sum takes four registers.  The next source's words and constants are
+    // loaded before this one's are used.  A word becomes a double for the
+    // estimate as hi 2^32 + lo in one rounding, which is (double)v.
     template <class AT>
     __device__ __forceinline__ void load_block(const BfInt& bf, AT at, u64 (&x)[E]) const {
         const u64 q = bf.q;
@@ -98,16 +100,26 @@ struct ExtView {
                 est[j] = 0.0;
                 acc[j] = U128{0, 0};
             }
+            u64 next[E / 2], next_c = terms[0].v[0];
+            double next_inv = src_inv[0];
+#pragma unroll
+            for (int j = 0; j < E / 2; ++j) next[j] = src[at(h + j)];
             for (int i = 0; i < ns; ++i) {
-                const u64* s = src + (long long)i * N;
-                const u64 c = terms[i].v[0];
-                const double inv = src_inv[i];
+                const int n = i + 1 < ns ? i + 1 : i;
+                const u64* s = src + (long long)n * N;
+                const u64 c = next_c;
+                const double inv = next_inv;
                 u64 v[E / 2];
 #pragma unroll
-                for (int j = 0; j < E / 2; ++j) v[j] = s[at(h + j)];
+                for (int j = 0; j < E / 2; ++j) v[j] = next[j];
+#pragma unroll
+                for (int j = 0; j < E / 2; ++j) next[j] = s[at(h + j)];
+                next_c = terms[n].v[0];
+                next_inv = src_inv[n];
 #pragma unroll
                 for (int j = 0; j < E / 2; ++j) {
-                    est[j] = __dadd_rn(est[j], __dmul_rn((double)v[j], inv));
+                    const double d = __builtin_fma((double)(u32)(v[j] >> 32), 0x1p32, (double)(u32)v[j]);
+                    est[j] = __dadd_rn(est[j], __dmul_rn(d, inv));
                     mac128(acc[j], v[j], c);
                 }
             }
@@ -135,8 +147,15 @@ struct ExtGrid {
     }
 };
 
-template <int LOGN, class Job>
-__global__ void __launch_bounds__(NTT_THREADS) k_ext_cols(NttTabs tb, Job job) {
+// A: Both, or Int for contexts whose moduli are all integers, held to three
+// waves per SIMD (164 registers).  Both takes 214 registers and two waves,
+// which suits the doubles (16 words in flight) but made integer key switches
+// slower than the separate extension had been.  N = 2^16, 30 + 10 limbs of 60
+// bits, us, separate / two waves / three: hoist 131 / 140 / 132, one key switch
+// 285 / 297 / 283, four 917 / 960 / 909, 32 7094 / 7230 / 6931.
+template <int LOGN, Arith A, class Job>
+__global__ void __launch_bounds__(NTT_THREADS) __attribute__((amdgpu_waves_per_eu(A == Arith::Int ? 3 : 1)))
+k_ext_cols(NttTabs tb, Job job) {
     constexpr int n1 = LOGN / 2, wpl = pass_wpl(n1, LOGN - n1);
     __shared__ u64 lds[NTT_LDS_WORDS];
     int tile, target;
@@ -146,8 +165,13 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ext_cols(NttTabs tb, Job job) {
     const ExtView v[1] = {job.view(source, target)};
     const bool live[1] = {true};
     const int w = tile - source * wpl;
-    if (tb.fp(v[0].basis)) pass_body<LOGN, true, false, 1, BfFp>(tb, v, live, w, lds);
-    else pass_body<LOGN, true, false, 1, BfInt>(tb, v, live, w, lds);
+    if constexpr (A == Arith::Both) {
+        if (tb.fp(v[0].basis)) {
+            pass_body<LOGN, true, false, 1, BfFp>(tb, v, live, w, lds);
+            return;
+        }
+    }
+    pass_body<LOGN, true, false, 1, BfInt>(tb, v, live, w, lds);
 }
 
 // Launches the fused extension and column pass of `sources` sources with up to
@@ -155,13 +179,16 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ext_cols(NttTabs tb, Job job) {
 template <class Job>
 void launch_ext_cols(const Context& c, Job job, int sources, int targets, hipStream_t s) {
     const NttTabs tb = tabs_of(c);
+    bool integer = true;
+    for (const BasisConst& b : c.h_bc) integer = integer && !b.fp;
 #define MI_EXT(LN)                                                                                    \
     {                                                                                                 \
         job.grid = ExtGrid{sources * pass_wpl(LN / 2, LN - LN / 2), targets, fast_div(targets)};      \
         const long long blocks = (long long)((job.grid.tiles + 7) / 8) * 8 * targets;                 \
         if (blocks >= (8LL << 20)) throw Error(-1, "base extension: too many limbs in one launch");   \
-        hipLaunchKernelGGL((k_ext_cols<LN, Job>), dim3((unsigned)blocks),                             \
-                           dim3(pass_threads(LN / 2, LN - LN / 2)), 0, s, tb, job);                   \
+        const dim3 g((unsigned)blocks), b(pass_threads(LN / 2, LN - LN / 2));                         \
+        if (integer) hipLaunchKernelGGL((k_ext_cols<LN, Arith::Int, Job>), g, b, 0, s, tb, job);      \
+        else hipLaunchKernelGGL((k_ext_cols<LN, Arith::Both, Job>), g, b, 0, s, tb, job);             \
     }
     MI_NTT_LOGN_CASES(MI_EXT)
 #undef MI_EXT
