@@ -13,7 +13,7 @@
 //                the QP basis, optionally through a Galois automorphism and
 //                with a b term added (:675-852, :373-416).
 //   ks_moddown   folded ModDown (:521-673, mi_moddown.hip), also with the key
-//                inner product folded in (mi_moddown_mac.hip).
+//                inner product folded in (mi_moddown_mac.hpp).
 // Reordering "+ acc" before "- NTT(contribution)" leaves every canonical
 // residue unchanged.
 #include "mi_extend.hpp"

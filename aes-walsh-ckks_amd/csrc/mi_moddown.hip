@@ -1,7 +1,7 @@
 // Folded ModDown of hybrid key switching (ckks_keyswitch.cpp:521-673): inverse
 // NTT of the P slots, contribution sum_j x_j p_j^-1 - alpha per Q limb (the
 // P-side HPS estimate computed once per coefficient), NTT, subtracted from Q.
-// The form with the key inner product folded in is mi_moddown_mac.hip.
+// The form with the key inner product folded in is mi_moddown_mac.hpp.
 #include "mi_extend.hpp"
 #include "mi_moddown.hpp"
 
@@ -139,6 +139,19 @@ void ks_moddown(Context& c, int level, u64* p0, u64* p1, const u64* base0, const
     const u64* b[2] = {base0, base1};
     u64* o[2] = {out0, out1};
     ks_moddown_n(c, level, p1 ? 2 : 1, p, b, o, T, s);
+}
+
+void ks_moddown_mac(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,
+                    u64* T, bool montgomery, hipStream_t s, int first, int period) {
+    if (period < 1) period = first + n;
+    if (n < 1 || n > KS_MAX_ITEMS) throw Error(-1, "key switch batch size out of range");
+    if (c.np > MAX_ALPHA) throw Error(-1, "more than 16 special moduli");
+    switch (c.parts(level)) {
+        case 1: return moddown_mac<1>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period);
+        case 2: return moddown_mac<2>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period);
+        case 3: return moddown_mac<3>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period);
+        default: throw Error(-1, "folded key product takes at most 3 digits");
+    }
 }
 
 }  // namespace mi

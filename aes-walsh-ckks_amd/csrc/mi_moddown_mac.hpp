@@ -1,3 +1,6 @@
+// ModDown with the key inner product folded in, for one number of digits: each
+// of mi_moddown_mac{1,2,3}.hip instantiates it, so that they compile side by side.
+#pragma once
 #include "mi_moddown.hpp"
 
 namespace mi {
@@ -12,11 +15,35 @@ namespace mi {
 // nor read back.  Each sum holds PARTS <= 3 canonical products (below q
 // 2^64: REDC's precondition), reduced once.
 // Operands are residues below 4q.
-template <int PARTS>
+//
+// What the keys and moduli are, the same for a whole launch.  Where it is known
+// at compile time a thread's 16 products are straight-line code whose loads go
+// out together; chosen in the code, each product is a branch of its own and
+// waits for its own loads.  One switch of a one-limb digit at N = 2^15 and
+// 61-bit special limbs (rotation at level 1): 86 -> 80 us, and before the
+// choice was made in the code 87.
+enum class KeyForm {
+    MontBelow61,  // Montgomery-form keys, integer moduli below 2^61
+    Mont,         // Montgomery-form keys
+    Normal,       // keys in normal form
+    Any,          // chosen per product
+};
+inline KeyForm key_form(const Context& c, bool montgomery) {
+    if (!montgomery) return KeyForm::Normal;
+    for (const BasisConst& b : c.h_bc)
+        if (b.q >= (1ull << 61)) return KeyForm::Mont;
+    return KeyForm::MontBelow61;
+}
+template <KeyForm F>
+__device__ __forceinline__ bool form_mont(int mont) {
+    return F == KeyForm::Any ? mont != 0 : F != KeyForm::Normal;
+}
+
+template <KeyForm F, int PARTS>
 __device__ __forceinline__ u64 key_product(const u64* dig, long long dstep, const u64* key, long long kstep, int i,
                                            const BasisConst& b, int mont) {
     U128 s{0, 0};
-    if (b.q < (1ull << 61)) {
+    if (F == KeyForm::MontBelow61 || (F == KeyForm::Any && b.q < (1ull << 61))) {
         // at most 3 products below 16 q^2: the sum fits in 128 bits and its
         // high word is reduced once, not every operand
 #pragma unroll
@@ -27,11 +54,11 @@ __device__ __forceinline__ u64 key_product(const u64* dig, long long dstep, cons
             mac128(s, reduce_4q(dig[d * dstep + i], b.q), reduce_4q(key[d * kstep + i], b.q));
     }
     s.hi = reduce64(s.hi, b.q, b.mu_hi);
-    return mont ? redc128(s.lo, s.hi, b.q, b.qninv) : barrett128(s.lo, s.hi, b.q, b.mu_lo, b.mu_hi);
+    return form_mont<F>(mont) ? redc128(s.lo, s.hi, b.q, b.qninv) : barrett128(s.lo, s.hi, b.q, b.mu_lo, b.mu_hi);
 }
 // The same as an integer-valued double of magnitude below 3/4 q (Montgomery
 // keys; else q/2): moduli below 2^50.
-template <int PARTS>
+template <KeyForm F, int PARTS>
 __device__ __forceinline__ double key_product_fp(const u64* dig, long long dstep, const u64* key, long long kstep,
                                                  int i, const BasisConst& b, int mont) {
     const FpMod m{b.qd, b.inv_d};
@@ -39,7 +66,7 @@ __device__ __forceinline__ double key_product_fp(const u64* dig, long long dstep
 #pragma unroll
     for (int d = 0; d < PARTS; ++d)
         s += m.centred(m.mulq(fp_from_u64(dig[d * dstep + i]), fp_from_u64(key[d * kstep + i])));
-    return mont ? m.mul(s, b.rinv_fp, b.rinv_fpq) : m.centred(s);
+    return form_mont<F>(mont) ? m.mul(s, b.rinv_fp, b.rinv_fpq) : m.centred(s);
 }
 
 struct KeyProductLists {
@@ -61,7 +88,7 @@ struct KeyProductLists {
 };
 
 // inverse NTT first (row) pass over the P slots: load = key product
-template <int PARTS>
+template <KeyForm F, int PARTS>
 struct MacPJob {
     KeyProductLists kp;
     u64* p[2 * KS_MAX_ITEMS];  // poly k's P accumulator (K limbs)
@@ -75,8 +102,8 @@ struct MacPJob {
         long long dstep, kstep;
         int mont;
         BasisConst b;
-        __device__ u64 load(int i) const { return key_product<PARTS>(dig, dstep, key, kstep, i, b, mont); }
-        __device__ double load_fp(int i) const { return key_product_fp<PARTS>(dig, dstep, key, kstep, i, b, mont); }
+        __device__ u64 load(int i) const { return key_product<F, PARTS>(dig, dstep, key, kstep, i, b, mont); }
+        __device__ double load_fp(int i) const { return key_product_fp<F, PARTS>(dig, dstep, key, kstep, i, b, mont); }
         __device__ void store(int i, u64 v) const { p[i] = v; }
     };
     __device__ View view(int k) const {
@@ -101,7 +128,7 @@ struct MacPJob {
 // MAPPED: items may store through an automorphism.  A form of its own: with the
 // map in every switch the 128 switches took 14.8 ms instead of 14.3 and the
 // Walsh pairs' relinearisations 40 us more.
-template <int PARTS, bool MAPPED>
+template <KeyForm F, int PARTS, bool MAPPED>
 struct MdMacOutJob {
     KeyProductLists kp;
     const u64* tmp;                        // [npoly][L][N] NTT'd contributions
@@ -132,12 +159,12 @@ struct MdMacOutJob {
         // one other block, so mapped stores still fill whole lines.
         __device__ u32 place(int i) const { return MAPPED && to ? galois_index((u32)i, to, logN) : (u32)i; }
         __device__ void store_pre(int i, u64 v, u64 base) const {
-            const u64 acc = add_mod(key_product<PARTS>(dig, dstep, key, kstep, i, b, mont), base, b.q);
+            const u64 acc = add_mod(key_product<F, PARTS>(dig, dstep, key, kstep, i, b, mont), base, b.q);
             out[place(i)] = sub_mod(acc, v, b.q);
         }
         __device__ void store_fp(int i, double x, u64 base) const {
             // at most 3/4 q + 5.2q + q < 8q
-            const double p = key_product_fp<PARTS>(dig, dstep, key, kstep, i, b, mont);
+            const double p = key_product_fp<F, PARTS>(dig, dstep, key, kstep, i, b, mont);
             out[place(i)] = FpMod{b.qd, b.inv_d}.canonical(p - x + fp_from_u64(base));
         }
     };
@@ -161,12 +188,12 @@ struct MdMacOutJob {
     __device__ bool skip(int) const { return false; }
 };
 
-template <int PARTS, bool MAPPED>
+template <KeyForm F, int PARTS, bool MAPPED>
 void moddown_mac_out(Context& c, int level, int n, const KsItem* items, const KeyProductLists& kp, u64* const* p,
                      u64* T, hipStream_t s) {
     const int L = level + 1, npoly = 2 * n;
     const u64 N = c.N;
-    MdMacOutJob<PARTS, MAPPED> o{};
+    MdMacOutJob<F, PARTS, MAPPED> o{};
     o.kp = kp;
     o.tmp = T;
     for (int i = 0; i < n; ++i) {
@@ -199,7 +226,7 @@ void moddown_mac_out(Context& c, int level, int n, const KsItem* items, const Ke
     c.probe_close(probe, s);
 }
 
-template <int PARTS>
+template <KeyForm F, int PARTS>
 void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,
                    u64* T, bool montgomery, hipStream_t s, int first, int period) {
     const int K = c.np, npoly = 2 * n;
@@ -223,7 +250,7 @@ void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64*
         p[2 * i + 1] = p[2 * i] + (size_t)K * N;
     }
     {
-        MacPJob<PARTS> in{};
+        MacPJob<F, PARTS> in{};
         in.kp = kp;
         for (int k = 0; k < npoly; ++k) in.p[k] = p[k];
         in.npoly = npoly;
@@ -235,21 +262,22 @@ void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64*
     }
     bool mapped = false;
     for (int i = 0; i < n; ++i) mapped = mapped || items[i].galois != 0;
-    if (mapped) moddown_mac_out<PARTS, true>(c, level, n, items, kp, p, T, s);
-    else moddown_mac_out<PARTS, false>(c, level, n, items, kp, p, T, s);
+    // Unmapped stores keep the choice: straight-line, the pass spills 36 to 44
+    // bytes at 128 registers, and 32 switches at N = 2^15 took 940 us, not 912.
+    if (mapped) moddown_mac_out<F, PARTS, true>(c, level, n, items, kp, p, T, s);
+    else moddown_mac_out<KeyForm::Any, PARTS, false>(c, level, n, items, kp, p, T, s);
 }
 
-void ks_moddown_mac(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP,
-                    u64* T, bool montgomery, hipStream_t s, int first, int period) {
-    if (period < 1) period = first + n;
-    if (n < 1 || n > KS_MAX_ITEMS) throw Error(-1, "key switch batch size out of range");
-    if (c.np > MAX_ALPHA) throw Error(-1, "more than 16 special moduli");
-    const int parts = c.parts(level);
-    switch (parts) {
-        case 1: moddown_mac_t<1>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period); break;
-        case 2: moddown_mac_t<2>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period); break;
-        case 3: moddown_mac_t<3>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period); break;
-        default: throw Error(-1, "folded key product takes at most 3 digits");
+template <int PARTS>
+void moddown_mac(Context& c, int level, int n, const KsItem* items, const u64* D, long long dstride, u64* AP, u64* T,
+                 bool montgomery, hipStream_t s, int first, int period) {
+    switch (key_form(c, montgomery)) {
+        case KeyForm::MontBelow61:
+            return moddown_mac_t<KeyForm::MontBelow61, PARTS>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period);
+        case KeyForm::Mont:
+            return moddown_mac_t<KeyForm::Mont, PARTS>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period);
+        default:
+            return moddown_mac_t<KeyForm::Normal, PARTS>(c, level, n, items, D, dstride, AP, T, montgomery, s, first, period);
     }
 }
 
