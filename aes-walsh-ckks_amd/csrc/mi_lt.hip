@@ -11,7 +11,8 @@
 //              (automorphism_qp_pair_accumulate, :373-416)
 //   result   = folded ModDown of out                  (moddown_qp_pair_to_q_eval, :641-718)
 // The baby steps exist only inside the fused inner-product kernel, which reads
-// the digits through each rotation's map.
+// the digits through each rotation's map (or, for many giant steps over
+// integers alone, are written out for k_lt_inner_all).
 #include "mi_ntt_kernels.hpp"
 
 #include <algorithm>
@@ -338,6 +339,23 @@ __global__ void __launch_bounds__(LT_THREADS) k_lt_fused(LtFusedArgs a) {
     }
 }
 
+// Contexts whose moduli are all integers: one ciphertext per workgroup, at most
+// NG giant steps.  Nothing is shared between ciphertexts here, and the forms
+// above run two or four of them one after the other.  8 baby steps, us, separate
+// baby steps / the forms above / this one: N = 2^15, 12 limbs of 60 bits, 6
+// digits, one giant step, 5 ciphertexts 641 / 937 / 529; 3 digits, 4 giant
+// steps, 16 ciphertexts 3464 / 3396 / 2904; N = 2^16, 30 limbs, 2 giant steps, 5
+// ciphertexts 3564 / 4572 / 3021.
+template <int NG>
+__global__ void __launch_bounds__(LT_THREADS) k_lt_int(LtFusedArgs a) {
+    const int tps = (1 << a.logN) / LT_THREADS;
+    const TileMap tm = map_tile(blockIdx.x, a.items, tps, a.L + a.K);
+    if (!tm.valid) return;
+    const long long i = (long long)tm.tile * LT_THREADS + threadIdx.x;
+    const BasisConst b = a.bc[tm.slot < a.L ? tm.slot : a.nq + (tm.slot - a.L)];
+    lt_fused_int<NG>(a, b, tm.item, 0, tm.slot, i);
+}
+
 static u64 powmod_u64(u64 a, u64 e, u64 m) {
     unsigned __int128 r = 1, x = a % m;
     while (e) {
@@ -484,6 +502,12 @@ void launch_inner(Context& c, const Compiled& k, const LtStage& st, int m, int K
     }
 }
 
+bool all_integer(const Context& c) {
+    for (const BasisConst& b : c.h_bc)
+        if (b.fp) return false;
+    return true;
+}
+
 // Baby steps and inner products of m items from their hoisted digits; outputs
 // as launch_inner.
 void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const u64* const* a, const u64* const* b,
@@ -491,11 +515,13 @@ void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const
                   long long outg_giant, long long outg_item, hipStream_t s) {
     const int L = st.level + 1, T = L + c.np;
     const int tps = (int)(c.N / LT_THREADS);
+    const bool integer = all_integer(c);
+    const size_t most = integer ? 8 : LT_NG;
     for (int s0 = 0; s0 < k.nslots; s0 += LT_NB) {
-        for (size_t gk0 = 0; gk0 < k.glist.size(); gk0 += LT_NG) {
+        for (size_t gk0 = 0; gk0 < k.glist.size(); gk0 += most) {
             LtFusedArgs f{};
             f.nb = std::min(LT_NB, k.nslots - s0);
-            f.ng = (int)std::min<size_t>(LT_NG, k.glist.size() - gk0);
+            f.ng = (int)std::min<size_t>(most, k.glist.size() - gk0);
             f.slot0 = s0;
             for (int r = 0; r < f.nb; ++r) {
                 f.key[r] = k.baby_key[s0 + r];
@@ -529,6 +555,13 @@ void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const
             f.mont = st.montgomery ? 1 : 0;
             f.pt_mont = st.pt_montgomery ? 1 : 0;
             f.bc = c.d_bc;
+            if (integer) {
+                const dim3 grid(tile_grid(m, tps, T));
+                if (f.ng <= 4) hipLaunchKernelGGL(k_lt_int<4>, grid, dim3(LT_THREADS), 0, s, f);
+                else hipLaunchKernelGGL(k_lt_int<8>, grid, dim3(LT_THREADS), 0, s, f);
+                MI_HIP(hipGetLastError());
+                continue;
+            }
             // the fewest giant steps that hold f.ng, and with them as many items
 #define MI_LT_FUSED(NG, IT, PARTS)                                                                     \
     hipLaunchKernelGGL((k_lt_fused<NG, IT, PARTS>), dim3(tile_grid((m + IT - 1) / IT, tps, T)),        \
@@ -570,9 +603,21 @@ void linear_transform_qp_batch(Context& c, const LtStage& st, int n, const u64* 
     const long long W = (long long)T * (long long)N, LN = (long long)L * (long long)N;
     const int nbaby = k.nslots - 1, ngp = k.ngp;
 
-    // per-item scratch: digits | C | out (a, b) | giant inners (a, b) | ModDown temp
-    const long long dw = (long long)parts * W;
-    const long long item_words = dw + LN + 2 * W + 2 * (long long)ngp * W + 2 * LN;
+    // Integers alone and more than 8 giant steps: the baby steps are written once
+    // and read by every giant step, unless the batch is small.  The fused kernel
+    // holds 8 steps' sums (16 took up to 7 % longer) and forms each baby step again
+    // for the next 8, which costs less than the extra launches up to some 850,000
+    // coefficients.  16 baby and 16 giant steps of 60 bits, us, separate / fused:
+    // N = 2^14, 10 limbs, 4 digits, 1, 5 and 16 ciphertexts (164 k, 819 k, 2.6 M)
+    // 1866 / 1562, 2709 / 2667, 5235 / 5522; N = 2^15, 14 limbs, 6 digits, 1, 2 and
+    // 5 (459 k, 918 k, 2.3 M) 2510 / 2473, 3247 / 3397, 5866 / 6375; N = 2^16, 40
+    // limbs, 3 digits, 1 (2.6 M) 6223 / 6509.
+    const bool separate = nbaby > 0 && k.glist.size() > 8 && n * W > 850000 && all_integer(c);
+
+    // per-item scratch: digits | C | babies (a, b; separate) | out (a, b) | giant
+    // inners (a, b) | ModDown temp
+    const long long dw = (long long)parts * W, bw = separate ? 2 * (long long)nbaby * W : 0;
+    const long long item_words = dw + LN + bw + 2 * W + 2 * (long long)ngp * W + 2 * LN;
     const long long budget_words = (32LL << 30) / 8;
     int chunk = (int)std::min<long long>(KS_MAX_ITEMS, std::max<long long>(1, budget_words / item_words));
     chunk = std::min(chunk, n);
@@ -582,7 +627,8 @@ void linear_transform_qp_batch(Context& c, const LtStage& st, int n, const u64* 
         const int m = std::min(chunk, n - i0);
         u64* D = ws;
         u64* C = D + m * dw;
-        u64* OAB = C + m * LN;
+        u64* BAB = C + m * LN;
+        u64* OAB = BAB + m * bw;
         u64* IAB = OAB + m * 2 * W;
         u64* Tm = IAB + m * 2 * (long long)ngp * W;
         auto inner = [&](int it, int gp) { return IAB + it * 2LL * ngp * W + (long long)gp * 2 * W; };
@@ -591,7 +637,27 @@ void linear_transform_qp_batch(Context& c, const LtStage& st, int n, const u64* 
         // one hoisted ModUp, then the baby steps (hoisted QP rotations, :675-852,
         // b added in the Q limbs) and every giant step's inner product
         if (nbaby > 0) ks_modup_n(c, level, m, a + i0, D, dw, C, s);
-        launch_fused(c, k, st, m, a + i0, b + i0, D, dw, OAB, 2 * W, IAB, 2 * W, 2LL * ngp * W, s);
+        if (separate) {
+            // the baby steps' key products are independent (each writes its
+            // own slot from the shared digits): spread over the streams
+            over_streams(c, s, nbaby, 0, [&](hipStream_t bst, u64*, int i) {
+                MacArgs ma = mac_args(c, level, D, k.baby_key[i + 1], st.montgomery != 0);
+                ma.items = m;
+                ma.digits_stride = dw;
+                ma.qp_out = 1;
+                ma.galois = k.baby_gal[i + 1];
+                for (int it = 0; it < m; ++it) {
+                    ma.key[it] = k.baby_key[i + 1];
+                    ma.a_out[it] = BAB + it * bw + i * 2LL * W;
+                    ma.b_out[it] = ma.a_out[it] + W;
+                    ma.init_b[it] = b[i0 + it];
+                }
+                ks_mac(c, ma, level, bst);
+            });
+            launch_inner(c, k, st, m, K, a + i0, b + i0, BAB, bw, 2 * W, OAB, 2 * W, IAB, 2 * W, 2LL * ngp * W, s);
+        } else {
+            launch_fused(c, k, st, m, a + i0, b + i0, D, dw, OAB, 2 * W, IAB, 2 * W, 2LL * ngp * W, s);
+        }
 
         // giant steps > 0: key term = ModDown(inner.a); QP switch; rotate-accumulate
         // with inner.b (automorphism_qp_pair_accumulate, :373-416)

@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
     (3, 1, 4, [0, 1, 3, 4, 6, 9]),
     (3, 7, 8, list(range(1, 8)) + [8, 11, 24, 40]),    # 49 baby pairs: 32 + 17; giants 0, 1, 3, 5
     (2, 5, 4, [5, 6, 9, 11, 14]),                      # no giant step 0
-    (6, 3, 4, [0, 2, 5, 7, 13]),                       # six digits: one after the other
+    (6, 3, 4, [0, 2, 5, 7, 13]),                       # five digits at this level
     (3, 3, 20, [0, 3, 17, 19, 20, 36, 39]),            # baby steps beyond 16
 ])
 def test_stage_batches_match_the_oracle(evaluator, dnum, count, bs, index, monkeypatch):
@@ -53,6 +53,49 @@ def test_stage_batches_match_the_oracle(evaluator, dnum, count, bs, index, monke
         for (a, b), (oa, ob) in zip(cts[:2], outs[:2]):
             wa, wb = octx.lt_stage_qp(level, a, b, index, np.concatenate(diags), bs, keys)
             assert np.array_equal(M.from_dev(oa), wa) and np.array_equal(M.from_dev(ob), wb)
+
+
+@pytest.mark.parametrize("kind", ["both", "integer", "double"])
+@pytest.mark.parametrize("dnum,level,count,bs,giants", [
+    (6, 5, 1, 4, 2), (6, 5, 3, 4, 5),  # six digits: one after the other
+    (3, 5, 1, 4, 5),                   # one ciphertext, more giant steps than four
+    (3, 5, 3, 4, 8), (2, 3, 5, 2, 6),  # five to eight giant steps, an odd last ciphertext
+    (3, 4, 2, 4, 9), (4, 5, 3, 2, 16),  # nine to sixteen, more than one ciphertext
+    (2, 3, 2, 2, 17),                  # a second launch of giant steps
+    (3, 5, 2, 18, 17),                 # and of baby steps
+    (3, 3, 2, 1, 10),                  # no baby step
+    (6, 5, 105, 2, 9),                 # more than 850,000 coefficients
+])
+def test_qp_stage_shapes_match_the_oracle(kind, dnum, level, count, bs, giants):
+    """The QP evaluator's fused kernel in each of its shapes (giant steps at a
+    time, ciphertexts at a time, digits unrolled or not), over moduli below and
+    above 2^50 in one basis and of one kind alone; a term of every second
+    diagonal is missing, giant step 1 is whole."""
+    M = product()
+    N = 1 << 10
+    p_bits, q_bits = {"both": ([61, 50], [36, 61, 42, 50, 38, 60]), "integer": ([61, 55], [60, 61, 52, 55, 58, 60]),
+                      "double": ([50, 49], [36, 50, 42, 50, 38, 27])}[kind]
+    p, q = O.find_primes(p_bits, q_bits, N)
+    ctx, octx = M.Context(N, q, p, dnum), O.Ctx(N, q, p, dnum)
+    assert (ctx.parts(level) > 5) == (dnum == 6)
+    rng = np.random.default_rng(dnum + 10 * giants + 1000 * count)
+    Q, basis, T = list(q[: level + 1]), list(q) + list(p), list(q[: level + 1]) + list(p)
+    index = [d for d in range(bs * giants) if bs == 1 or d // bs == 1 or d % 2 == 0 or d == bs * giants - 1]
+    assert {d // bs for d in index} == set(range(giants))
+    pool = [rand_residues(rng, T, N) for _ in range(5)]
+    diags = [pool[i % 5] for i in range(len(index))]
+    rots = sorted(({d % bs for d in index} | {d - d % bs for d in index}) - {0})
+    made = [np.concatenate([rand_residues(rng, basis, N) for _ in range(2 * octx.parts(len(q) - 1))]) for _ in range(3)]
+    keys = {r: made[i % 3] for i, r in enumerate(rots)}
+    cts = [(rand_residues(rng, Q, N), rand_residues(rng, Q, N)) for _ in range(count)]
+    dev = {id(x): M.to_dev(x) for x in pool + made}
+    W = (level + 1) * N
+    outs = [(M.to_dev(np.zeros(W, np.uint64)), M.to_dev(np.zeros(W, np.uint64))) for _ in cts]
+    ctx.linear_transform_qp_batch(level, [(M.to_dev(a), M.to_dev(b)) for a, b in cts], index,
+                                  [dev[id(d)] for d in diags], bs, {r: dev[id(k)] for r, k in keys.items()}, outs)
+    for i in {0, count - 1}:
+        wa, wb = octx.lt_stage_qp(level, *cts[i], index, np.concatenate(diags), bs, keys)
+        assert np.array_equal(M.from_dev(outs[i][0]), wa) and np.array_equal(M.from_dev(outs[i][1]), wb), i
 
 
 def _sequential(M, N, q, p, dnum, monkeypatch):
