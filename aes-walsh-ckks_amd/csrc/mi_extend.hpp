@@ -179,8 +179,7 @@ k_ext_cols(NttTabs tb, Job job) {
 template <class Job>
 void launch_ext_cols(const Context& c, Job job, int sources, int targets, hipStream_t s) {
     const NttTabs tb = tabs_of(c);
-    bool integer = true;
-    for (const BasisConst& b : c.h_bc) integer = integer && !b.fp;
+    const bool integer = c.integer_only();
 #define MI_EXT(LN)                                                                                    \
     {                                                                                                 \
         job.grid = ExtGrid{sources * pass_wpl(LN / 2, LN - LN / 2), targets, fast_div(targets)};      \

@@ -179,6 +179,12 @@ struct Context {
         int pp = (L + alpha - 1) / alpha;
         return pp < dnum ? pp : dnum;
     }
+    // every modulus is computed in integers (none below 2^50)
+    bool integer_only() const {
+        for (const BasisConst& b : h_bc)
+            if (b.fp) return false;
+        return true;
+    }
     void* workspace(hipStream_t s, size_t bytes);
     // `want` bytes, or at least `need` where those cannot be had (device memory, or a
     // capture, in which the buffer cannot grow); *whole says which.

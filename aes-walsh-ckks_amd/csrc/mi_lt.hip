@@ -502,12 +502,6 @@ void launch_inner(Context& c, const Compiled& k, const LtStage& st, int m, int K
     }
 }
 
-bool all_integer(const Context& c) {
-    for (const BasisConst& b : c.h_bc)
-        if (b.fp) return false;
-    return true;
-}
-
 // Baby steps and inner products of m items from their hoisted digits; outputs
 // as launch_inner.
 void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const u64* const* a, const u64* const* b,
@@ -515,7 +509,7 @@ void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const
                   long long outg_giant, long long outg_item, hipStream_t s) {
     const int L = st.level + 1, T = L + c.np;
     const int tps = (int)(c.N / LT_THREADS);
-    const bool integer = all_integer(c);
+    const bool integer = c.integer_only();
     const size_t most = integer ? 8 : LT_NG;
     for (int s0 = 0; s0 < k.nslots; s0 += LT_NB) {
         for (size_t gk0 = 0; gk0 < k.glist.size(); gk0 += most) {
@@ -612,7 +606,7 @@ void linear_transform_qp_batch(Context& c, const LtStage& st, int n, const u64* 
     // 1866 / 1562, 2709 / 2667, 5235 / 5522; N = 2^15, 14 limbs, 6 digits, 1, 2 and
     // 5 (459 k, 918 k, 2.3 M) 2510 / 2473, 3247 / 3397, 5866 / 6375; N = 2^16, 40
     // limbs, 3 digits, 1 (2.6 M) 6223 / 6509.
-    const bool separate = nbaby > 0 && k.glist.size() > 8 && n * W > 850000 && all_integer(c);
+    const bool separate = nbaby > 0 && k.glist.size() > 8 && n * W > 850000 && c.integer_only();
 
     // per-item scratch: digits | C | babies (a, b; separate) | out (a, b) | giant
     // inners (a, b) | ModDown temp

@@ -7,25 +7,6 @@
 
 namespace mi {
 
-// ---- in-place NTT over a list of polys (limb-major: shared twiddles) ----
-struct ListJob {
-    u64* p[2 * KS_MAX_ITEMS];
-    int npoly, basis0;
-    u64 N;
-    FastDiv per_limb;  // npoly
-    struct View {
-        int basis;
-        u64* p;
-        __device__ u64 load(int i) const { return p[i]; }
-        __device__ void store(int i, u64 v) const { p[i] = v; }
-    };
-    __device__ View view(int k) const {
-        const int l = per_limb.div(k), poly = k - l * npoly;
-        return View{basis0 + l, p[poly] + (long long)l * N};
-    }
-    __device__ bool skip(int) const { return false; }
-};
-
 // Contributions of the coefficient-domain P limbs to every Q limb, fused with
 // the forward column pass.
 struct MdExtJob {
@@ -94,18 +75,16 @@ void moddown_ext_cols(const Context& c, int level, int npoly, u64* const* p, u64
     launch_ext_cols(c, j, npoly, level + 1, s);
 }
 
-static ListJob list_job(const Context& c, int npoly, u64* const* p) {
-    ListJob j{};
-    for (int k = 0; k < npoly; ++k) j.p[k] = p[k];
-    j.npoly = npoly;
-    j.per_limb = fast_div(npoly);
-    j.basis0 = c.nq;
-    j.N = c.N;
-    return j;
+// The P limbs of npoly polys, a fixed distance apart, as an in-place batch.
+static PlainJob p_limbs(const Context& c, int npoly, u64* const* p) {
+    const long long stride = npoly > 1 ? p[1] - p[0] : 0;
+    for (int k = 1; k < npoly; ++k)
+        if (p[k] - p[k - 1] != stride) throw Error(-1, "ModDown needs evenly spaced P limbs");
+    return plain_job(LimbBatch{p[0], stride, c.np, c.nq, c.np * npoly}, c.N);
 }
 
 void moddown_p_cols(const Context& c, int npoly, u64* const* p, hipStream_t s) {
-    launch_pass<false, false>(c, list_job(c, npoly, p), c.np * npoly, s);
+    launch_pass<false, false>(c, p_limbs(c, npoly, p), c.np * npoly, s);
 }
 
 void ks_moddown_n(Context& c, int level, int npoly, u64* const* p, const u64* const* base, u64* const* out,
@@ -114,7 +93,7 @@ void ks_moddown_n(Context& c, int level, int npoly, u64* const* p, const u64* co
     const u64 N = c.N;
     if (npoly < 1 || npoly > 2 * KS_MAX_ITEMS) throw Error(-1, "ModDown batch size out of range");
     if (K > MAX_ALPHA) throw Error(-1, "more than 16 special moduli");
-    const ListJob j = list_job(c, npoly, p);
+    const PlainJob j = p_limbs(c, npoly, p);
     run_ntt_inv(c, j, j, K * npoly, s);
     MdOutJob o{};
     o.tmp = T;
