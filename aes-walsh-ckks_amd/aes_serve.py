@@ -9,9 +9,10 @@ and runs `lanes` evaluation lanes of it (own stream and working memory each)
 on native threads; a free lane packs the waiting requests, first come first
 served and whole, into the 1024 blocks of its next evaluation (ckks_aes_ctr_
 walsh_sbox_complex_blocks, ckks_aes_ctr_walsh_sbox.cpp:1037-1051: logical
-block j in complex slot j mod 512, real lane below 512, imaginary above), so
-requests that arrive while evaluations run are admitted into the next free
-lane and the lanes overlap on the device.  Admission is by device memory:
+block j in complex slot j mod 512, real lane below 512, imaginary above).
+Requests that arrive while an evaluation is in flight start when it ends, or
+as soon as they fill another lane's; full evaluations of several lanes overlap
+on the device.  Admission is by device memory:
 lanes open while their measured footprint fits the budget, and a request is
 refused (alone) when it exceeds one evaluation or when the work queued and
 in flight would exceed the open lanes' memory.

@@ -878,6 +878,12 @@ struct CKKSAesRequestResult {
 // counts, first come first served) taken whole into one evaluation of
 // `capacity` blocks; the first request that does not fit ends the batch.
 std::vector<size_t> ckks_aes_serve_take(const std::vector<size_t>& queued_blocks, size_t capacity);
+// Whether a free lane starts an evaluation of the queued requests now: at once
+// while no other is in flight, else only when they fill one.  An evaluation
+// costs the same however few blocks it holds, and two in flight share the
+// device: a nearly empty one beside another delays both, and the requests that
+// arrive meanwhile wait for the longer of the two.
+bool ckks_aes_serve_starts(const std::vector<size_t>& queued_blocks, size_t capacity, size_t in_flight);
 class CKKSAesCtrServer {
 public:
     // Encrypts the round keys under `owner` and opens the lanes (a warm-up

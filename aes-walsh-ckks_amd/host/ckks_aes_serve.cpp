@@ -11,9 +11,10 @@
 // and workspaces, the owner's keys read in place) runs on its own host
 // thread.  A free lane takes the waiting requests first come first served,
 // whole requests only, up to 1024 blocks, evaluates them (the 16 S-boxes of
-// a round as one batch), decrypts the 128 output bits and completes them;
-// requests that arrive meanwhile wait for the next free lane, and the lanes'
-// evaluations overlap on the device.
+// a round as one batch), decrypts the 128 output bits and completes them.
+// Requests that arrive while an evaluation is in flight wait for its end, or
+// until they fill another lane's (ckks_aes_serve_starts); under load the lanes'
+// full evaluations overlap on the device.
 //
 // Admission is by device memory: a lane opens only if its measured footprint
 // (the peak of its memory pool over a warm-up evaluation) fits the budget
@@ -58,6 +59,13 @@ std::vector<size_t> ckks_aes_serve_take(const std::vector<size_t>& queued, size_
     return offsets;
 }
 
+bool ckks_aes_serve_starts(const std::vector<size_t>& queued, size_t capacity, size_t in_flight) {
+    if (queued.empty()) return false;
+    if (in_flight == 0) return true;
+    const std::vector<size_t> offsets = ckks_aes_serve_take(queued, capacity);
+    return offsets.size() < queued.size() || offsets.back() + queued.back() == capacity;
+}
+
 struct CKKSAesCtrServer::Impl {
     struct Pending {
         uint64_t id;
@@ -77,7 +85,7 @@ struct CKKSAesCtrServer::Impl {
     std::map<uint64_t, CKKSAesRequestResult> done;
     int64_t charged = 0;  // bytes of the requests queued and in flight
     uint64_t next_id = 1;
-    size_t evaluations = 0;
+    size_t evaluations = 0, in_flight = 0;
     bool stopping = false;
     std::vector<std::thread> threads;
 
@@ -174,16 +182,21 @@ struct CKKSAesCtrServer::Impl {
             std::vector<size_t> offset;
             {
                 std::unique_lock<std::mutex> lk(mu);
-                cv_work.wait(lk, [&] { return stopping || !queue.empty(); });
-                if (queue.empty()) return;  // stopping with nothing left
                 std::vector<size_t> sizes;
-                for (const auto& r : queue) sizes.push_back(r.counters.size());
+                cv_work.wait(lk, [&] {
+                    sizes.clear();
+                    for (const auto& r : queue) sizes.push_back(r.counters.size());
+                    return (stopping && queue.empty()) || ckks_aes_serve_starts(sizes, kBlocksPerEvaluation, in_flight);
+                });
+                if (queue.empty()) return;  // stopping with nothing left
                 offset = ckks_aes_serve_take(sizes, kBlocksPerEvaluation);
                 for (size_t k = 0; k < offset.size(); ++k) {
                     batch.push_back(std::move(queue.front()));
                     queue.pop_front();
                 }
+                ++in_flight;
             }
+            cv_work.notify_all();  // the rest may fill another lane's evaluation
             const double start = now_s();
             std::vector<std::array<uint8_t, 16>> counters(kBlocksPerEvaluation), cts(kBlocksPerEvaluation);
             for (size_t k = 0; k < batch.size(); ++k) {
@@ -228,6 +241,8 @@ struct CKKSAesCtrServer::Impl {
                 done.emplace(batch[k].id, std::move(results[k]));
             }
             ++evaluations;
+            --in_flight;
+            cv_work.notify_all();
             cv_done.notify_all();
         }
     }

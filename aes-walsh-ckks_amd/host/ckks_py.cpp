@@ -717,6 +717,7 @@ PYBIND11_MODULE(ckks_py, m) {
         .def("evaluationBytes", &CKKSAesCtrServer::evaluationBytes)
         .def("evaluations", &CKKSAesCtrServer::evaluations);
     m.def("ckks_aes_serve_take", &ckks_aes_serve_take);
+    m.def("ckks_aes_serve_starts", &ckks_aes_serve_starts);
     m.def("steady_clock_seconds", [] {
         return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
     });

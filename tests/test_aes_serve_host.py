@@ -37,3 +37,83 @@ def test_batches_are_fifo_whole_requests_within_one_evaluation():
     assert list(take) == [0, 32, 532]          # the 100-block request would overflow: it waits
     assert list(H.ckks_aes_serve_take([1024, 1], 1024)) == [0]
     assert list(H.ckks_aes_serve_take([], 1024)) == []
+
+
+def test_a_lane_starts_at_once_alone_and_else_when_full():
+    starts = aes_serve._host().ckks_aes_serve_starts
+    assert not starts([], 1024, 0) and not starts([], 1024, 1)
+    assert starts([1], 1024, 0)
+    assert not starts([1], 1024, 1) and not starts([500, 523], 1024, 1)
+    assert starts([500, 524], 1024, 1) and starts([1024], 1024, 3)   # full to the last block
+    assert starts([1000, 25], 1024, 1)                               # the next request does not fit
+
+
+def _serve(arrivals, evaluation_s, starts, lanes=2, capacity=1024):
+    """Finish times of (time, blocks) requests: a free lane takes what waits
+    (first come first served, whole) when `starts` says so; the evaluations in
+    flight share the device evenly."""
+    take = aes_serve._host().ckks_aes_serve_take
+    queue, flight, finish, now, k = [], [], {}, 0.0, 0
+    while len(finish) < len(arrivals):
+        while len(flight) < lanes and starts([n for _, n in queue], capacity, len(flight)):
+            n = len(take([b for _, b in queue], capacity))
+            flight.append([evaluation_s, [i for i, _ in queue[:n]]])
+            queue = queue[n:]
+        end = now + min(f[0] for f in flight) * len(flight) if flight else float("inf")
+        nxt = min(end, arrivals[k][0] if k < len(arrivals) else float("inf"))
+        for f in flight:
+            f[0] -= (nxt - now) / len(flight)
+        now = nxt
+        if k < len(arrivals) and arrivals[k][0] <= now:
+            queue.append((k, arrivals[k][1]))
+            k += 1
+        for f in [f for f in flight if f[0] < 1e-9]:
+            finish.update({i: now for i in f[1]})
+            flight.remove(f)
+    return np.array([finish[i] for i in range(len(arrivals))])
+
+
+def greedy(queued, capacity, in_flight):
+    return len(queued) > 0
+
+
+def test_the_timed_request_sequence():
+    """bench.py's 48 served requests.  Where any free lane takes whatever waits,
+    evaluations of 0.52 s end the run later (2.60 s, median 1.54 s, as measured)
+    than ones of 0.59 s do (1.77 s, 1.26 s): the second lane's nearly empty
+    evaluations delay the first's.  By the server's rule the median is 0.75 s."""
+    rng, sizes = np.random.default_rng(55), []
+    for _ in range(48):
+        sizes.append(int(rng.integers(1, 33)))
+        rng.integers(0, 256, (sizes[-1], 16), dtype=np.uint8)
+    at = np.cumsum(rng.exponential(1.0 / 40.0, 48))
+    reqs = [(float(t), n) for t, n in zip(at, sizes)]
+    end = lambda s, rule: _serve(reqs, s, rule).max() - at[0]  # noqa: E731
+    median = lambda s, rule: float(np.median(_serve(reqs, s, rule) - at))  # noqa: E731
+    starts = aes_serve._host().ckks_aes_serve_starts
+    assert end(0.52, greedy) > 1.4 * end(0.59, greedy) and median(0.52, greedy) > 1.2 * median(0.59, greedy)
+    assert end(0.52, starts) < 0.85 * end(0.52, greedy)
+    assert median(0.52, starts) < median(0.59, starts) < 0.75 * median(0.59, greedy)
+
+
+@pytest.mark.parametrize("rate,count", [(40.0, 48), (40.0, 240), (400.0, 600), (2.0, 30)])
+def test_faster_evaluations_never_serve_slower(rate, count):
+    """Poisson arrivals of 1-32 blocks: shorter evaluations give earlier results,
+    and at no load is the median or the last result later than it is when any
+    free lane takes whatever waits (beyond one part in twenty)."""
+    starts = aes_serve._host().ckks_aes_serve_starts
+    ends, medians = {}, {}
+    for seed in range(5):
+        rng = np.random.default_rng(seed)
+        at = np.cumsum(rng.exponential(1.0 / rate, count))
+        reqs = [(float(t), int(n)) for t, n in zip(at, rng.integers(1, 33, count))]
+        for name, rule in (("server", starts), ("greedy", greedy)):
+            for s in (0.52, 0.59):  # seconds of an evaluation
+                f = _serve(reqs, s, rule)
+                ends.setdefault((name, s), []).append(f.max())
+                medians.setdefault((name, s), []).append(float(np.median(f - at)))
+    mean = lambda d, k: float(np.mean(d[k]))  # noqa: E731
+    assert mean(medians, ("server", 0.52)) < mean(medians, ("server", 0.59))
+    assert mean(ends, ("server", 0.52)) < mean(ends, ("server", 0.59))
+    assert mean(ends, ("server", 0.52)) <= 1.05 * mean(ends, ("greedy", 0.52))
+    assert mean(medians, ("server", 0.52)) <= 1.05 * mean(medians, ("greedy", 0.52))
