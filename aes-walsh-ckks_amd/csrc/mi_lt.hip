@@ -556,7 +556,8 @@ void launch_fused(Context& c, const Compiled& k, const LtStage& st, int m, const
                 MI_HIP(hipGetLastError());
                 continue;
             }
-            // the fewest giant steps that hold f.ng, and with them as many items
+            // several ciphertexts: the fewest giant steps that hold f.ng, and with
+            // them as many ciphertexts; one: 16 giant steps whatever f.ng is
 #define MI_LT_FUSED(NG, IT, PARTS)                                                                     \
     hipLaunchKernelGGL((k_lt_fused<NG, IT, PARTS>), dim3(tile_grid((m + IT - 1) / IT, tps, T)),        \
                        dim3(LT_THREADS), 0, s, f)

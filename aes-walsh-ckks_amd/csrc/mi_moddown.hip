@@ -1,6 +1,7 @@
 // Folded ModDown of hybrid key switching (ckks_keyswitch.cpp:521-673): inverse
 // NTT of the P slots, contribution sum_j x_j p_j^-1 - alpha per Q limb (the
-// P-side HPS estimate computed once per coefficient), NTT, subtracted from Q.
+// P-side HPS estimate summed again for every Q limb: mi_extend.hpp), NTT,
+// subtracted from Q.
 // The form with the key inner product folded in is mi_moddown_mac.hpp.
 #include "mi_extend.hpp"
 #include "mi_moddown.hpp"
@@ -75,7 +76,9 @@ void moddown_ext_cols(const Context& c, int level, int npoly, u64* const* p, u64
     launch_ext_cols(c, j, npoly, level + 1, s);
 }
 
-// The P limbs of npoly polys, a fixed distance apart, as an in-place batch.
+// The P limbs of npoly polys, a fixed distance apart, as an in-place batch.  They
+// run with one limb per workgroup: the tuned plan is measured over the whole
+// basis, and these are usually of one kind, for which that form has kernels.
 static PlainJob p_limbs(const Context& c, int npoly, u64* const* p) {
     const long long stride = npoly > 1 ? p[1] - p[0] : 0;
     for (int k = 1; k < npoly; ++k)
@@ -84,7 +87,7 @@ static PlainJob p_limbs(const Context& c, int npoly, u64* const* p) {
 }
 
 void moddown_p_cols(const Context& c, int npoly, u64* const* p, hipStream_t s) {
-    launch_pass<false, false>(c, p_limbs(c, npoly, p), c.np * npoly, s);
+    launch_plain_pass(c, false, false, 1, p_limbs(c, npoly, p), c.np * npoly, s);
 }
 
 void ks_moddown_n(Context& c, int level, int npoly, u64* const* p, const u64* const* base, u64* const* out,
@@ -93,8 +96,13 @@ void ks_moddown_n(Context& c, int level, int npoly, u64* const* p, const u64* co
     const u64 N = c.N;
     if (npoly < 1 || npoly > 2 * KS_MAX_ITEMS) throw Error(-1, "ModDown batch size out of range");
     if (K > MAX_ALPHA) throw Error(-1, "more than 16 special moduli");
-    const PlainJob j = p_limbs(c, npoly, p);
-    run_ntt_inv(c, j, j, K * npoly, s);
+    {
+        const PlainJob j = p_limbs(c, npoly, p);
+        const long probe = c.probe_open(s, K * npoly);
+        launch_plain_pass(c, false, true, 1, j, K * npoly, s);
+        launch_plain_pass(c, false, false, 1, j, K * npoly, s);
+        c.probe_close(probe, s);
+    }
     MdOutJob o{};
     o.tmp = T;
     for (int k = 0; k < npoly; ++k) {
