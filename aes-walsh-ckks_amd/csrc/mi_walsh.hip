@@ -77,7 +77,7 @@ constexpr int WALSH_BLOCK = 8 * WALSH_COEFFS;
 // six instructions per product.  Integers: the combinations as two sums of
 // halves and one double quotient, 128-bit lazy products.  Measured at N = 2^15
 // over 36-, 61- and 42-bit limbs, 16 output pairs and their relinearisations:
-// 739 us with integer multiply-adds throughout, 555 us.
+// 751 us with integer multiply-adds throughout, 583 us.
 struct WalshShared {
     u64 cst[2 * WALSH_MASKS];
     u64 part[2][2][4][WALSH_COEFFS];  // [side][product][quarter][coefficient]

@@ -938,15 +938,17 @@ def bench_ntt_qp(args, M, torch):
 
 def aes_ntt_roofline(M, torch, P, probe):
     """The NTT passes are the largest kernel family of the AES evaluation
-    (about half of its kernel time; the rest is spread over the Walsh product
-    sums, key-switch inner products, element-wise ops and copies).  `probe`
+    (two thirds of its kernel time, a third of that in column passes that form
+    their input by a base extension; the rest is spread over the Walsh product
+    sums, the linear transforms' inner products and element-wise ops).  `probe`
     is what the context's NTT probe measured over one whole evaluation, run
     with the side streams off so that no pair overlaps other work: HIP
     events on each launch pair's own stream around every forward and inverse
     NTT (column + row pass; standalone, inside key switches, rescales,
     ModRaise and the linear transforms), 16 N bytes per limb algorithmically
     (each limb read and written once).  achieved = algorithmic bytes of all
-    pairs / their summed event time.  For comparison the forward NTT of one
+    pairs / their summed event time, which holds the base extensions and key
+    products that are formed inside a pair.  For comparison the forward NTT of one
     QP ciphertext at the top level alone (2 polys x 17 limbs, N=2^15, the
     key switches' ModUp / ModDown shape) is timed the same way."""
     ntt_ms, pairs, ntt_bytes, ntt_limbs, probe_s = probe
@@ -974,7 +976,8 @@ def aes_ntt_roofline(M, torch, P, probe):
     return {"bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
             "frac": achieved / HBM_PEAK, "traffic": None if ratio is None else ratio * avg_bytes,
             "traffic_over_algorithmic": ratio, "valu_busy": _profile_traffic("ntt15_aes_inrun_valu_busy"),
-            "kernel": "NTT launch pairs (column + row pass) inside one walsh15 AES-CTR evaluation, N=2^15",
+            "kernel": "NTT launch pairs (column + row pass, with the base extensions and key products inside them) "
+                      "of one walsh15 AES-CTR evaluation, N=2^15",
             "launch_pairs": int(pairs), "limbs": int(ntt_limbs),
             "avg_pair_us": 1e3 * ntt_ms / max(1.0, pairs), "avg_limbs_per_pair": ntt_limbs / max(1.0, pairs),
             "ntt_event_ms": ntt_ms, "evaluation_ms": 1e3 * probe_s,
