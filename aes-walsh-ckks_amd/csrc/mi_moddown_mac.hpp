@@ -187,7 +187,7 @@ struct MdMacOutJob {
     __device__ bool skip(int) const { return false; }
 };
 
-template <KeyForm F, int PARTS, bool MAPPED>
+template <KeyForm F, int PARTS, bool MAPPED, Arith A = Arith::Both>
 void moddown_mac_out(Context& c, int level, int n, const KsItem* items, const KeyProductLists& kp, u64* const* p,
                      u64* T, hipStream_t s) {
     const int L = level + 1, npoly = 2 * n;
@@ -221,7 +221,7 @@ void moddown_mac_out(Context& c, int level, int n, const KsItem* items, const Ke
     o.per_limb = fast_div(npoly);
     const long long probe = c.probe_open(s, npoly * L);
     moddown_ext_cols(c, level, npoly, p, T, s);
-    launch_rows_w4<true>(c, o, npoly * L, s);
+    launch_rows_w4<true, A>(c, o, npoly * L, s);
     c.probe_close(probe, s);
 }
 
@@ -261,9 +261,12 @@ void moddown_mac_t(Context& c, int level, int n, const KsItem* items, const u64*
     }
     bool mapped = false;
     for (int i = 0; i < n; ++i) mapped = mapped || items[i].galois != 0;
-    // Unmapped stores keep the choice: straight-line, the pass spills 36 to 44
-    // bytes at 128 registers, and 32 switches at N = 2^15 took 940 us, not 912.
+    // Unmapped stores keep the choice where the kernel holds both arithmetics:
+    // straight-line, the pass spills 36 to 44 bytes at 128 registers, and 32
+    // switches at N = 2^15 took 940 us, not 912.  Integers alone: one switch of one
+    // digit at N = 2^14 with the choice 79.1 us, without 76.3.
     if (mapped) moddown_mac_out<F, PARTS, true>(c, level, n, items, kp, p, T, s);
+    else if (c.integer_only()) moddown_mac_out<F, PARTS, false, Arith::Int>(c, level, n, items, kp, p, T, s);
     else moddown_mac_out<KeyForm::Any, PARTS, false>(c, level, n, items, kp, p, T, s);
 }
 

@@ -276,10 +276,10 @@ __global__ void __launch_bounds__(NTT_THREADS) k_ntt_rows(NttTabs tb, Job job, i
 // The same pass held to 128 VGPRs (four waves per SIMD, the LDS limit), for
 // jobs whose load or store does enough work of its own that the scheduler
 // would otherwise trade occupancy for loads hoisted across the whole pass.
-template <int LOGN, bool FWD, class Job>
+template <int LOGN, bool FWD, Arith A, class Job>
 __global__ void __launch_bounds__(NTT_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 k_ntt_rows_w4(NttTabs tb, Job job, int count) {
-    ntt_pass<LOGN, FWD, true, 1, false, Arith::Both>(tb, job, count);
+    ntt_pass<LOGN, FWD, true, 1, false, A>(tb, job, count);
 }
 
 #define MI_NTT_LOGN_CASES(K)                                                                          \
@@ -320,12 +320,12 @@ void launch_rows(const Context& c, const Job& job, int count, hipStream_t s) {
     MI_HIP(hipGetLastError());
 }
 
-template <bool FWD, class Job>
+template <bool FWD, Arith A = Arith::Both, class Job>
 void launch_rows_w4(const Context& c, const Job& job, int count, hipStream_t s) {
     if (count >= (1 << 20)) throw Error(-1, "ntt: more than 2^20 limbs in one launch");
     const NttTabs tb = tabs_of(c);
 #define MI_ROWS(LN)                                                                                   \
-    hipLaunchKernelGGL((k_ntt_rows_w4<LN, FWD, Job>), dim3((unsigned)count * pass_wpl(LN - LN / 2, LN / 2)), \
+    hipLaunchKernelGGL((k_ntt_rows_w4<LN, FWD, A, Job>), dim3((unsigned)count * pass_wpl(LN - LN / 2, LN / 2)), \
                        dim3(pass_threads(LN - LN / 2, LN / 2)), 0, s, tb, job, count)
     MI_NTT_LOGN_CASES(MI_ROWS)
 #undef MI_ROWS
